@@ -206,7 +206,8 @@ def main() -> int:
                           "achieved": ach,
                           "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": ach / PEAK_FP32_TFLOPS,
                           "traffic": traffic, "alg_flops_per_launch": kernel_flops[k], "avg_ms": passes[k]})
-    if passes.get("bin", 0.0) > 0:
+    if passes.get("bin", 0.0) > 0 and kind != "gbsw":
+        # (GBSW bins only its active points, inside its volume pass)
         # binning moves bytes: per quadrature point its cell slot (a 4 B packed point, or a 16 B
         # record on grids binned by cells) or a 4 B volume (decided directly), plus the atom
         # positions; it is bound by its atomics' latency

@@ -109,9 +109,19 @@ struct SysHost {
 // atomics they save.
 constexpr double kBrickEdgeNm = 0.45;
 int brick_edge(const SysHost& s) {
-    if (s.kind == gbi::GRID_BRUTE) return 1;
+    if (s.kind == gbi::GRID_BRUTE || s.vol == gbi::VOL_GBSW) return 1;  // GBSW: k_gbsw_points
     const int sk = (int)std::lround(kBrickEdgeNm / s.g);
     return sk >= 3 ? std::min(gbi::kMaxBrickEdge, sk) : 1;
+}
+
+// Point slots per cell: 1.6 times the points of a cell at 100 atoms/nm^3; of a GBSW system, whose
+// slots hold its active points only (7 % of the points in a 25,000-atom globule, at most three
+// times that in a cell near the surface), a quarter of it.  An overflow doubles them.
+int pt_cap_estimate(const SysHost& s) {
+    if (s.kind == gbi::GRID_BRUTE) return std::max(1, s.N * s.Q);
+    const double share = s.vol == gbi::VOL_GBSW ? 0.25 : 1.0;
+    const double est = share * 1.6 * 100.0 * s.Q * s.g * s.g * s.g + 64.0;
+    return std::max(1, (int)std::min<double>(est, (double)s.N * s.Q));
 }
 
 // Cells per axis rounded up to whole bricks.
@@ -171,7 +181,12 @@ struct gbi_ctx {
     DevBuf<int> brick_count, cell_ctr;
     DevBuf<uint2> brick_rec;
     int brick_total = 0, brick_max = 0;
-    bool any_bricks = false, any_cells = true;
+    bool any_bricks = false, any_cells = true, any_cellbin = false;
+    DevBuf<unsigned long long> cell_sub;
+    DevBuf<ulonglong2> cell_mask;
+    DevBuf<float4> grec;
+    DevBuf<float2> gval;
+    DevBuf<int> atom_nact;
     DevBuf<float> quad_r2, vsig, vval;
     DevBuf<long long> force_fix, dedr_fix, vacc_fix;
 
@@ -236,6 +251,11 @@ struct gbi_ctx {
         brick_count.release();
         cell_ctr.release();
         brick_rec.release();
+        cell_sub.release();
+        cell_mask.release();
+        grec.release();
+        gval.release();
+        atom_nact.release();
         quad_r2.release();
         vsig.release();
         vval.release();
@@ -425,14 +445,16 @@ gbi::SysDesc make_desc(const gbi_ctx& c, const SysHost& s, long long cell_base, 
 // Cell, slot and worklist buffers for the systems' current capacities; uploads the
 // system descriptors and the cell -> system map.
 gbi_status layout(gbi_ctx& c) {
-    long long cells = 0, slots = 0, raw = 0, bricks = 0, brick_max = 0, brick_slots = 0;
+    long long cells = 0, slots = 0, gslots = 0, raw = 0, bricks = 0, brick_max = 0, brick_slots = 0;
     bool any_bricks = false, any_cells = false;
+    c.any_cellbin = false;
     for (const SysHost& s : c.sys) {
         cells += s.cell_cap;
-        slots += s.cell_cap * (long long)s.pt_cap;
+        (s.vol == gbi::VOL_GBSW ? gslots : slots) += s.cell_cap * (long long)s.pt_cap;
         raw += s.cell_cap * (long long)s.tmp_cap;
         const int sk = brick_edge(s);
         any_cells |= sk == 1;
+        c.any_cellbin |= sk == 1 && s.vol != gbi::VOL_GBSW;
         if (sk == 1) continue;  // binned by cells
         bricks += s.cell_cap / (sk * sk * sk);
         brick_max = std::max(brick_max, s.cell_cap / (sk * sk * sk));
@@ -441,7 +463,7 @@ gbi_status layout(gbi_ctx& c) {
     // brick slots share the prec slot layout (a system binning by cells leaves its range unused)
     brick_slots = any_bricks ? slots : 1;
     if (cells > kMaxCells) return fail(GBI_ERR_GRID_TOO_LARGE, "more than 16M lookup cells in the batch");
-    if (slots * (long long)sizeof(float4) > (200ll << 30))
+    if (slots * (long long)sizeof(float4) + gslots * (long long)(sizeof(float4) + sizeof(float2)) > (200ll << 30))
         return fail(GBI_ERR_GRID_TOO_LARGE, "point slots of the lookup grids exceed 200 GB");
     if (raw * (long long)sizeof(int) > (64ll << 30))
         return fail(GBI_ERR_GRID_TOO_LARGE, "raw cell lists of the lookup grids exceed 64 GB");
@@ -456,9 +478,9 @@ gbi_status layout(gbi_ctx& c) {
     // other small buffers, that pass was measured 15-20 % slower in some processes (0.26 vs
     // 0.215 ms at 5k atoms, 0.49 vs 0.445 ms at 25k), never with its own allocation
     HIP_TRY(c.cell_pt_count.ensure(cells, kOwnAllocation));
-    // counters on a line per 128 cells for the cells way (k_point_bin<false>: 0.419 -> 0.412 ms at
-    // 25,000 GBSW atoms, 9,284 -> 9,959 conformation-evals/s for 8 x 2,000); bricks-only contexts
-    // count in cell_pt_count, their split gaining nothing from it
+    // counters permuted so that neighbouring cells count on different lines (ctr_slot) where points
+    // reserve slots of their cells directly; bricks-only contexts count in cell_pt_count, their
+    // split gaining nothing from it
     if (any_cells) HIP_TRY(c.cell_ctr.ensure((cells + 4095) / 4096 * 4096, kOwnAllocation));
     HIP_TRY(c.brick_count.ensure(std::max<long long>(1, bricks) * gbi::kBrickStride, kOwnAllocation));
     HIP_TRY(c.brick_rec.ensure(brick_slots));
@@ -472,18 +494,25 @@ gbi_status layout(gbi_ctx& c) {
     HIP_TRY(c.worklist_sys.ensure(gbi::VOL_KINDS * cells));
     HIP_TRY(c.cell_sys.ensure(cells));
     HIP_TRY(c.scan_tmp.ensure((cells + 4095) / 4096 + 16));
-    HIP_TRY(c.prec.ensure(slots));
+    HIP_TRY(c.prec.ensure(std::max<long long>(1, slots)));
+    if (c.kinds[gbi::VOL_GBSW]) {
+        HIP_TRY(c.grec.ensure(gslots));
+        HIP_TRY(c.gval.ensure(gslots));
+        HIP_TRY(c.cell_sub.ensure(64 * cells));
+        HIP_TRY(c.cell_mask.ensure(cells));
+    }
     HIP_TRY(c.cell_atoms_tmp.ensure(std::max<long long>(1, raw)));
     std::vector<int> cs(cells);
     std::vector<gbi::SysDesc> desc(c.S);
-    long long cb = 0, pb = 0, tb = 0, bb = 0;
+    long long cb = 0, pb = 0, gb = 0, tb = 0, bb = 0;
     for (int s = 0; s < c.S; ++s) {
-        desc[s] = make_desc(c, c.sys[s], cb, pb, tb);
+        long long& slot_base = c.sys[s].vol == gbi::VOL_GBSW ? gb : pb;
+        desc[s] = make_desc(c, c.sys[s], cb, slot_base, tb);
         desc[s].brick_base = (int)bb;
         if (desc[s].sk > 1) bb += c.sys[s].cell_cap / (desc[s].sk * desc[s].sk * desc[s].sk);
         std::fill(cs.begin() + cb, cs.begin() + cb + c.sys[s].cell_cap, s);
         cb += c.sys[s].cell_cap;
-        pb += c.sys[s].cell_cap * (long long)c.sys[s].pt_cap;
+        slot_base += c.sys[s].cell_cap * (long long)c.sys[s].pt_cap;
         tb += c.sys[s].cell_cap * (long long)c.sys[s].tmp_cap;
     }
     HIP_TRY(hipMemcpyAsync(c.cell_sys.p, cs.data(), sizeof(int) * cells, hipMemcpyHostToDevice, c.stream));
@@ -847,7 +876,17 @@ gbi::KParams make_kparams(gbi_ctx& c, bool adjoint) {
     k.brick_total = c.brick_total;
     k.brick_max = c.brick_max;
     k.any_bricks = c.any_bricks ? 1 : 0;
-    k.any_cells = c.any_cells ? 1 : 0;
+    k.any_cellbin = c.any_cellbin ? 1 : 0;
+    for (const SysHost& s : c.sys)
+        if (s.vol == gbi::VOL_GBSW) {
+            (s.kind == gbi::GRID_TIGHT && !s.periodic() ? k.gbsw_exact : k.gbsw_other) = 1;
+            k.gbsw_q = std::max(k.gbsw_q, (s.Q + 1) & ~1);
+        }
+    k.cell_sub = c.cell_sub.p;
+    k.cell_mask = c.kinds[gbi::VOL_GBSW] ? c.cell_mask.p : nullptr;
+    k.grec = c.grec.p;
+    k.gval = c.gval.p;
+    k.atom_nact = c.atom_nact.p;
     k.frec0 = c.frec0.p;
     k.frec1 = c.frec1.p;
     k.frec2 = c.frec2.p;
@@ -1027,8 +1066,7 @@ gbi_status apply_tight_grid(gbi_ctx& c, double g) {
             s.g = g;
             s.cell_cap = 0;
             s.tmp_cap = 0;
-            const double est = 1.6 * 100.0 * s.Q * g * g * g + 64.0;
-            s.pt_cap = std::max(1, (int)std::min<double>(est, (double)s.N * s.Q));
+            s.pt_cap = pt_cap_estimate(s);
             changed = true;
         }
     if (!changed) return GBI_OK;
@@ -1080,9 +1118,7 @@ gbi_status setup_host(gbi_ctx& c, int S, const int32_t* n_atoms, const double* c
         h.g = h.kind == gbi::GRID_FAITHFUL ? h.P.grid_length : h.P.tight_grid_length;
         h.halfdiag = std::sqrt(3.0) / 2.0 * h.P.grid_length;
         h.gpad = 0.03 + h.halfdiag + h.P.buffer;  // CustomGBIntegral.cpp:174-175
-        const double est = 1.6 * 100.0 * h.Q * h.g * h.g * h.g + 64.0;
-        h.pt_cap = h.kind == gbi::GRID_BRUTE ? h.N * h.Q : (int)std::min<double>(est, (double)h.N * h.Q);
-        h.pt_cap = std::max(h.pt_cap, 1);
+        h.pt_cap = pt_cap_estimate(h);
         c.kinds[h.vol] = true;
         c.any_cut = c.any_cut || h.cutoff();
         c.any_trunc = c.any_trunc || (h.cutoff() && h.P.model == GBI_MODEL_GBSW);
@@ -1118,7 +1154,10 @@ gbi_status host_tables(const gbi_ctx& c, HostTables& t) {
             return fail(GBI_ERR_INVALID_ARGUMENT, e.what());
         }
         for (int q = 0; q < h.Q; ++q) {
-            const size_t row = (size_t)h.quad_base + q;
+            // GBSW: rows along the rays (direction-major), so that neighbouring lanes of k_gbsw_points
+            // have neighbouring points and share the lines of the masks and lists that they gather
+            const int k = h.vol == gbi::VOL_GBSW ? (q % h.P.n_lebedev) * h.P.n_radial + q / h.P.n_lebedev : q;
+            const size_t row = (size_t)h.quad_base + k;
             for (int d = 0; d < 3; ++d) t.off[3 * row + d] = table[q][d];
             for (int k = 0; k < 2; ++k)
                 t.pw[k * (size_t)qrow + row] = table[q][4] / std::pow(table[q][3], h.P.orders[k] - 2);
@@ -1198,11 +1237,13 @@ gbi_status create_batch(int S, const int32_t* n_atoms, const double* charge, con
     HIP_TRY(c->energy.ensure(S));
     HIP_TRY(c->stats.ensure(6));
     HIP_TRY(c->work.ensure(8));
-    HIP_TRY(c->frec0.ensure(NQ));
-    HIP_TRY(c->frec1.ensure(NQ));
+    const bool any_gbmv = c->kinds[gbi::VOL_GBMV1] || c->kinds[gbi::VOL_GBMV2];
+    HIP_TRY(c->frec0.ensure(any_gbmv ? NQ : 1));
+    HIP_TRY(c->frec1.ensure(any_gbmv ? NQ : 1));
     HIP_TRY(c->frec2.ensure(c->kinds[gbi::VOL_GBMV2] ? NQ : 1));
     HIP_TRY(c->vrec.ensure(NQ));
-    HIP_TRY(c->vval.ensure(NQ));
+    HIP_TRY(c->vval.ensure(any_gbmv ? NQ : 1));
+    HIP_TRY(c->atom_nact.ensure(N));
     HIP_TRY(c->force_fix.ensure(3 * N));
     HIP_TRY(c->bin_order.ensure(N));
     HIP_TRY(c->pair_atom.ensure(N));
@@ -1830,7 +1871,8 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
             clear(c.cell_act_count), clear(c.cell_sys), clear(c.cell_start), clear(c.frec_base), clear(c.worklist);
             clear(c.worklist_sys), clear(c.scan_tmp), clear(c.cell_atoms_tmp), clear(c.cell_atoms), clear(c.ent_pos);
             clear(c.ent_par), clear(c.prec), clear(c.frec0), clear(c.frec1), clear(c.frec2), clear(c.vval);
-            clear(c.vrec), clear(c.brick_count), clear(c.brick_rec);
+            clear(c.vrec), clear(c.brick_count), clear(c.brick_rec), clear(c.cell_sub), clear(c.cell_mask), clear(c.grec);
+            clear(c.gval), clear(c.atom_nact);
         }
     } unborrow{c};
     const int32_t n = n_atoms;
@@ -1864,6 +1906,8 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     c.brick_total = c.brick_max = 0;
     c.any_bricks = false;
     c.any_cells = true;
+    const bool gbsw = sh.vol == gbi::VOL_GBSW;
+    c.any_cellbin = !gbsw;
 
     // the buffers, carved once without a base (the size check, before the device is touched)
     // and once from the scratch array
@@ -1882,9 +1926,16 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     sc.take(c.frec_base, cells + 1), sc.take(c.worklist, gbi::VOL_KINDS * cells);
     sc.take(c.worklist_sys, gbi::VOL_KINDS * cells), sc.take(c.scan_tmp, (cells + 4095) / 4096 + 16);
     sc.take(c.cell_atoms_tmp, cells * (size_t)caps.tmp_cap), sc.take(c.cell_atoms, caps.entries);
-    sc.take(c.ent_pos, caps.entries), sc.take(c.ent_par, caps.entries), sc.take(c.prec, c.prec_total);
-    sc.take(c.frec0, NQ), sc.take(c.frec1, NQ), sc.take(c.frec2, c.kinds[gbi::VOL_GBMV2] ? NQ : 1);
-    sc.take(c.vval, NQ), sc.take(c.vrec, NQ);
+    sc.take(c.ent_pos, caps.entries), sc.take(c.ent_par, caps.entries);
+    sc.take(c.prec, gbsw ? 1 : c.prec_total), sc.take(c.grec, gbsw ? c.prec_total : 1);
+    sc.take(c.gval, gbsw ? c.prec_total : 1), sc.take(c.cell_mask, gbsw ? cells : 1), sc.take(c.atom_nact, gbsw ? N : 1);
+    sc.take(c.frec0, gbsw ? 1 : NQ), sc.take(c.frec1, gbsw ? 1 : NQ);
+    sc.take(c.frec2, c.kinds[gbi::VOL_GBMV2] ? NQ : 1), sc.take(c.vval, gbsw ? 1 : NQ);
+    // the sub-cell lists are read last by the points' pass, before the chain-rule pass writes vrec:
+    // both in one piece
+    const size_t sub = gbsw ? 64 * cells : 0;
+    sc.take(c.vrec, std::max(NQ, (sub * sizeof(unsigned long long) + sizeof(float4) - 1) / sizeof(float4)));
+    c.cell_sub.p = reinterpret_cast<unsigned long long*>(c.vrec.p);
     sc.take(c.brick_count, gbi::kBrickStride), sc.take(c.brick_rec, 1);
     sc.take(c.bbox_part, (size_t)gbi::kBboxMaxSlices * gbi::kBboxPart), sc.take(c.bbox_done, 1);
     };

@@ -96,7 +96,7 @@ struct SysDesc {
     int pt_base;               // pid = pt_base + (i - atom_begin) * Q + q
     int cell_base, cell_cap;   // global cells [cell_base, cell_base + cell_cap)
     int pt_cap;                // point slots per cell
-    long long prec_base;       // slot s of local cell c: prec_base + c * pt_cap + s
+    long long prec_base;       // slot s of local cell c: prec_base + c * pt_cap + s (GBSW: of KParams::grec)
     int sk;                    // bricks of sk x sk x sk cells reserve point slots together (binning; 1: cells)
     int brick_base;            // the system's first brick in KParams::brick_count
     long long tmp_base;        // raw member k of local cell c: cell_atoms_tmp[tmp_base + c * tmp_cap + k]
@@ -220,8 +220,8 @@ struct KParams {
     int* cell_count_eff;     // cell_total
     int* cell_atoms_tmp;     // entry_cap
     int* cell_atoms;         // entry_cap
-    float4* ent_pos;         // entry_cap: position relative to the cell corner, .w = atom index bits
-    float4* ent_par;         // entry_cap: aparam of the atom
+    float4* ent_pos;         // entry_cap: position relative to the cell corner, aparam.x
+    float4* ent_par;         // entry_cap: aparam.y, aparam.z, atom index bits, R
     // points
     int* cell_pt_count;      // cell_total: points per cell (gathered from cell_ctr by the scan)
     int* cell_ctr;           // ctr_len: the binning passes' point counters, cell c's at ctr_slot(c)
@@ -234,18 +234,26 @@ struct KParams {
     int brick_total;         // sum of the systems' brick ranges
     int brick_max;           // the largest brick range of a system
     int any_bricks;          // some system bins by bricks (SysDesc::sk > 1)
-    int any_cells;           // some system bins by cells (SysDesc::sk = 1)
+    int any_cellbin;         // some GBMV system bins by cells (SysDesc::sk = 1)
     int* cell_act_count;     // cell_total
     int* frec_base;          // cell_total + 1: exclusive scan of the point counts
     int* worklist;           // VOL_KINDS x cell_total
     int* worklist_sys;       // VOL_KINDS x cell_total: system of each worklist cell
     float4* prec;            // per system: cell_cap x pt_cap slots; records (FP32 point - corner, packed point),
                              // or, binning by bricks, packed points (atom << kQBits | q) in the range's first quarter
-    float4* frec0;           // NQ: active points, grouped by cell (corner-relative FP32 point, packed point)
-    float4* frec1;           // NQ: GBSW (V, 0, 0, 0) / GBMV1 (dV/dS, V, 0, 0) / GBMV2 (c1, c2, c3, vx)
+    int gbsw_exact, gbsw_other;    // some GBSW system has the exact non-periodic grid, another one
+    int gbsw_q;                    // the most points per atom of a GBSW system, rounded up to even
+    ulonglong2* cell_mask;         // cell_total (null without GBSW systems): sub-cells with V = 0, with V = 1
+    unsigned long long* cell_sub;  // cell_total x 64 (GBSW cells with atoms): the atoms that reach each sub-cell
+    float4* grec;            // GBSW systems: slots of their active points (prec_base, pt_cap as in prec)
+    float2* gval;            // per grec slot: V, rank among its owner's active points
+    int* atom_nact;          // N: active points of each atom (GBSW)
+    float4* frec0;           // NQ (GBMV): active points, grouped by cell (corner-relative FP32 point, packed point)
+    float4* frec1;           // NQ: GBMV1 (dV/dS, V, 0, 0) / GBMV2 (c1, c2, c3, vx)
     float4* frec2;           // NQ: GBMV2 (vy, vz, V, 0)
-    float* vval;             // NQ by pid: V, sign bit set on the points with a chain-rule factor
-    float4* vrec;            // NQ by pid: owner force of those points only (others stale), .w unused
+    float* vval;             // NQ by pid (GBMV): V, sign bit set on the points with a chain-rule factor
+    float4* vrec;            // NQ: owner force of those points only (others stale), .w unused; by pid, GBSW:
+                             // by rank among the owner's active points
     float* vsig;             // NQ (adjoint, GBMV) by pid: S of the sigmoid, NaN where V has no derivative
     // per atom
     double* integrals;       // 2 x N

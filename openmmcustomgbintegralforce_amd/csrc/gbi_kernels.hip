@@ -3,8 +3,9 @@
 // One evaluation (launch_evaluate) of a batch of systems runs, on one stream, one launch
 // per pass for all systems together:
 //   clear -> bounding boxes / grid geometry (workgroup per system) -> cell lists (count,
-//   scan, fill, sort+cap) -> point binning -> volume pass (per cell, lanes = points, one
-//   launch per volume kind present) -> integrals + Born map (per atom) -> STILL pair pass
+//   scan, fill, sort+cap) -> GBSW: volumes, integrals and Born map (per atom); GBMV: point
+//   binning -> volume pass (per cell, lanes = points, one launch per kind present) ->
+//   integrals + Born map (per atom) -> STILL pair pass
 //   (tiles of 64 rows x a column range inside one system) -> per-atom chain (dE/dB ->
 //   dE/dI, self energy) -> energy per system -> chain-rule force pass (per cell, lanes =
 //   list atoms x points) -> owner-force reduction [-> adjoint reductions].
@@ -28,12 +29,14 @@
 #include <climits>
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace gbi {
 
 namespace {
 
 constexpr int kWave = 64;
+constexpr int kXcds = 8;  // workgroups go to the XCDs round-robin
 constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanThreads * kScanItems;
@@ -583,9 +586,10 @@ __global__ void __launch_bounds__(256) k_grid_fill(KParams p) {
 }
 
 // Entry of key (atom, image code) relative to the cell corner: for periodic systems the
-// wrapped atom moved by the code's box vectors, i.e. its image nearest the cell.
-__device__ inline void write_entry(const KParams& p, const SysDesc& sd, const SysGeom& G, int e, int key,
-                                   const double* corner) {
+// wrapped atom moved by the code's box vectors, i.e. its image nearest the cell.  ent_pos:
+// (position - corner, aparam.x); ent_par: (aparam.y, aparam.z, atom index bits, R).
+__device__ inline float4 write_entry(const KParams& p, const SysDesc& sd, const SysGeom& G, int e, int key,
+                                     const double* corner) {
 #pragma clang fp contract(off)
     const int j = key >> kImageBits;
     double x[3];
@@ -597,9 +601,12 @@ __device__ inline void write_entry(const KParams& p, const SysDesc& sd, const Sy
             x[d] = wrap_coord(G, d, x[d]) - img * G.L[d];  // the cell image sits img boxes away
         }
     }
-    p.ent_pos[e] = make_float4((float)(x[0] - corner[0]), (float)(x[1] - corner[1]), (float)(x[2] - corner[2]),
-                               __int_as_float(j));
-    p.ent_par[e] = p.aparam[j];
+    const float4 a = p.aparam[j];
+    const float4 pos =
+        make_float4((float)(x[0] - corner[0]), (float)(x[1] - corner[1]), (float)(x[2] - corner[2]), a.x);
+    p.ent_pos[e] = pos;
+    p.ent_par[e] = make_float4(a.y, a.z, __int_as_float(j), a.w);
+    return pos;
 }
 
 // One wave per cell: order the cell's atoms by index (rank sort), keep the first `cap`
@@ -610,15 +617,78 @@ __device__ inline void write_entry(const KParams& p, const SysDesc& sd, const Sy
 // cell), as the reference would; equal keys then take consecutive ranks.
 constexpr int kSortLds = 256;  // cells with more raw members sort in global memory
 
+// GBSW: what is known of a cell's 4 x 4 x 4 sub-cells (x y z, z fastest; lane = sub-cell).
+// cell_mask: the sub-cells that the burial sphere R' - w of a list atom holds wholly (V = 0 at
+// every point) and those that no atom's switching sphere R' + w reaches (V = 1).  cell_sub, for
+// the others: bit m for each list atom m that reaches the sub-cell (the rest have H = 1 there),
+// or kSubScan in cells of more than 63 atoms.  k_gbsw_points reads V from the masks for 64 % of
+// the points outside their owner in a 25,000-atom globule (2 x 2 x 2 sub-cells: 36 %; 8 x 8 x 8:
+// 80 %, for 8 times this work) and runs the others down 6 atoms instead of 17.  kSubMargin exceeds
+// the rounding of the FP32 coordinates and distances (1e-7 nm), so a point has the V that its
+// whole list would give.
+constexpr int kSub = 4;
+constexpr float kSubMargin = 1e-6f;
+constexpr unsigned long long kSubScan = 1ull << 63;
+
+__device__ inline void sub_cell_lists(const KParams& p, const SysDesc& sd, const SysGeom& G, int c, int base, int n,
+                                      int lane, float4* s_e) {
+    unsigned long long* out = p.cell_sub + (long long)c * kWave + lane;
+    if (sd.grid_kind == GRID_BRUTE) {  // one cell without bounds: every point is evaluated
+        *out = kSubScan;
+        if (lane == 0) p.cell_mask[c] = make_ulonglong2(0ull, 0ull);
+        return;
+    }
+    const int sub[3] = {lane / (kSub * kSub), (lane / kSub) % kSub, lane % kSub};
+    float mid[3], half[3];
+    for (int d = 0; d < 3; ++d) {
+        const float edge = (float)(sd.periodic ? G.step[d] : sd.g) / kSub;
+        mid[d] = ((float)sub[d] + 0.5f) * edge;
+        half[d] = 0.5f * edge;
+    }
+    bool buried = false;
+    uint32_t reach[2] = {0u, 0u};
+    for (int m0 = 0; m0 < n; m0 += 32) {
+        if ((m0 & (kWave - 1)) == 0) {  // the next 64 entries; each lane reads those that it wrote
+            __syncthreads();
+            if (m0 + lane < n) s_e[lane] = p.ent_pos[base + m0 + lane];
+            __syncthreads();
+        }
+        uint32_t bits = 0u;
+        for (int m = 0; m < min(32, n - m0); ++m) {
+            const float4 e = s_e[(m0 & 32) + m];
+            const float dx = fabsf(e.x - mid[0]), dy = fabsf(e.y - mid[1]), dz = fabsf(e.z - mid[2]);
+            const float fx = dx + half[0], fy = dy + half[1], fz = dz + half[2];
+            const float nx = fmaxf(dx - half[0], 0.f), ny = fmaxf(dy - half[1], 0.f), nz = fmaxf(dz - half[2], 0.f);
+            const float far2 = fmaf(fx, fx, fmaf(fy, fy, fz * fz)), near2 = fmaf(nx, nx, fmaf(ny, ny, nz * nz));
+            const float lo = e.w - sd.sw - kSubMargin, hi = e.w + sd.sw + kSubMargin;
+            buried |= lo > 0.f && far2 < lo * lo;
+            bits |= near2 <= hi * hi ? 1u << m : 0u;
+        }
+        reach[(m0 >> 5) & 1] |= bits;
+    }
+    const unsigned long long r = ((unsigned long long)reach[1] << 32) | reach[0];
+    *out = n > 63 ? kSubScan : r;
+    const bool any = (reach[0] | reach[1]) != 0u;
+    const unsigned long long in = __ballot(buried), out_of = __ballot(!any && !buried);
+    if (lane == 0) p.cell_mask[c] = make_ulonglong2(in, out_of);
+}
+
+// SUB: some system is GBSW (its cells also get their sub-cells' lists; without them the kernel
+// holds 6 registers and 1 KB of LDS less).
+template <bool SUB>
 __global__ void __launch_bounds__(64) k_grid_sort(KParams p) {
     __shared__ __align__(16) int s_in[kSortLds];
     __shared__ int s_out[kSortLds];
+    __shared__ float4 s_e[SUB ? kWave : 1];
     if (batch_fatal(p)) return;
     const int lane = threadIdx.x;
     for (int c = blockIdx.x; c < p.cell_total; c += gridDim.x) {
         const int n_raw = p.cell_fill[c];
         if (n_raw == 0) {
-            if (lane == 0) p.cell_count_eff[c] = 0;
+            if (lane == 0) {
+                p.cell_count_eff[c] = 0;
+                if (SUB) p.cell_mask[c] = make_ulonglong2(0ull, ~0ull);  // no atom reaches it
+            }
             continue;
         }
         const int s = p.cell_sys[c];
@@ -665,6 +735,7 @@ __global__ void __launch_bounds__(64) k_grid_sort(KParams p) {
         }
         if (lane == 0) p.cell_count_eff[c] = eff;
         __syncthreads();
+        if (SUB && sd.vol_kind == VOL_GBSW) sub_cell_lists(p, sd, G, c, base, eff, lane, s_e);
     }
 }
 
@@ -773,7 +844,7 @@ __device__ inline void quad_point(const KParams& p, double xi, double yi, double
     pt[2] = zi + p.quad_off[3 * row + 2];
 }
 
-// Binning.  k_point_bin: one workgroup per atom (systems in turn, each visited with a stride
+// Binning of the GBMV kinds.  k_point_bin: one workgroup per atom (systems in turn, each visited with a stride
 // coprime to its size so concurrent workgroups hit distant counters) finds the cell of every
 // quadrature point (FP64, the oracle's arithmetic), counts its points per key in an LDS hash
 // table (local ranks) and reserves each key's slots with one global atomic; these returning
@@ -783,25 +854,22 @@ __device__ inline void quad_point(const KParams& p, double xi, double yi, double
 //     counter on a 128-byte line of its own; the workgroup files (packed point, cell in brick)
 //     in the brick's slots and k_point_split moves the packed points into the cells.  An atom's 1,200 GBMV-II
 //     points fall into about 200 bricks of 0.45 nm against 670 cells of 0.15 nm.
-//   cells (sk = 1, the exact GBSW grid of 0.20 nm, where bricks of 0.40 nm save too few
-//     atomics to pay for the second pass): the key is the cell and the workgroup writes the
-//     cell's slots directly.
+//   cells (sk = 1: grids above 0.18 nm, where bricks save too few atomics to pay for the second
+//     pass, the brute cell, and gbi_execute_noalloc): the key is the cell and the workgroup
+//     writes the cell's slots directly.
 // What a cell slot holds depends on the way (pt_slot / point_record):
 //   bricks: the packed point (atom << kQBits | q), 4 bytes; the volume pass recomputes the
 //     point from the atom's FP64 position and the quadrature row.  Against a 16-byte record
 //     this halves k_point_split (0.062 -> 0.030 ms at 5,000 GBMV-II atoms) for 0.005 ms more
 //     in the volume pass.
 //   cells: the record (the point relative to its cell's corner in FP32, the packed point),
-//     16 bytes.  There the binning pass is bound by its atomics, not by its writes, and the
-//     GBSW volume pass, whose points mostly leave after a few atoms on burial, took 20 % longer
-//     recomputing the points.
-// Points outside the grid, in an empty cell, or (GBSW) inside the owner's own burial radius get
-// their volume directly.
+//     16 bytes.  There the binning pass is bound by its atomics, not by its writes.
+// Points outside the grid or in an empty cell get their volume directly.
 constexpr int kBinHash = 2048;  // > Q: the table never fills
 // Threads per workgroup: bricks 512 (4 points per thread, 56 VGPRs, 8 waves per SIMD: 0.088 ->
-// 0.075 ms at 5,000 GBMV-II atoms against 256 threads); cells 256 (8 points per thread: the
-// 512-thread form took 0.62 ms against 0.42 at 25,000 GBSW atoms, whose pass is bound by its
-// returning atomics).
+// 0.075 ms at 5,000 GBMV-II atoms against 256 threads); cells 256 (8 points per thread: with 512
+// threads its pass, bound by its returning atomics, took 0.62 ms against 0.42 for 25,000 atoms on
+// a 0.20 nm grid).
 template <bool BRICKS>
 constexpr int bin_threads() { return BRICKS ? 512 : 256; }
 
@@ -846,17 +914,13 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
     const SysGeom G = p.geom[s];
     const int Q = sd.Q, qb = sd.quad_base, cb = sd.cell_base, sk = sd.sk, pt_cap = sd.pt_cap;
     constexpr bool bricks = BRICKS;
-    if ((sk > 1) != BRICKS) return;
+    if ((sk > 1) != BRICKS || sd.vol_kind == VOL_GBSW) return;
     const long long key_slots = (long long)sk * sk * sk * pt_cap;
     const long long prec_base = sd.prec_base;
     const int pbase = sd.pt_base + (i - sd.atom_begin) * Q;
-    // only lists that surely hold the owner (exact or brute) may skip it; the reference
-    // GBMV-form grid is under-padded and can miss it (GBSWIntegral.cpp:59-60)
-    const bool shortcut = sd.vol_kind == VOL_GBSW && sd.grid_kind != GRID_FAITHFUL;
     const float v_empty = sd.v_empty;
     const float sig_empty = sd.vol_kind == VOL_GBMV1 ? 0.0f : __int_as_float(0x7fc00000);
     const double xi = p.pos[3 * i], yi = p.pos[3 * i + 1], zi = p.pos[3 * i + 2];
-    const float own_lo2 = p.aparam[i].y;
     for (int k = tid; k < kBinHash; k += kBinThreads) {
         t_key[k] = -1;
         t_cnt[k] = 0;
@@ -875,15 +939,12 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
         const int row = qb + q;
         int c = -1, idx[3] = {0, 0, 0};
         double pt[3] = {0.0, 0.0, 0.0};
-        const bool owner_buried = shortcut && p.quad_r2[row] <= own_lo2;
-        if (!owner_buried) {
-            quad_point(p, xi, yi, zi, row, pt);
-            c = sd.periodic ? point_cell_periodic(G, pt, idx) : point_cell(sd, G, pt[0], pt[1], pt[2], idx);
-            if (c >= 0 && p.cell_count_eff[cb + c] == 0) c = -1;
-        }
+        quad_point(p, xi, yi, zi, row, pt);
+        c = sd.periodic ? point_cell_periodic(G, pt, idx) : point_cell(sd, G, pt[0], pt[1], pt[2], idx);
+        if (c >= 0 && p.cell_count_eff[cb + c] == 0) c = -1;
         if (c < 0) {
-            p.vval[pbase + q] = owner_buried ? 0.0f : v_empty;
-            if (p.adjoint) p.vsig[pbase + q] = owner_buried ? __int_as_float(0x7fc00000) : sig_empty;
+            p.vval[pbase + q] = v_empty;
+            if (p.adjoint) p.vsig[pbase + q] = sig_empty;
             continue;
         }
         int key = c;
@@ -1012,6 +1073,275 @@ __global__ void __launch_bounds__(256) k_point_split(KParams p) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// GBSW points: V, the integrals and the Born radius of one atom per workgroup, and the records
+// of its active points (0 < V < 1) for the chain-rule pass.
+//   1. Every point is located in FP64 (the oracle's arithmetic) and takes V = 0 or 1 from its
+//      cell's masks where they decide (or from its owner's burial radius); the others queue.
+//   2. Queued points, one per lane, run down their sub-cell's list: V = prod_j H_j, H = 0 inside
+//      R' - w, the cubic in the shell, 1 beyond R' + w (GBSWIntegral.cpp:187-224); a lane leaves
+//      at V = 0.
+//   3. Active points (about 7 %) are ranked in q order; each reserves a slot of its cell with one
+//      atomic and writes (point - corner, packed point) and (V, rank).
+//   4. I_k = sum_q w_q / r_q^(n_k - 2) (1 - V) in FP64 in a fixed order, and the Born map.
+// Sorting all points into cells first (an atomic per atom and cell, 345 of them per atom, and a
+// pass over the cells' points with the atoms in LDS) took 0.42 + 0.36 ms at 25,000 atoms plus
+// 0.04 ms for the integrals, for points of which 93 % have V = 0 or 1 after an atom or two; this
+// kernel takes 0.274 ms (25k evaluation 1.43 -> 0.87 ms, the adjoint of 8 x 2,000 atoms 1.00 -> 0.70).
+// What bounds it: the gathers.  Each lane's 16 bytes lie on a line of their own (84 M L1 lookups,
+// 0.14 ms at one per cycle and CU); with V = 1 taken for every queued point it took 0.227 ms of
+// 0.359, and without the sub-cells' bits 0.073, in a form that gathered the 8-byte lists of all
+// points in step 1 (the 16-byte masks of a whole cell there instead: 0.274).  Whole lists in place
+// of the sub-cells': 0.51 ms.  VALU issue is at 60 %; the atomics of step 3 are 0.02 ms.
+// ---------------------------------------------------------------------------
+constexpr int kGbswThreads = 256;
+constexpr int kGbswMaxQ = 1 << kQBits;
+constexpr int kGbswBatch = 4;  // points whose gathers a lane has in flight
+
+// The integrals of atom i and, for the canonical energy, its Born radius and dB/dI (one lane).
+__device__ inline void atom_integrals(const KParams& p, const SysDesc& sd, int s, int i, double a0, double a1) {
+    p.integrals[i] = a0;
+    p.integrals[p.N + i] = a1;
+    if (sd.custom) return;  // the generated kernels map the integrals
+    const double I4 = sd.i4 == 0 ? a0 : a1;
+    const double I7 = sd.i7 == 0 ? a0 : a1;
+    const double eta = sd.eta;
+    const double eta4 = eta * eta * eta * eta;
+    const double T = 1.0 / (4.0 * eta4) - I7;
+    const double T4 = sqrt(sqrt(T));  // T^(1/4): two square roots for one pow, to the same rounding
+    const double D = sd.alpha0 * (1.0 / eta - I4) + sd.alpha1 * T4;
+    const double B = sd.slope / D + sd.shift;
+    p.born[i] = B;
+    p.dbdi[sd.i4 * p.N + i] = sd.slope * sd.alpha0 / (D * D);
+    p.dbdi[sd.i7 * p.N + i] = sd.slope * 0.25 * sd.alpha1 / (T4 * T4 * T4) / (D * D);
+    if (!isfinite(B) || !(B > 0.0)) raise_flag(p, s, FLAG_NONFINITE_RESULT);
+}
+
+// Cell of a point (local index, -1 outside) and its corner-relative FP32 coordinates.
+__device__ inline int gbsw_locate(const KParams& p, const SysDesc& sd, const SysGeom& G, double xi, double yi,
+                                  double zi, int row, float* r) {
+#pragma clang fp contract(off)
+    double pt[3], corner[3];
+    int idx[3];
+    quad_point(p, xi, yi, zi, row, pt);
+    const int c = sd.periodic ? point_cell_periodic(G, pt, idx) : point_cell(sd, G, pt[0], pt[1], pt[2], idx);
+    if (c < 0) return -1;
+    cell_corner_idx(sd, G, idx[0], idx[1], idx[2], corner);
+    for (int d = 0; d < 3; ++d) r[d] = (float)(pt[d] - corner[d]);
+    return c;
+}
+
+// EXACT: the exact non-periodic grid (the standalone GBSW force), whose cell indices are the
+// truncated quotients.  The sub-cell then comes from the quotient's fraction, whose rounding
+// (1e-12 of a cell) is far inside kSubMargin.
+template <bool EXACT>
+__device__ inline int gbsw_sub_cell(const KParams& p, const SysDesc& sd, const SysGeom& G, double xi, double yi,
+                                    double zi, int row, const float* sub, int& bit) {
+#pragma clang fp contract(off)
+    int b[3], c = 0;
+    if (EXACT) {
+        double pt[3];
+        quad_point(p, xi, yi, zi, row, pt);
+        bool in = true;
+        for (int d = 0; d < 3; ++d) {
+            const double t = (pt[d] - G.origin[d]) * sd.inv_g;
+            const double f = floor(t);
+            const int idx = (int)f;
+            in &= (unsigned)idx < (unsigned)G.n[d];
+            c = c * G.n[d] + idx;
+            b[d] = (int)((float)(t - f) * kSub);  // 0 .. kSub (t - f may round to 1)
+        }
+        if (!in) return -1;
+    } else {
+        float r[3];
+        c = gbsw_locate(p, sd, G, xi, yi, zi, row, r);
+        if (c < 0) return -1;
+        for (int d = 0; d < 3; ++d) b[d] = max((int)(r[d] * sub[d]), 0);
+    }
+    bit = (min(b[0], kSub - 1) * kSub + min(b[1], kSub - 1)) * kSub + min(b[2], kSub - 1);
+    return c;
+}
+
+// Corner-relative coordinates of a point that gbsw_sub_cell has placed.
+template <bool EXACT>
+__device__ inline int gbsw_place(const KParams& p, const SysDesc& sd, const SysGeom& G, double xi, double yi,
+                                 double zi, int row, float* r) {
+#pragma clang fp contract(off)
+    if (!EXACT) return gbsw_locate(p, sd, G, xi, yi, zi, row, r);
+    double pt[3];
+    int c = 0;
+    quad_point(p, xi, yi, zi, row, pt);
+    for (int d = 0; d < 3; ++d) {
+        const double f = floor((pt[d] - G.origin[d]) * sd.inv_g);
+        c = c * G.n[d] + (int)f;
+        r[d] = (float)(pt[d] - (G.origin[d] + f * sd.g));
+    }
+    return c;
+}
+
+// Dynamic LDS of k_gbsw_points, per quadrature point: V, and the index of a queued point.
+constexpr int kGbswLds = 4 + 2;
+
+template <bool EXACT>
+__global__ void __launch_bounds__(kGbswThreads) k_gbsw_points(KParams p) {
+    constexpr int kWords = kGbswMaxQ / 32;
+    extern __shared__ __align__(16) char s_dyn[];
+    __shared__ uint32_t s_bits[kWords];
+    __shared__ int s_pre[kWords];
+    __shared__ int s_nq, s_nact;
+    __shared__ double s_sum[2][kGbswThreads / kWave];
+    if (batch_fatal(p)) return;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+    // workgroup b runs on XCD b mod 8: each XCD takes a run of atoms, neighbours along the chain, so
+    // the lists that their points share stay in its L2 (atoms in the strided binning order: 2.6 GB
+    // of L2 misses at 25,000 atoms against 0.7)
+    const int i = (int)(blockIdx.x % kXcds) * (int)(gridDim.x / kXcds) + (int)(blockIdx.x / kXcds);
+    if (i >= p.N) return;
+    const int s = p.atom_sys[i];
+    const SysDesc sd = p.sys[s];
+    if (sd.vol_kind != VOL_GBSW || (sd.grid_kind == GRID_TIGHT && !sd.periodic) != EXACT) return;
+    const SysGeom G = p.geom[s];
+    const int Q = sd.Q, qb = sd.quad_base, cb = sd.cell_base;
+    float* s_v = reinterpret_cast<float*>(s_dyn);
+    uint16_t* s_q = reinterpret_cast<uint16_t*>(s_v + p.gbsw_q);
+    // only lists that surely hold the owner (exact or brute) may skip it; the reference
+    // GBMV-form grid is under-padded and can miss it (GBSWIntegral.cpp:59-60)
+    const float own_lo2 = sd.grid_kind != GRID_FAITHFUL ? p.aparam[i].y : -1.f;
+    const double xi = p.pos[3 * i], yi = p.pos[3 * i + 1], zi = p.pos[3 * i + 2];
+    float sub[3];  // sub-cells per nm
+    for (int d = 0; d < 3; ++d) sub[d] = kSub * fast_rcp((float)(!EXACT && sd.periodic ? G.step[d] : sd.g));
+    if (tid == 0) s_nq = 0;
+    if (tid < kWords) s_bits[tid] = 0u;
+    __syncthreads();
+    for (int q0 = 0; q0 < Q; q0 += kGbswThreads * kGbswBatch) {
+        // kGbswBatch points per thread: their gathers are all in flight together
+        int cell[kGbswBatch], bit[kGbswBatch];
+        ulonglong2 m[kGbswBatch];
+#pragma unroll
+        for (int u = 0; u < kGbswBatch; ++u) {
+            const int q = q0 + u * kGbswThreads + tid;
+            cell[u] = -1;
+            bit[u] = 0;
+            m[u] = make_ulonglong2(0ull, ~0ull);
+            if (q >= Q) continue;
+            if (p.quad_r2[qb + q] <= own_lo2)
+                m[u] = make_ulonglong2(~0ull, 0ull);  // inside its owner
+            else
+                cell[u] = gbsw_sub_cell<EXACT>(p, sd, G, xi, yi, zi, qb + q, sub, bit[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kGbswBatch; ++u)
+            if (cell[u] >= 0) m[u] = p.cell_mask[cb + cell[u]];
+#pragma unroll
+        for (int u = 0; u < kGbswBatch; ++u) {
+            const int q = q0 + u * kGbswThreads + tid;
+            const bool in = (m[u].x >> bit[u]) & 1ull, queue = !in && !((m[u].y >> bit[u]) & 1ull);
+            if (q < Q) s_v[q] = in ? 0.f : 1.f;
+            const unsigned long long b = __ballot(queue);
+            if (b) {
+                int at = 0;
+                if (lane == 0) at = atomicAdd(&s_nq, __popcll(b));
+                at = __builtin_amdgcn_readfirstlane(at);
+                if (queue) s_q[at + __popcll(b & ((1ull << lane) - 1ull))] = (uint16_t)q;
+            }
+        }
+    }
+    __syncthreads();
+    const int nq = s_nq;
+    const float k1 = sd.k1, k3 = sd.k3, w = sd.sw;
+    int c = 0;
+    float r[3] = {0.f, 0.f, 0.f}, V = 1.f;
+    for (int e = tid; e < nq; e += kGbswThreads) {
+        const int q = s_q[e];
+        c = gbsw_place<EXACT>(p, sd, G, xi, yi, zi, qb + q, r);
+        int b = 0;
+        for (int d = 0; d < 3; ++d) b = b * kSub + min(max((int)(r[d] * sub[d]), 0), kSub - 1);
+        unsigned long long todo = p.cell_sub[(long long)(cb + c) * kWave + b];
+        const float4* ep = p.ent_pos + p.cell_start[cb + c];
+        V = 1.f;
+        auto smooth = [&](const float4& a) {  // H of one atom
+            const float dx = a.x - r[0], dy = a.y - r[1], dz = a.z - r[2];
+            const float x = fast_sqrt(fmaf(dx, dx, fmaf(dy, dy, dz * dz))) - a.w;
+            const float h = fmaxf(fmaf(x, fmaf(-k3 * x, x, k1), 0.5f), 0.f);
+            return x >= w ? 1.f : x <= -w ? 0.f : h;
+        };
+        if (todo == kSubScan) {
+            const int n = p.cell_count_eff[cb + c];
+            for (int m = 0; m < n && V != 0.f; ++m) V *= smooth(ep[m]);
+        } else {
+            while (todo != 0ull && V != 0.f) {  // two atoms at a time
+                const int m0 = __ffsll(todo) - 1;
+                todo &= todo - 1ull;
+                const bool two = todo != 0ull;
+                const int m1 = two ? __ffsll(todo) - 1 : m0;
+                todo &= todo - 1ull;  // (0 stays 0)
+                const float4 a0 = ep[m0], a1 = ep[m1];
+                V *= smooth(a0);
+                const float h1 = smooth(a1);
+                V *= two ? h1 : 1.f;
+            }
+        }
+        s_v[q] = V;
+        if (V > 0.f && V < 1.f) atomicOr(&s_bits[q >> 5], 1u << (q & 31));
+    }
+    __syncthreads();
+    if (wid == 0) {  // active points before each word of 32
+        const int n = __popc(s_bits[lane]);
+        const int incl = wave_scan_incl(n, lane);
+        s_pre[lane] = incl - n;
+        if (lane == kWave - 1) s_nact = incl;
+    }
+    __syncthreads();
+    for (int e = tid; e < nq; e += kGbswThreads) {
+        const int q = s_q[e];
+        const uint32_t word = s_bits[q >> 5], bit = 1u << (q & 31);
+        if (!(word & bit)) continue;
+        if (nq > kGbswThreads) {  // else this lane's registers still hold its only point
+            c = gbsw_place<EXACT>(p, sd, G, xi, yi, zi, qb + q, r);
+            V = s_v[q];
+        }
+        const int k = s_pre[q >> 5] + __popc(word & (bit - 1u));
+        int slot;
+        if (!EXACT && sd.grid_kind == GRID_BRUTE) {  // one cell: one atomic per wave
+            const unsigned long long m = __ballot(true);
+            const int first = __ffsll(m) - 1;
+            int at = 0;
+            if (lane == first) at = atomicAdd(&p.cell_ctr[cell_ctr_slot(p, cb)], __popcll(m));
+            slot = __shfl(at, first, kWave) + __popcll(m & ((1ull << lane) - 1ull));
+        } else {
+            slot = atomicAdd(&p.cell_ctr[cell_ctr_slot(p, cb + c)], 1);
+        }
+        if (slot >= sd.pt_cap) {
+            raise_flag(p, s, FLAG_POINT_OVERFLOW);
+            continue;
+        }
+        const long long o = sd.prec_base + (long long)c * sd.pt_cap + slot;
+        p.grec[o] = make_float4(r[0], r[1], r[2], __uint_as_float(((uint32_t)i << kQBits) | (uint32_t)q));
+        p.gval[o] = make_float2(V, __int_as_float(k));
+    }
+    double a0 = 0.0, a1 = 0.0;
+    for (int q = tid; q < Q; q += kGbswThreads) {
+        const double f = 1.0 - (double)s_v[q];
+        a0 += p.quad_pw[qb + q] * f;
+        a1 += p.quad_pw[p.quad_rows + qb + q] * f;
+    }
+    a0 = wave_sum(a0);
+    a1 = wave_sum(a1);
+    if (lane == 0) {
+        s_sum[0][wid] = a0;
+        s_sum[1][wid] = a1;
+    }
+    __syncthreads();
+    if (tid != 0) return;
+    p.atom_nact[i] = s_nact;
+    a0 = a1 = 0.0;
+    for (int k = 0; k < kGbswThreads / kWave; ++k) {
+        a0 += s_sum[0][k];
+        a1 += s_sum[1][k];
+    }
+    atom_integrals(p, sd, s, i, a0, a1);
+}
+
 // Cells holding points, one list per volume kind (order irrelevant: every later sum is
 // order independent).  One atomic per workgroup and kind: all of them go to one counter
 // per kind, which serialises them (one per wave took 0.009 ms for 770 waves at 5,000 atoms,
@@ -1076,10 +1406,9 @@ __global__ void __launch_bounds__(kWorkThreads) k_worklist(KParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Volume pass: one wave per cell, lanes = quadrature points, the cell's atoms staged in
-// LDS (corner-relative FP32).  Writes V per point (vval, by point; stored negated, -0 for
+// Volume pass of the GBMV kinds: one wave per cell, lanes = quadrature points, the cell's
+// atoms staged in LDS (corner-relative FP32).  Writes V per point (vval, by point; stored negated, -0 for
 // V = 0, on the points that carry a chain-rule factor) and their compacted records.
-// GBSW: V = prod_j H_j, early exit on burial (GBSWIntegral.cpp:187-224);
 // GBMV-I: S = sum exp(gamma_j d^4) (GBMVIntegralTypeI.cpp:155-173);
 // GBMV-II: sum1, sum2, v, S = S0 sum1 sum2/|v|^2 (GBMVIntegralTypeII.cpp:163-191).
 // ---------------------------------------------------------------------------
@@ -1109,7 +1438,7 @@ __device__ inline float volume_of(float vv) { return __int_as_float(__float_as_i
 template <int VK>
 __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
     __shared__ float s_x[kMaxAtomChunk], s_y[kMaxAtomChunk], s_z[kMaxAtomChunk];
-    __shared__ float s_a[kMaxAtomChunk], s_b[kMaxAtomChunk], s_c[kMaxAtomChunk];
+    __shared__ float s_a[kMaxAtomChunk], s_b[kMaxAtomChunk];
     if (batch_fatal(p)) return;
     const int lane = threadIdx.x;
     const int nwork = p.work[VK];
@@ -1133,9 +1462,9 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
         const bool ids = sd.sk > 1;  // the slots hold packed points (bricks), else records
         double corner[3];
         cell_corner(sd, G, c - sd.cell_base, corner);
-        const float k1 = sd.k1, k3 = sd.k3, fclamp = sd.fclamp, S0 = sd.S0, vguard = sd.vguard;
+        const float fclamp = sd.fclamp, S0 = sd.S0, vguard = sd.vguard;
         const float beta = sd.beta, lambda = sd.lambda;
-        const bool acc64 = VK != VOL_GBSW && sd.acc64;
+        const bool acc64 = sd.acc64;
         auto stage = [&](int ab, int cnt) {
             for (int k = lane; k < cnt; k += kWave) {
                 const float4 e = p.ent_pos[as + ab + k];
@@ -1143,15 +1472,8 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
                 s_x[k] = e.x;
                 s_y[k] = e.y;
                 s_z[k] = e.z;
-                s_a[k] = q.x;
-                s_b[k] = q.y;
-                s_c[k] = q.z;
-            }
-            if (VK == VOL_GBSW && lane < ((cnt + 3) & ~3) - cnt) {
-                // pad to a multiple of 4 with atoms that neither bury nor touch any point
-                const int k = cnt + lane;
-                s_x[k] = s_y[k] = s_z[k] = s_a[k] = 0.f;
-                s_b[k] = s_c[k] = -1.f;
+                s_a[k] = e.w;
+                s_b[k] = q.x;
             }
         };
         __syncthreads();
@@ -1174,8 +1496,6 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
             }
             const int i = (int)(pk >> kQBits), q = (int)(pk & ((1u << kQBits) - 1));
             const float prx = pr.x, pry = pr.y, prz = pr.z;
-            float V = 1.f;
-            bool done = !valid;
             float s1 = 0.f, s2 = 0.f, vx = 0.f, vy = 0.f, vz = 0.f;
             double S1 = 0.0, S2 = 0.0, VX = 0.0, VY = 0.0, VZ = 0.0;  // acc64 systems
             for (int ab = 0; ab < na; ab += kMaxAtomChunk) {
@@ -1185,25 +1505,7 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
                     stage(ab, cnt);
                     __syncthreads();
                 }
-                if (VK == VOL_GBSW) {
-                    // branch-free: H = 0 inside R' - w, the cubic in the shell, 1 beyond R' + w;
-                    // the wave leaves once every point is buried (V = 0), checked every 4 atoms
-                    if (done) V = 0.f;
-                    const int cnt4 = (cnt + 3) & ~3;
-                    for (int m = 0; m < cnt4; m += 4) {
-                        if (__all(V == 0.f)) break;
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            const float dx = s_x[m + u] - prx, dy = s_y[m + u] - pry, dz = s_z[m + u] - prz;
-                            const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                            const float x = fast_sqrt(d2) - s_a[m + u];
-                            float h = fmaxf(fmaf(x, fmaf(-k3 * x, x, k1), 0.5f), 0.f);
-                            h = d2 < s_c[m + u] ? h : 1.f;
-                            h = d2 <= s_b[m + u] ? 0.f : h;
-                            V *= h;
-                        }
-                    }
-                } else if (VK == VOL_GBMV2) {
+                if (VK == VOL_GBMV2) {
                     if (valid && !acc64) {
                         #pragma unroll 4
                         for (int m = 0; m < cnt; ++m) {
@@ -1256,11 +1558,7 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
             float4 r1 = make_float4(0.f, 0.f, 0.f, 0.f), r2 = make_float4(0.f, 0.f, 0.f, 0.f);
             if (valid) {
                 const int pid = pt_base + (i - abeg) * Q + q;
-                if (VK == VOL_GBSW) {
-                    active = V > 0.f && V < 1.f;
-                    p.vval[pid] = mark_active(V, active);
-                    r1.x = V;
-                } else if (VK == VOL_GBMV2) {
+                if (VK == VOL_GBMV2) {
                     float vsq, S, t;
                     bool guard;
                     if (acc64) {
@@ -1327,7 +1625,7 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
 
 // ---------------------------------------------------------------------------
 // Integrals and Born radii: one wave per atom, fixed-order FP64 sums over q.
-// I_k(i) = sum_q w_q / r_q^(n_k - 2) * (1 - V) [GBSW] or * V [GBMV]
+// I_k(i) = sum_q w_q / r_q^(n_k - 2) * (1 - V) [GBSW, in k_gbsw_points] or * V [GBMV]
 // (GBSWIntegral.cpp:142-146; GBMVIntegralTypeII.cpp:145-149).
 // B = slope / (a0 (1/eta - I4) + a1 (1/(4 eta^4) - I7)^(1/4)) + shift
 // (CharmmReferenceGBSW.cpp:591-593; dB/dI as :607-609).
@@ -1338,10 +1636,10 @@ __global__ void __launch_bounds__(64) k_integrals(KParams p) {
     const int i = blockIdx.x, lane = threadIdx.x;
     const int s = p.atom_sys[i];
     const SysDesc& sd = p.sys[s];
+    if (sd.vol_kind == VOL_GBSW) return;  // k_gbsw_points
     const int Q = sd.Q, qb = sd.quad_base;
     const int pbase = sd.pt_base + (i - sd.atom_begin) * Q;
     double a0 = 0.0, a1 = 0.0;
-    const bool gbsw = sd.vol_kind == VOL_GBSW;
     // Q a multiple of 4 (every system's points start on a multiple of 4): 4 points per lane
     // and load (0.045 -> 0.037 ms at 25k GBSW atoms), in a fixed order either way
     if ((Q & 3) == 0) {
@@ -1352,8 +1650,7 @@ __global__ void __launch_bounds__(64) k_integrals(KParams p) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int q = 4 * q4 + j;
-                const double v = (double)volume_of(vv[j]);
-                const double f = gbsw ? 1.0 - v : v;
+                const double f = (double)volume_of(vv[j]);
                 a0 += p.quad_pw[qb + q] * f;
                 a1 += p.quad_pw[p.quad_rows + qb + q] * f;
             }
@@ -1361,8 +1658,7 @@ __global__ void __launch_bounds__(64) k_integrals(KParams p) {
     } else {
 #pragma unroll 4
         for (int q = lane; q < Q; q += kWave) {
-            const double v = (double)volume_of(p.vval[pbase + q]);
-            const double f = gbsw ? 1.0 - v : v;
+            const double f = (double)volume_of(p.vval[pbase + q]);
             a0 += p.quad_pw[qb + q] * f;
             a1 += p.quad_pw[p.quad_rows + qb + q] * f;
         }
@@ -1370,20 +1666,7 @@ __global__ void __launch_bounds__(64) k_integrals(KParams p) {
     a0 = wave_sum(a0);
     a1 = wave_sum(a1);
     if (lane != 0) return;
-    p.integrals[i] = a0;
-    p.integrals[p.N + i] = a1;
-    if (sd.custom) return;  // the generated kernels map the integrals
-    const double I4 = sd.i4 == 0 ? a0 : a1;
-    const double I7 = sd.i7 == 0 ? a0 : a1;
-    const double eta = sd.eta;
-    const double eta4 = eta * eta * eta * eta;
-    const double T = 1.0 / (4.0 * eta4) - I7;
-    const double D = sd.alpha0 * (1.0 / eta - I4) + sd.alpha1 * pow(T, 0.25);
-    const double B = sd.slope / D + sd.shift;
-    p.born[i] = B;
-    p.dbdi[sd.i4 * p.N + i] = sd.slope * sd.alpha0 / (D * D);
-    p.dbdi[sd.i7 * p.N + i] = sd.slope * 0.25 * sd.alpha1 * pow(T, -0.75) / (D * D);
-    if (!isfinite(B) || !(B > 0.0)) raise_flag(p, s, FLAG_NONFINITE_RESULT);
+    atom_integrals(p, sd, s, i, a0, a1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1866,11 +2149,13 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
     for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
         const int c = worklist[w];
         const int s = worklist_sys[w];
-        const int nact = p.cell_act_count[c];
-        if (nact == 0) continue;
         const SysDesc sd = p.sys[s];  // a copy: read once per cell
+        const int nact = VK == VOL_GBSW ? min(p.cell_pt_count[c], sd.pt_cap) : p.cell_act_count[c];
+        if (nact == 0) continue;
         const int na = p.cell_count_eff[c];
-        const int ps = p.frec_base[c];
+        using RecIndex = std::conditional_t<VK == VOL_GBSW, long long, int>;
+        const RecIndex ps = VK == VOL_GBSW ? (RecIndex)(sd.prec_base + (long long)(c - sd.cell_base) * sd.pt_cap)
+                                           : (RecIndex)p.frec_base[c];
         const int as = p.cell_start[c];
         const int pt_base = sd.pt_base, abeg = sd.atom_begin, Q = sd.Q, qb = sd.quad_base;
         const float k1 = sd.k1, k3 = sd.k3, fclamp = sd.fclamp, sign_chain = sd.sign_chain;
@@ -1885,7 +2170,7 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
                 const int sl = ab + ag + 8 * k;
-                float4 e = make_float4(0.f, 0.f, 0.f, __int_as_float(-1)), q = make_float4(0.f, 0.f, 0.f, 0.f);
+                float4 e = make_float4(0.f, 0.f, 0.f, 0.f), q = make_float4(0.f, 0.f, __int_as_float(-1), 0.f);
                 if (sl < na) {
                     e = p.ent_pos[as + sl];
                     q = p.ent_par[as + sl];
@@ -1893,10 +2178,10 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
                 ax[k] = e.x;
                 ay[k] = e.y;
                 az[k] = e.z;
-                aj[k] = __float_as_int(e.w);
-                a0[k] = q.x;
-                a1[k] = q.y;
-                a2[k] = q.z;
+                a0[k] = e.w;
+                a1[k] = q.x;
+                a2[k] = q.y;
+                aj[k] = __float_as_int(q.z);
                 aR[k] = q.w;
             }
             double acc[8][3];
@@ -1914,9 +2199,17 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
                 const int cntp = min(kWave, nact - pb);
                 __syncthreads();
                 if (lane < cntp) {
-                    const int o = ps + pb + lane;
-                    const float4 r0 = p.frec0[o];
-                    const float4 r1 = p.frec1[o];
+                    const RecIndex o = ps + pb + lane;
+                    const float4 r0 = VK == VOL_GBSW ? p.grec[o] : p.frec0[o];
+                    float4 r1 = make_float4(0.f, 0.f, 0.f, 0.f);
+                    int own_slot = 0;  // GBSW: the point's rank among its owner's active points
+                    if (VK == VOL_GBSW) {
+                        const float2 g = p.gval[o];
+                        r1.x = g.x;
+                        own_slot = __float_as_int(g.y);
+                    } else {
+                        r1 = p.frec1[o];
+                    }
                     const uint32_t pk = __float_as_uint(r0.w);
                     const int i = (int)(pk >> kQBits), q = (int)(pk & ((1u << kQBits) - 1));
                     const double fac = p.dedi[i] * p.quad_pw[qb + q] + p.dedi[p.N + i] * p.quad_pw[p.quad_rows + qb + q];
@@ -1936,7 +2229,7 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
                         q_tf[lane] = !trunc || rq < sd.trunc_in ? 0 : (rq > sd.trunc_out ? 2 : 1);
                     }
                     q_own[lane] = i;
-                    q_pid[lane] = pt_base + (i - abeg) * Q + q;
+                    q_pid[lane] = pt_base + (i - abeg) * Q + (VK == VOL_GBSW ? own_slot : q);
                     if (VK == VOL_GBSW) {
                         q_0[lane] = facs;
                         q_1[lane] = r1.x;
@@ -2068,7 +2361,7 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
             // then every lane adds its atom's totals (the partials are integers on the 2^-24
             // grid, so any order gives the same sum)
             const int my_sl = ab + lane;
-            const int my_atom = my_sl < na ? __float_as_int(p.ent_pos[as + my_sl].w) : -1;
+            const int my_atom = my_sl < na ? __float_as_int(p.ent_par[as + my_sl].z) : -1;
             for (int d = 0; d < (ADJ ? 4 : 3); ++d) {
 #pragma unroll
                 for (int k = 0; k < 8; ++k) s_red[k][lane] = d < 3 ? acc[k][d] : accr[k];
@@ -2101,7 +2394,8 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
 }
 
 // Owner forces: one wave per atom, fixed-order FP64 sum of its points' owner forces, read
-// only where the sign bit of V marks a point with a chain-rule factor (V >= 0 always).
+// only where the sign bit of V marks a point with a chain-rule factor (V >= 0 always); GBSW
+// systems keep those points' forces together (about 66 of 912: 0.052 -> 0.012 ms at 25,000 atoms).
 // ADJ (GBMV): the sigmoid parts of dE/dbeta, dE/dlambda, dE/dS0 with
 // V = 1/(1 + exp(beta (S - lambda))): dV/dbeta = -V(1-V)(S - lambda), dV/dlambda = V(1-V) beta,
 // dV/dS0 = -V(1-V) beta S/S0; dE/dtheta = -sum s fac dV/dtheta.
@@ -2126,7 +2420,7 @@ __global__ void __launch_bounds__(64) k_owner_reduce(KParams p) {
         a[0] += marked ? (double)v.x : 0.0;
         a[1] += marked ? (double)v.y : 0.0;
         a[2] += marked ? (double)v.z : 0.0;
-        if (ADJ && !gbsw) {
+        if (ADJ) {
             const float S = p.vsig[pid];
             if (!isnan(S)) {
                 const double facs = sc * (e4 * p.quad_pw[qb + q] + e7 * p.quad_pw[p.quad_rows + qb + q]);
@@ -2138,7 +2432,15 @@ __global__ void __launch_bounds__(64) k_owner_reduce(KParams p) {
             }
         }
     };
-    if ((Q & 3) == 0) {  // 4 points per lane and load, as k_integrals
+    if (gbsw) {  // dense: the active points in q order (k_gbsw_points)
+        const int n = p.atom_nact[i];
+        for (int k = lane; k < n; k += kWave) {
+            const float4 v = p.vrec[pbase + k];
+            a[0] += (double)v.x;
+            a[1] += (double)v.y;
+            a[2] += (double)v.z;
+        }
+    } else if ((Q & 3) == 0) {  // 4 points per lane and load, as k_integrals
         const float4* v4 = reinterpret_cast<const float4*>(p.vval + pbase);
         for (int q4 = lane; q4 < (Q >> 2); q4 += kWave) {
             const float4 w = v4[q4];
@@ -2243,16 +2545,44 @@ __global__ void __launch_bounds__(kThetaThreads) k_theta_reduce(KParams p) {
 }
 
 // Points, point/atom pairs of the volume pass, and the active points and point/atom pairs
-// of the chain-rule pass (counts of the last evaluation; diagnostics only).
+// of the chain-rule pass (counts of the last evaluation; diagnostics only).  GBSW systems keep
+// no count of their points: k_stats_gbsw locates them again.
+__global__ void __launch_bounds__(kGbswThreads) k_stats_gbsw(KParams p, double* out) {
+    if (batch_fatal(p)) return;
+    const int i = blockIdx.x, s = p.atom_sys[i];
+    const SysDesc sd = p.sys[s];
+    if (sd.vol_kind != VOL_GBSW) return;
+    const SysGeom G = p.geom[s];
+    const float own_lo2 = sd.grid_kind != GRID_FAITHFUL ? p.aparam[i].y : -1.f;
+    double np = 0.0, pairs = 0.0;
+    for (int q = threadIdx.x; q < sd.Q; q += kGbswThreads) {
+        float r[3];
+        if (p.quad_r2[sd.quad_base + q] <= own_lo2) continue;
+        const int c = gbsw_locate(p, sd, G, p.pos[3 * i], p.pos[3 * i + 1], p.pos[3 * i + 2], sd.quad_base + q, r);
+        const int n = c >= 0 ? p.cell_count_eff[sd.cell_base + c] : 0;
+        np += n > 0 ? 1.0 : 0.0;
+        pairs += n;
+    }
+    np = wave_sum(np);
+    pairs = wave_sum(pairs);
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        atomicAdd(&out[0], np);
+        atomicAdd(&out[1], pairs);
+    }
+}
+
 __global__ void k_stats(KParams p, double* out) {
     if (batch_fatal(p)) return;
     double np = 0.0, pairs = 0.0, nact = 0.0, fpairs = 0.0;
     const int stride = gridDim.x * blockDim.x;
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < p.cell_total; c += stride) {
         const double a = p.cell_pt_count[c];
-        const double act = a > 0.0 ? p.cell_act_count[c] : 0.0;  // written only for cells with points
-        np += a;
-        pairs += a * p.cell_count_eff[c];
+        const bool gbsw = a > 0.0 && p.sys[p.cell_sys[c]].vol_kind == VOL_GBSW;  // its slots hold the active points
+        const double act = gbsw ? a : a > 0.0 ? p.cell_act_count[c] : 0.0;  // written only for cells with points
+        if (!gbsw) {
+            np += a;
+            pairs += a * p.cell_count_eff[c];
+        }
         nact += act;
         fpairs += act * p.cell_count_eff[c];
     }
@@ -2304,9 +2634,23 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
     err = scan_exclusive(p.cell_fill, p.cell_start, p.cell_total, p.scan_tmp, p.entry_cap, p.flags_all,
                          FLAG_ENTRY_OVERFLOW, stream);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(k_grid_sort, dim3(std::max(1, std::min(p.cell_total, 65536))), dim3(64), 0, stream, p);
+    const dim3 sort_grid(std::max(1, std::min(p.cell_total, 65536)));
+    if (kinds[VOL_GBSW])
+        hipLaunchKernelGGL(k_grid_sort<true>, sort_grid, dim3(64), 0, stream, p);
+    else
+        hipLaunchKernelGGL(k_grid_sort<false>, sort_grid, dim3(64), 0, stream, p);
     mark(1);
-    if (p.any_cells) hipLaunchKernelGGL(k_point_bin<false>, dim3(p.N), dim3(bin_threads<false>()), 0, stream, p);
+    // GBSW's volumes are k_gbsw_points' work, before the scan and the worklist: timed as the volume
+    // pass in contexts without GBMV systems, with the binning otherwise
+    const bool any_gbmv = kinds[VOL_GBMV1] || kinds[VOL_GBMV2];
+    if (!any_gbmv) mark(2);
+    if (kinds[VOL_GBSW]) {
+        const dim3 grid((p.N + kXcds - 1) / kXcds * kXcds);
+        const size_t lds = (size_t)p.gbsw_q * kGbswLds;
+        if (p.gbsw_exact) hipLaunchKernelGGL(k_gbsw_points<true>, grid, dim3(kGbswThreads), lds, stream, p);
+        if (p.gbsw_other) hipLaunchKernelGGL(k_gbsw_points<false>, grid, dim3(kGbswThreads), lds, stream, p);
+    }
+    if (p.any_cellbin) hipLaunchKernelGGL(k_point_bin<false>, dim3(p.N), dim3(bin_threads<false>()), 0, stream, p);
     if (p.any_bricks) hipLaunchKernelGGL(k_point_bin<true>, dim3(p.N), dim3(bin_threads<true>()), 0, stream, p);
     if (p.any_bricks)
         hipLaunchKernelGGL(k_point_split, dim3(std::max(1, std::min(p.brick_max, 4096)), p.S, kSplitParts), dim3(256),
@@ -2322,12 +2666,11 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
     hipLaunchKernelGGL(k_worklist, dim3(std::max(1, std::min((p.cell_total + kWorkThreads - 1) / kWorkThreads, 4096))),
                        dim3(kWorkThreads), 0, stream, p);
     const int pb = std::max(1, std::min(p.cell_total, p.persist_blocks));
-    mark(2);
-    if (kinds[VOL_GBSW]) hipLaunchKernelGGL(k_volume<VOL_GBSW>, dim3(pb), dim3(64), 0, stream, p);
+    if (any_gbmv) mark(2);
     if (kinds[VOL_GBMV1]) hipLaunchKernelGGL(k_volume<VOL_GBMV1>, dim3(pb), dim3(64), 0, stream, p);
     if (kinds[VOL_GBMV2]) hipLaunchKernelGGL(k_volume<VOL_GBMV2>, dim3(pb), dim3(64), 0, stream, p);
     mark(3);
-    hipLaunchKernelGGL(k_integrals, dim3(p.N), dim3(64), 0, stream, p);
+    if (any_gbmv) hipLaunchKernelGGL(k_integrals, dim3(p.N), dim3(64), 0, stream, p);
     mark(4);
     if (p.custom) {
         // general expressions (one system): values, pair tiles, chain
@@ -2442,6 +2785,7 @@ hipError_t launch_add_forces_fixed(long long* dst, int padded_n, const long long
 
 hipError_t launch_stats(const KParams& p, double* out6, hipStream_t stream) {
     hipLaunchKernelGGL(k_stats, dim3(256), dim3(256), 0, stream, p, out6);
+    hipLaunchKernelGGL(k_stats_gbsw, dim3(p.N), dim3(kGbswThreads), 0, stream, p, out6);
     return hipGetLastError();
 }
 
