@@ -1871,7 +1871,7 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
             clear(c.cell_act_count), clear(c.cell_sys), clear(c.cell_start), clear(c.frec_base), clear(c.worklist);
             clear(c.worklist_sys), clear(c.scan_tmp), clear(c.cell_atoms_tmp), clear(c.cell_atoms), clear(c.ent_pos);
             clear(c.ent_par), clear(c.prec), clear(c.frec0), clear(c.frec1), clear(c.frec2), clear(c.vval);
-            clear(c.vrec), clear(c.brick_count), clear(c.brick_rec), clear(c.cell_sub), clear(c.cell_mask), clear(c.grec);
+            clear(c.vrec), clear(c.brick_count), clear(c.brick_rec), clear(c.cell_mask), clear(c.grec);
             clear(c.gval), clear(c.atom_nact);
         }
     } unborrow{c};
@@ -1930,12 +1930,7 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     sc.take(c.prec, gbsw ? 1 : c.prec_total), sc.take(c.grec, gbsw ? c.prec_total : 1);
     sc.take(c.gval, gbsw ? c.prec_total : 1), sc.take(c.cell_mask, gbsw ? cells : 1), sc.take(c.atom_nact, gbsw ? N : 1);
     sc.take(c.frec0, gbsw ? 1 : NQ), sc.take(c.frec1, gbsw ? 1 : NQ);
-    sc.take(c.frec2, c.kinds[gbi::VOL_GBMV2] ? NQ : 1), sc.take(c.vval, gbsw ? 1 : NQ);
-    // the sub-cell lists are read last by the points' pass, before the chain-rule pass writes vrec:
-    // both in one piece
-    const size_t sub = gbsw ? 64 * cells : 0;
-    sc.take(c.vrec, std::max(NQ, (sub * sizeof(unsigned long long) + sizeof(float4) - 1) / sizeof(float4)));
-    c.cell_sub.p = reinterpret_cast<unsigned long long*>(c.vrec.p);
+    sc.take(c.frec2, c.kinds[gbi::VOL_GBMV2] ? NQ : 1), sc.take(c.vval, gbsw ? 1 : NQ), sc.take(c.vrec, NQ);
     sc.take(c.brick_count, gbi::kBrickStride), sc.take(c.brick_rec, 1);
     sc.take(c.bbox_part, (size_t)gbi::kBboxMaxSlices * gbi::kBboxPart), sc.take(c.bbox_done, 1);
     };

@@ -244,7 +244,8 @@ struct KParams {
     int gbsw_exact, gbsw_other;    // some GBSW system has the exact non-periodic grid, another one
     int gbsw_q;                    // the most points per atom of a GBSW system, rounded up to even
     ulonglong2* cell_mask;         // cell_total (null without GBSW systems): sub-cells with V = 0, with V = 1
-    unsigned long long* cell_sub;  // cell_total x 64 (GBSW cells with atoms): the atoms that reach each sub-cell
+    unsigned long long* cell_sub;  // cell_total x 64 (GBSW cells with atoms): the atoms that reach each sub-cell;
+                                   // null in gbi_execute_noalloc
     float4* grec;            // GBSW systems: slots of their active points (prec_base, pt_cap as in prec)
     float2* gval;            // per grec slot: V, rank among its owner's active points
     int* atom_nact;          // N: active points of each atom (GBSW)

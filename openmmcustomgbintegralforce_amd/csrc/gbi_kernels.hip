@@ -29,7 +29,6 @@
 #include <climits>
 #include <algorithm>
 #include <cmath>
-#include <type_traits>
 
 namespace gbi {
 
@@ -621,7 +620,7 @@ constexpr int kSortLds = 256;  // cells with more raw members sort in global mem
 // cell_mask: the sub-cells that the burial sphere R' - w of a list atom holds wholly (V = 0 at
 // every point) and those that no atom's switching sphere R' + w reaches (V = 1).  cell_sub, for
 // the others: bit m for each list atom m that reaches the sub-cell (the rest have H = 1 there),
-// or kSubScan in cells of more than 63 atoms.  k_gbsw_points reads V from the masks for 64 % of
+// or kSubScan in cells of more than 63 atoms; gbi_execute_noalloc has no room for them and scans.  k_gbsw_points reads V from the masks for 64 % of
 // the points outside their owner in a 25,000-atom globule (2 x 2 x 2 sub-cells: 36 %; 8 x 8 x 8:
 // 80 %, for 8 times this work) and runs the others down 6 atoms instead of 17.  kSubMargin exceeds
 // the rounding of the FP32 coordinates and distances (1e-7 nm), so a point has the V that its
@@ -632,9 +631,9 @@ constexpr unsigned long long kSubScan = 1ull << 63;
 
 __device__ inline void sub_cell_lists(const KParams& p, const SysDesc& sd, const SysGeom& G, int c, int base, int n,
                                       int lane, float4* s_e) {
-    unsigned long long* out = p.cell_sub + (long long)c * kWave + lane;
+    unsigned long long* out = p.cell_sub ? p.cell_sub + (long long)c * kWave + lane : nullptr;
     if (sd.grid_kind == GRID_BRUTE) {  // one cell without bounds: every point is evaluated
-        *out = kSubScan;
+        if (out) *out = kSubScan;
         if (lane == 0) p.cell_mask[c] = make_ulonglong2(0ull, 0ull);
         return;
     }
@@ -667,7 +666,7 @@ __device__ inline void sub_cell_lists(const KParams& p, const SysDesc& sd, const
         reach[(m0 >> 5) & 1] |= bits;
     }
     const unsigned long long r = ((unsigned long long)reach[1] << 32) | reach[0];
-    *out = n > 63 ? kSubScan : r;
+    if (out) *out = n > 63 ? kSubScan : r;
     const bool any = (reach[0] | reach[1]) != 0u;
     const unsigned long long in = __ballot(buried), out_of = __ballot(!any && !buried);
     if (lane == 0) p.cell_mask[c] = make_ulonglong2(in, out_of);
@@ -1256,7 +1255,7 @@ __global__ void __launch_bounds__(kGbswThreads) k_gbsw_points(KParams p) {
         c = gbsw_place<EXACT>(p, sd, G, xi, yi, zi, qb + q, r);
         int b = 0;
         for (int d = 0; d < 3; ++d) b = b * kSub + min(max((int)(r[d] * sub[d]), 0), kSub - 1);
-        unsigned long long todo = p.cell_sub[(long long)(cb + c) * kWave + b];
+        unsigned long long todo = p.cell_sub ? p.cell_sub[(long long)(cb + c) * kWave + b] : kSubScan;
         const float4* ep = p.ent_pos + p.cell_start[cb + c];
         V = 1.f;
         auto smooth = [&](const float4& a) {  // H of one atom
@@ -2105,7 +2104,7 @@ __global__ void __launch_bounds__(1024) k_energy(KParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Chain-rule force pass: one wave per cell.  Lanes form an 8 x 8 tile: lane = atom group
+// Chain-rule force pass of the GBMV kinds: one wave per cell.  Lanes form an 8 x 8 tile: lane = atom group
 // (lane & 7) x point group (lane >> 3); a lane owns 8 atoms of the chunk (registers) and
 // 8 points of each 64-point chunk (LDS).  For a point p of owner i with
 // fac = sum_k dE/dI_k(i) w_q / r_q^(n_k - 2) and s = +1 (GBSW) / -1 (GBMV):
@@ -2114,8 +2113,8 @@ __global__ void __launch_bounds__(1024) k_energy(KParams p) {
 // (GBSWIntegral.cpp:271-314, GBMVIntegralTypeI.cpp:195-224, GBMVIntegralTypeII.cpp:221-282;
 //  CharmmReferenceGBMV.cpp:376-383).  Atom partials are quantised to 2^-24 and summed
 // exactly in FP64, so the per-cell totals do not depend on the point order.
-// ADJ: also s fac dV_p/dR_j (GBSW: dR'_j) for every list atom including the owner, and
-// the per-system parameter sums (VolAcc).
+// ADJ: also s fac dV_p/dR_j for every list atom including the owner, and the per-system
+// parameter sums (VolAcc).
 // ---------------------------------------------------------------------------
 
 // Sum over the 8 lanes 8g..8g+7 (DPP: quad xor 1, quad xor 2, half-row mirror).
@@ -2126,15 +2125,9 @@ __device__ inline float sum8(float v) {
     return v;
 }
 
-// TRUNC (GBSW): the standalone force with a cutoff applies dB_i/dx_j only to list atoms j
-// within the cutoff of the owner i (minimum image); the owner still takes the whole sum
-// (CharmmReferenceGBSW.cpp:285-296).  The truncation shapes the forces only: with ADJ the
-// radius and constant derivatives, which differentiate the energy, take every list atom.
-template <int VK, bool ADJ, bool TRUNC>
-__global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p) {
+template <int VK, bool ADJ>
+__global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
     __shared__ float q_x[kWave], q_y[kWave], q_z[kWave];
-    __shared__ float q_w[TRUNC ? 3 : 1][kWave];  // TRUNC: owner position relative to the cell corner
-    __shared__ int q_tf[TRUNC ? kWave : 1];      // TRUNC: 0 every shell atom within c of the owner, 1 test, 2 none
     __shared__ float q_0[kWave], q_1[kWave], q_2[kWave], q_3[kWave], q_4[kWave], q_5[kWave];
     __shared__ int q_own[kWave], q_pid[kWave];
     // one axis of the per-lane atom partials at a time; rows padded by 8 doubles so the 8 rows
@@ -2150,19 +2143,13 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
         const int c = worklist[w];
         const int s = worklist_sys[w];
         const SysDesc sd = p.sys[s];  // a copy: read once per cell
-        const int nact = VK == VOL_GBSW ? min(p.cell_pt_count[c], sd.pt_cap) : p.cell_act_count[c];
+        const int nact = p.cell_act_count[c];
         if (nact == 0) continue;
         const int na = p.cell_count_eff[c];
-        using RecIndex = std::conditional_t<VK == VOL_GBSW, long long, int>;
-        const RecIndex ps = VK == VOL_GBSW ? (RecIndex)(sd.prec_base + (long long)(c - sd.cell_base) * sd.pt_cap)
-                                           : (RecIndex)p.frec_base[c];
+        const int ps = p.frec_base[c];
         const int as = p.cell_start[c];
         const int pt_base = sd.pt_base, abeg = sd.atom_begin, Q = sd.Q, qb = sd.quad_base;
-        const float k1 = sd.k1, k3 = sd.k3, fclamp = sd.fclamp, sign_chain = sd.sign_chain;
-        const float inv_sw = sd.inv_sw, P1x10 = 10.f * sd.P1;
-        const bool trunc = TRUNC && sd.chain_trunc;
-        BoxF bx;
-        if (TRUNC) bx = box_f(p, s, sd);
+        const float fclamp = sd.fclamp, sign_chain = sd.sign_chain, P1x10 = 10.f * sd.P1;
         double pacc0 = 0.0, pacc1 = 0.0;  // ADJ: VolAcc partials of this lane
         for (int ab = 0; ab < na; ab += kWave) {
             float ax[8], ay[8], az[8], a0[8], a1[8], a2[8], aR[8];
@@ -2199,17 +2186,9 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
                 const int cntp = min(kWave, nact - pb);
                 __syncthreads();
                 if (lane < cntp) {
-                    const RecIndex o = ps + pb + lane;
-                    const float4 r0 = VK == VOL_GBSW ? p.grec[o] : p.frec0[o];
-                    float4 r1 = make_float4(0.f, 0.f, 0.f, 0.f);
-                    int own_slot = 0;  // GBSW: the point's rank among its owner's active points
-                    if (VK == VOL_GBSW) {
-                        const float2 g = p.gval[o];
-                        r1.x = g.x;
-                        own_slot = __float_as_int(g.y);
-                    } else {
-                        r1 = p.frec1[o];
-                    }
+                    const int o = ps + pb + lane;
+                    const float4 r0 = p.frec0[o];
+                    const float4 r1 = p.frec1[o];
                     const uint32_t pk = __float_as_uint(r0.w);
                     const int i = (int)(pk >> kQBits), q = (int)(pk & ((1u << kQBits) - 1));
                     const double fac = p.dedi[i] * p.quad_pw[qb + q] + p.dedi[p.N + i] * p.quad_pw[p.quad_rows + qb + q];
@@ -2217,23 +2196,9 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
                     q_x[lane] = r0.x;
                     q_y[lane] = r0.y;
                     q_z[lane] = r0.z;
-                    if (TRUNC) {
-                        // shell atoms lie within max(R' + w) of the point, the point r_q from its
-                        // owner: r_q + reach below c keeps them all, r_q - reach above c none
-                        // (not periodic: another image may be nearer)
-                        const int row = qb + q;
-                        q_w[0][lane] = r0.x - (float)p.quad_off[3 * row];
-                        q_w[1][lane] = r0.y - (float)p.quad_off[3 * row + 1];
-                        q_w[2][lane] = r0.z - (float)p.quad_off[3 * row + 2];
-                        const float rq = fast_sqrt(p.quad_r2[row]);
-                        q_tf[lane] = !trunc || rq < sd.trunc_in ? 0 : (rq > sd.trunc_out ? 2 : 1);
-                    }
                     q_own[lane] = i;
-                    q_pid[lane] = pt_base + (i - abeg) * Q + (VK == VOL_GBSW ? own_slot : q);
-                    if (VK == VOL_GBSW) {
-                        q_0[lane] = facs;
-                        q_1[lane] = r1.x;
-                    } else if (VK == VOL_GBMV2) {
+                    q_pid[lane] = pt_base + (i - abeg) * Q + q;
+                    if (VK == VOL_GBMV2) {
                         const float4 r2 = p.frec2[o];
                         q_0[lane] = facs * r1.x;
                         q_1[lane] = facs * r1.y;
@@ -2258,9 +2223,6 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
                         const float vx = VK == VOL_GBMV2 ? q_3[m] : 0.f;
                         const float vy = VK == VOL_GBMV2 ? q_4[m] : 0.f;
                         const float vz = VK == VOL_GBMV2 ? q_5[m] : 0.f;
-                        const float wx = TRUNC ? q_w[0][m] : 0.f, wy = TRUNC ? q_w[1][m] : 0.f,
-                                    wz = TRUNC ? q_w[2][m] : 0.f;
-                        const int tf = TRUNC ? q_tf[m] : 0;
 #pragma unroll
                         for (int k = 0; k < 8; ++k) {
                             if (aj[k] < 0) continue;
@@ -2269,25 +2231,7 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
                             const float dx = ax[k] - px, dy = ay[k] - py, dz = az[k] - pz;
                             const float dd = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
                             float sv = 0.f, c3F = 0.f;
-                            if (VK == VOL_GBSW) {
-                                // shell atoms only: (R'-w)^2 < d^2 < (R'+w)^2
-                                if (dd < a2[k] && dd > a1[k]) {
-                                    const float d = fast_sqrt(dd);
-                                    const float x = d - a0[k];
-                                    const float h = fmaf(x, fmaf(-k3 * x, x, k1), 0.5f);
-                                    if (h > 0.f) {
-                                        const float dh = fmaf(-3.f * k3 * x, x, k1);
-                                        const float gV = d0 * (d1 * fast_rcp(h));  // s fac V / H_j
-                                        sv = gV * dh * fast_rcp(d);
-                                        if (ADJ) {
-                                            // dV/dR'_j = -V H'_j/H_j; dV/dw = V (dH_j/dw)/H_j
-                                            accr[k] += quant(-gV * dh);
-                                            const float xw = x * inv_sw;
-                                            pacc0 += quant(gV * 0.75f * xw * inv_sw * fmaf(xw, xw, -1.f));
-                                        }
-                                    }
-                                }
-                            } else if (VK == VOL_GBMV2) {
+                            if (VK == VOL_GBMV2) {
                                 const float tt = fmaf(100.f, dd, a1[k]);
                                 const float rt = fast_rcp(tt);
                                 const float ct = a0[k] * rt;
@@ -2320,21 +2264,9 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
                             const float cx = fmaf(sv, dx, c3F * vx);
                             const float cy = fmaf(sv, dy, c3F * vy);
                             const float cz = fmaf(sv, dz, c3F * vz);
-                            bool keep = !TRUNC || tf != 2;
-                            if (TRUNC && tf == 1 && sv != 0.f) {
-                                float ex = ax[k] - wx, ey = ay[k] - wy, ez = az[k] - wz;
-                                if (sd.periodic) {
-                                    ex = min_image(ex, bx.L[0], bx.inv[0]);
-                                    ey = min_image(ey, bx.L[1], bx.inv[1]);
-                                    ez = min_image(ez, bx.L[2], bx.inv[2]);
-                                }
-                                keep = within_cutoff(p, s, sd, fmaf(ex, ex, fmaf(ey, ey, ez * ez)), own, aj[k]);
-                            }
-                            if (keep) {
-                                acc[k][0] += quant(cx);
-                                acc[k][1] += quant(cy);
-                                acc[k][2] += quant(cz);
-                            }
+                            acc[k][0] += quant(cx);
+                            acc[k][1] += quant(cy);
+                            acc[k][2] += quant(cz);
                             ox += cx;
                             oy += cy;
                             oz += cz;
@@ -2385,10 +2317,181 @@ __global__ void __launch_bounds__(64, (ADJ || TRUNC) ? 2 : 3) k_force(KParams p)
             pacc1 = wave_sum(pacc1);
             if (lane == 0) {
                 long long* va = p.vacc_fix + ((long long)s * kVaccCopies + (w & (kVaccCopies - 1))) * kVaccStride;
-                const int i0 = VK == VOL_GBSW ? VA_W : VK == VOL_GBMV2 ? VA_A : VA_GAMMA;
+                const int i0 = VK == VOL_GBMV2 ? VA_A : VA_GAMMA;
                 if (pacc0 != 0.0) add_fix(&va[i0], pacc0);
                 if (VK == VOL_GBMV2 && pacc1 != 0.0) add_fix(&va[VA_AR], pacc1);
             }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Chain-rule force pass of GBSW: one wave per cell, lanes = active points, the cell's atoms in
+// LDS.  A lane runs down the atoms of its point's sub-cell (cell_sub, 6 on average) and takes
+// those whose shell |d - R'| < w holds the point (2 or 3): dV/dx_j = V H'_j/H_j (x_j - p)/d.  The
+// owner's force stays in the lane's registers; the atoms' partials, integers on the 2^-24 grid,
+// are added in LDS in FP64 (exact: any order gives the same sum), then one int64 atomic per
+// (cell, atom, axis) as for the other kinds.
+// The 8 x 8 tile of k_force visits every list atom of every point (17), and for 86 % of them
+// nothing is to be added, at 3 waves per SIMD (2 with TRUNC or ADJ); it took 0.133 ms at 25,000
+// atoms, this form 0.085 at 8 waves (TRUNC 0.25 -> 0.11, ADJ at 8 x 2,000 atoms 0.095 -> 0.053).
+// What bounds it: the chain of loads of each cell (worklist, cell, points, dE/dI); without the LDS
+// adds it takes 0.070 ms, without the int64 atomics 0.079, VALU issue is 0.03.
+// TRUNC: the standalone force with a cutoff applies dB_i/dx_j only to list atoms j within the
+// cutoff of the owner i (minimum image); the owner still takes the whole sum
+// (CharmmReferenceGBSW.cpp:285-296).  The truncation shapes the forces only: with ADJ the
+// radius and constant derivatives, which differentiate the energy, take every list atom.
+// ADJ: also s fac dV_p/dR'_j for every list atom including the owner, and dV/dw (VA_W).
+// ---------------------------------------------------------------------------
+template <bool ADJ, bool TRUNC>
+__global__ void __launch_bounds__(64) k_force_gbsw(KParams p) {
+    __shared__ float4 s_a[kWave];                 // (position - corner, R')
+    __shared__ int s_j[kWave];
+    __shared__ double s_f[ADJ ? 4 : 3][kWave];    // force partials; ADJ: dE/dR' partials
+    if (batch_fatal(p)) return;
+    const int lane = threadIdx.x;
+    const int nwork = p.work[VOL_GBSW];
+    const int* worklist = p.worklist + VOL_GBSW * p.cell_total;
+    const int* worklist_sys = p.worklist_sys + VOL_GBSW * p.cell_total;
+    for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
+        const int c = worklist[w];
+        const int s = worklist_sys[w];
+        const SysDesc sd = p.sys[s];  // a copy: read once per cell
+        const int np = min(p.cell_pt_count[c], sd.pt_cap);
+        const int na = p.cell_count_eff[c];
+        const int as = p.cell_start[c];
+        const long long ps = sd.prec_base + (long long)(c - sd.cell_base) * sd.pt_cap;
+        const bool single = na <= kWave;
+        const float k1 = sd.k1, k3 = sd.k3, sw = sd.sw;
+        float per_nm[3];  // sub-cells per nm
+        for (int d = 0; d < 3; ++d) per_nm[d] = kSub * fast_rcp((float)(sd.periodic ? p.geom[s].step[d] : sd.g));
+        BoxF bx;
+        if (TRUNC) bx = box_f(p, s, sd);
+        double pacc = 0.0;
+        auto stage = [&](int ab) {
+            const int k = ab + lane;
+            s_a[lane] = k < na ? p.ent_pos[as + k] : make_float4(0.f, 0.f, 0.f, 0.f);
+            s_j[lane] = k < na ? __float_as_int(p.ent_par[as + k].z) : -1;
+            for (int d = 0; d < (ADJ ? 4 : 3); ++d) s_f[d][lane] = 0.0;
+        };
+        auto flush = [&]() {  // lane = atom
+            const int j = s_j[lane];
+            for (int d = 0; d < (ADJ ? 4 : 3); ++d) {
+                const double tot = s_f[d][lane];
+                if (j < 0 || tot == 0.0) continue;
+                if (!(fabs(tot) < kFixLimit24))  // NaN, inf, or beyond the int64 range
+                    raise_flag(p, s, FLAG_NONFINITE_RESULT);
+                else if (d < 3)
+                    add_fix(&p.force_fix[d * p.N + j], tot);
+                else
+                    add_fix(&p.dedr_fix[j], tot);
+            }
+        };
+        if (single) stage(0);
+        __syncthreads();
+        for (int pb = 0; pb < np; pb += kWave) {
+            const bool valid = pb + lane < np;
+            float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+            float2 g = make_float2(0.f, 0.f);
+            if (valid) {
+                r = p.grec[ps + pb + lane];
+                g = p.gval[ps + pb + lane];
+            }
+            const uint32_t pk = __float_as_uint(r.w);
+            const int own = (int)(pk >> kQBits), row = sd.quad_base + (int)(pk & ((1u << kQBits) - 1));
+            int b = 0;
+            b = min(max((int)(r.x * per_nm[0]), 0), kSub - 1);
+            b = b * kSub + min(max((int)(r.y * per_nm[1]), 0), kSub - 1);
+            b = b * kSub + min(max((int)(r.z * per_nm[2]), 0), kSub - 1);
+            const unsigned long long near =
+                !valid ? 0ull : p.cell_sub ? p.cell_sub[(long long)c * kWave + b] : kSubScan;
+            float gV = 0.f;  // s fac V
+            // TRUNC: shell atoms lie within max(R' + w) of the point, the point r_q from its owner:
+            // r_q + reach below c keeps them all (0), r_q - reach above c none (2; not periodic:
+            // another image may be nearer), else each is tested (1)
+            int tf = 0;
+            float wx = 0.f, wy = 0.f, wz = 0.f;  // the owner relative to the corner
+            if (valid) {
+                const double fac = p.dedi[own] * p.quad_pw[row] + p.dedi[p.N + own] * p.quad_pw[p.quad_rows + row];
+                gV = sd.sign_chain * (float)fac * g.x;
+                if (TRUNC && sd.chain_trunc) {
+                    const float rq = fast_sqrt(p.quad_r2[row]);
+                    tf = rq < sd.trunc_in ? 0 : (rq > sd.trunc_out ? 2 : 1);
+                    wx = r.x - (float)p.quad_off[3 * row];
+                    wy = r.y - (float)p.quad_off[3 * row + 1];
+                    wz = r.z - (float)p.quad_off[3 * row + 2];
+                }
+            }
+            float ox = 0.f, oy = 0.f, oz = 0.f;
+            for (int ab = 0; ab < na; ab += kWave) {
+                if (!single) {
+                    __syncthreads();
+                    stage(ab);
+                    __syncthreads();
+                }
+                const int cnt = min(kWave, na - ab);
+                const unsigned long long all = cnt == kWave ? ~0ull : (1ull << cnt) - 1ull;
+                // the whole list where the sub-cells have no bits of their own (na > 63)
+                unsigned long long todo = near == kSubScan ? all : near;
+                while (todo != 0ull) {
+                    const int m = __ffsll(todo) - 1;
+                    todo &= todo - 1ull;
+                    const float4 a = s_a[m];
+                    const float dx = a.x - r.x, dy = a.y - r.y, dz = a.z - r.z;
+                    const float dd = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                    const float d = fast_sqrt(dd);
+                    const float x = d - a.w;
+                    const float h = fmaf(x, fmaf(-k3 * x, x, k1), 0.5f);
+                    if (!(fabsf(x) < sw && h > 0.f)) continue;
+                    const int j = s_j[m];
+                    const bool is_own = j == own;
+                    if (!ADJ && is_own) continue;
+                    const float dh = fmaf(-3.f * k3 * x, x, k1);
+                    const float gh = gV * fast_rcp(h) * dh;  // s fac V H'_j / H_j
+                    if (ADJ) {
+                        // dV/dR'_j = -V H'_j/H_j; dV/dw = V (dH_j/dw)/H_j
+                        unsafeAtomicAdd(&s_f[3][m], quant(-gh));
+                        const float xw = x * sd.inv_sw;
+                        pacc += quant(gV * fast_rcp(h) * 0.75f * xw * sd.inv_sw * fmaf(xw, xw, -1.f));
+                        if (is_own) continue;  // the owner moves with its points
+                    }
+                    const float sv = gh * fast_rcp(d);
+                    const float cx = sv * dx, cy = sv * dy, cz = sv * dz;
+                    ox += cx;
+                    oy += cy;
+                    oz += cz;
+                    bool keep = !TRUNC || tf != 2;
+                    if (TRUNC && tf == 1) {
+                        float ex = a.x - wx, ey = a.y - wy, ez = a.z - wz;
+                        if (sd.periodic) {
+                            ex = min_image(ex, bx.L[0], bx.inv[0]);
+                            ey = min_image(ey, bx.L[1], bx.inv[1]);
+                            ez = min_image(ez, bx.L[2], bx.inv[2]);
+                        }
+                        keep = within_cutoff(p, s, sd, fmaf(ex, ex, fmaf(ey, ey, ez * ez)), own, j);
+                    }
+                    if (keep) {
+                        unsafeAtomicAdd(&s_f[0][m], quant(cx));
+                        unsafeAtomicAdd(&s_f[1][m], quant(cy));
+                        unsafeAtomicAdd(&s_f[2][m], quant(cz));
+                    }
+                }
+                if (!single) {
+                    __syncthreads();
+                    flush();
+                }
+            }
+            if (valid)
+                p.vrec[sd.pt_base + (long long)(own - sd.atom_begin) * sd.Q + __float_as_int(g.y)] =
+                    make_float4(-ox, -oy, -oz, 0.f);
+        }
+        __syncthreads();
+        if (single) flush();
+        __syncthreads();  // the next cell stages over these
+        if (ADJ) {
+            pacc = wave_sum(pacc);
+            if (lane == 0 && pacc != 0.0)
+                add_fix(p.vacc_fix + ((long long)s * kVaccCopies + (w & (kVaccCopies - 1))) * kVaccStride + VA_W, pacc);
         }
     }
 }
@@ -2609,12 +2712,12 @@ void launch_force(const KParams& p, int vk, int blocks, hipStream_t stream) {
     switch (vk) {
     case VOL_GBSW:
         if (p.any_trunc)
-            hipLaunchKernelGGL((k_force<VOL_GBSW, ADJ, true>), dim3(blocks), dim3(64), 0, stream, p);
+            hipLaunchKernelGGL((k_force_gbsw<ADJ, true>), dim3(blocks), dim3(64), 0, stream, p);
         else
-            hipLaunchKernelGGL((k_force<VOL_GBSW, ADJ, false>), dim3(blocks), dim3(64), 0, stream, p);
+            hipLaunchKernelGGL((k_force_gbsw<ADJ, false>), dim3(blocks), dim3(64), 0, stream, p);
         break;
-    case VOL_GBMV1: hipLaunchKernelGGL((k_force<VOL_GBMV1, ADJ, false>), dim3(blocks), dim3(64), 0, stream, p); break;
-    default: hipLaunchKernelGGL((k_force<VOL_GBMV2, ADJ, false>), dim3(blocks), dim3(64), 0, stream, p); break;
+    case VOL_GBMV1: hipLaunchKernelGGL((k_force<VOL_GBMV1, ADJ>), dim3(blocks), dim3(64), 0, stream, p); break;
+    default: hipLaunchKernelGGL((k_force<VOL_GBMV2, ADJ>), dim3(blocks), dim3(64), 0, stream, p); break;
     }
 }
 
