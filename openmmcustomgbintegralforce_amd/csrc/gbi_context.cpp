@@ -55,6 +55,12 @@ constexpr int kDefaultBlocksPerCU = 128;  // about one workgroup per occupied ce
 // Cell edge of the exact GBSW grid (lists are exact at any edge): 0.20 nm measured fastest at
 // 5k and 25k atoms (0.15 nm: 14 % slower, more distinct cells to bin; 0.30 nm: longer lists).
 constexpr double kDefaultTightGrid = 0.20;
+// Form of a system's pair tiles, by its 64-atom blocks only, so that a system's sums are grouped
+// alike alone and in a batch.  Pair pass measured (us), 4 waves / one row block / two row blocks:
+// 300 atoms 9.4 / 14.2 / -, 2,500 12.9 / 17.6 / 25.6, 5,000 25.6 / 27.3 / 33.3, 8,000 59 / 46 / 48.6,
+// 12,000 - / 102 / 87, 25,000 - / 339 / 274.
+constexpr int kPairWaves4Blocks = 48;   // up to 3,072 atoms: 4 waves (no gain above in a batch)
+constexpr int kPairRows2Blocks = 140;   // from 8,897 atoms, without cutoffs or exclusions: two row blocks
 constexpr int kCutoffTileBlocks = 3;  // column blocks per pair tile of a cutoff system
 constexpr double kSigmoidFp64Above = 16.0;  // |beta lambda| above which GBMV sums S in FP64
 constexpr size_t kOwnAllocation = 2u << 20;  // bytes: a buffer not sub-allocated beside others
@@ -91,7 +97,7 @@ struct SysHost {
     long long cell_cap = 0;
     int pt_cap = 1;
     int tmp_cap = 0;  // raw member slots per cell: estimated from the positions, grown from the device counts
-    int pair_splits = 1, pair_k = 1, nblk = 1, blk_base = 0;
+    int pair_splits = 1, pair_k = 1, pair_rows = 1, nblk = 1, blk_base = 0;
     long long colpart_base = 0;
     double box[3] = {0.0, 0.0, 0.0};  // periodic box edges (gbi_set_periodic_box)
     bool box_set = false;
@@ -170,7 +176,7 @@ struct gbi_ctx {
     DevBuf<int> c_ex_ptr, c_ex_idx;
     bool any_cut = false, any_trunc = false;
     DevBuf<float> colpart;
-    int n_tiles = 0, max_splits = 1, n_colblocks = 0;
+    int n_tiles = 0, n_tiles4 = 0, n_tiles1 = 0, max_splits = 1, n_colblocks = 0;
     long long colpart_total = 1;
     DevBuf<double> pos, d_charge, d_radius, d_reach, quad_off, quad_pw, integrals, born, dbdi, dedi, pair_part,
         atom_energy, energy, stats, dedq, dedr, theta_atom, theta;
@@ -386,6 +392,7 @@ gbi::SysDesc make_desc(const gbi_ctx& c, const SysHost& s, long long cell_base, 
     d.cap = (P.cell_cap > 0 && s.kind != gbi::GRID_BRUTE) ? P.cell_cap : INT_MAX;
     d.pair_splits = s.pair_splits;
     d.pair_k = s.pair_k;
+    d.pair_rows = s.pair_rows;
     d.nblk = s.nblk;
     d.colpart_base = s.colpart_base;
     d.i4 = P.orders[0] == 4 ? 0 : 1;
@@ -521,51 +528,63 @@ gbi_status layout(gbi_ctx& c) {
     return GBI_OK;
 }
 
-// Pair tiles: row block I x column blocks [J0, J1) of the same system, J >= I (each
-// unordered pair once).  K column blocks per tile: `pair_columns` / 64 when set, else the
-// smallest K that keeps about 8192 tiles over the batch (every system's share of the block
-// pairs).  Column partials: one entry per (row block, atom) of each system.
+// Pair tiles: row block I (or blocks I, I + 1) x column blocks [J0, J1) of the same system,
+// J >= I (each unordered pair once).  K column blocks per tile: `pair_columns` / 64 when set, else the
+// smallest K that keeps about 12,800 tiles over the batch (every system's share of the block
+// pairs; with 8,192 the 25,000-atom pass and its reduction took 323 us, with 12,800 310).
+// Column partials: one entry per (row tile, atom) of each system.
 void tile_layout(gbi_ctx& c, std::vector<int4>& tiles, std::vector<int>& colblk) {
     long long pairs_total = 0;
     for (const SysHost& s : c.sys) {
         const long long nb = (s.N + 63) / 64;
         pairs_total += nb * (nb + 1) / 2;
     }
-    const long long target = 8192;
+    const long long target = 12800;
+    std::vector<int4> tiles1, tiles2;
     tiles.clear();
     colblk.clear();
     c.max_splits = 1;
     long long cp = 0;
     for (SysHost& s : c.sys) {
         const int nb = (s.N + 63) / 64;
+        const int R = !c.any_cut && !c.any_excl && !c.cprog && nb >= kPairRows2Blocks ? 2 : 1;
         int K;
         if (c.tuning.pair_columns > 0) {
             K = std::max(1, c.tuning.pair_columns / 64);
         } else {
             const long long pairs = (long long)nb * (nb + 1) / 2;
             const double share = (double)target * pairs / (double)pairs_total;  // tiles for this system
-            K = (int)std::ceil((double)pairs / std::max(1.0, share));
+            K = (int)std::ceil((double)pairs / R / std::max(1.0, share));
         }
         // cutoff systems: most block pairs are skipped and the work gathers near the diagonal,
         // so narrow tiles spread it (3 blocks measured best at 25k atoms, cutoff 0.5-1.6 nm)
         if (c.tuning.pair_columns <= 0 && s.cutoff()) K = std::min(K, kCutoffTileBlocks);
+        const bool small = nb <= kPairWaves4Blocks;
         K = std::max(1, std::min(K, nb));
         s.pair_k = K;
+        s.pair_rows = R;
         s.nblk = nb;
         s.pair_splits = (nb + K - 1) / K;  // pieces of row block 0, the most of any block
         s.colpart_base = cp;
         s.blk_base = (int)colblk.size();
-        cp += 64ll * nb * (nb - 1) / 2;  // row blocks I < J for every column block J
+        // row tiles that begin before column block J, for every J
+        cp += 64ll * (R == 1 ? (long long)nb * (nb - 1) / 2 : (long long)nb * nb / 4);
         c.max_splits = std::max(c.max_splits, s.pair_splits);
         for (int I = 0; I < nb; ++I) {
             colblk.push_back(s.atom_begin + 64 * I);
+            if (I % R != 0) continue;
             for (int J0 = I, k = 0; J0 < nb; J0 += K, ++k) {
                 const int J1 = std::min(nb, J0 + K);
-                tiles.push_back(make_int4(s.atom_begin + 64 * I, s.atom_begin + 64 * J0,
-                                          s.atom_begin + std::min(s.N, 64 * J1), k));
+                (small ? tiles : R == 1 ? tiles1 : tiles2)
+                    .push_back(make_int4(s.atom_begin + 64 * I, s.atom_begin + 64 * J0,
+                                         s.atom_begin + std::min(s.N, 64 * J1), k));
             }
         }
     }
+    c.n_tiles4 = (int)tiles.size();
+    c.n_tiles1 = (int)tiles1.size();
+    tiles.insert(tiles.end(), tiles1.begin(), tiles1.end());
+    tiles.insert(tiles.end(), tiles2.begin(), tiles2.end());
     c.n_tiles = (int)tiles.size();
     c.n_colblocks = (int)colblk.size();
     c.colpart_total = std::max<long long>(1, cp);
@@ -816,6 +835,8 @@ gbi::KParams make_kparams(gbi_ctx& c, bool adjoint) {
     k.cell_total = (int)c.cell_total;
     k.entry_cap = c.entry_cap;
     k.n_tiles = c.n_tiles;
+    k.n_tiles4 = c.n_tiles4;
+    k.n_tiles1 = c.n_tiles1;
     k.max_splits = c.max_splits;
     k.n_colblocks = c.n_colblocks;
     k.colpart_total = c.colpart_total;
@@ -1558,7 +1579,13 @@ gbi_status gbi_set_exclusions(gbi_ctx* ctx, int32_t system, int32_t n_pairs, con
             return fail(GBI_ERR_INVALID_ARGUMENT, "excluded pair out of range or of an atom with itself");
     s.excl.assign(pairs, pairs + 2 * (size_t)n_pairs);
     if (ctx->cprog) return build_custom_exclusions(*ctx);
-    return build_exclusions(*ctx);
+    const bool before = ctx->any_excl;
+    ST_TRY(build_exclusions(*ctx));
+    if (ctx->any_excl != before) {  // tiles of two row blocks take no exclusions
+        ST_TRY(build_tiles(*ctx));
+        if (ctx->cell_total > 0) ST_TRY(layout(*ctx));  // the tiles' shape lives in the descriptors
+    }
+    return GBI_OK;
 }
 
 gbi_status gbi_create_custom(int32_t n_atoms, const gbi_params* params, const gbi_custom_spec* spec, gbi_ctx** out) {

@@ -104,8 +104,9 @@ struct SysDesc {
     int cap;                   // atoms kept per cell
     int pair_splits;           // pair tiles of row block 0 (the most of any block)
     int pair_k;                // column blocks per pair tile
+    int pair_rows;             // row blocks per pair tile: 1, or 2 (k_pairs2)
     int nblk;                  // 64-atom blocks
-    long long colpart_base;    // column partials (row block I < block J of atom j): colpart_base + 64 (J(J-1)/2 + I) + j % 64
+    long long colpart_base;    // column partials of the system (colpart_index)
     int i4, i7;                // which integral is order 4 / 7
     // nonbonded method
     int periodic;              // rectangular periodic box (KParams::box), lookup grid tiling it
@@ -174,6 +175,8 @@ struct KParams {
     int cell_total;          // sum of the systems' cell ranges
     int entry_cap;
     int n_tiles;             // pair tiles
+    int n_tiles4;            // those of small systems (4 waves each), which come first
+    int n_tiles1;            // those of one row block, which come next; the rest have two
     int max_splits;          // pair_part planes (row pieces of block 0, the most of any block)
     int n_colblocks;         // 64-atom blocks of all systems (k_atom_chain workgroups)
     long long colpart_total; // column partial entries per plane

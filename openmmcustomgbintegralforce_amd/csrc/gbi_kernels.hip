@@ -1684,8 +1684,45 @@ __global__ void __launch_bounds__(64) k_integrals(KParams p) {
 // One pair's terms (from i's side: d = x_j - x_i).  ex = exp(-r^2/(4 B_i B_j)) as
 // exp2(-(r^2 kexp_i) / B_j) with kexp_i = log2(e) / (4 B_i); rf = 1/f.
 struct PairTerms {
-    float dx, dy, dz, r2, ex, rf;
+    float dx, dy, dz, r2, bb, ex, rf;
 };
+
+// Sums over one block's pairs of a row or a column atom.  g = t3 ex (r^2/4 + B_i B_j), the same on
+// both sides: dE/dB_i = -g / (2 B_i).
+struct PairSums {
+    float e, fx, fy, fz, g, dq;
+    __device__ void add(const PairSums& o) {
+        e += o.e;
+        fx += o.fx;
+        fy += o.fy;
+        fz += o.fz;
+        g += o.g;
+        dq += o.dq;
+    }
+};
+
+// One pair's terms into its row atom's sums and, off the diagonal blocks (COL), its column
+// atom's.  qq = P q_i q_j, pi = P q_i, pj = P q_j.
+template <bool ADJ, bool COL>
+__device__ inline void add_pair(const PairTerms& t, float qq, float pi, float pj, PairSums& row, PairSums& col) {
+    const float e = qq * t.rf;
+    row.e += e;
+    const float t3 = e * (t.rf * t.rf);
+    const float dGdr = t3 * fmaf(0.25f, t.ex, -1.f);  // -P q_i q_j (4 - ex) / (4 f^3)
+    const float te = t3 * t.ex, u = fmaf(0.25f, t.r2, t.bb);
+    row.fx = fmaf(t.dx, dGdr, row.fx);
+    row.fy = fmaf(t.dy, dGdr, row.fy);
+    row.fz = fmaf(t.dz, dGdr, row.fz);
+    row.g = fmaf(te, u, row.g);
+    if (ADJ) row.dq = fmaf(pj, t.rf, row.dq);
+    if (COL) {
+        col.fx = fmaf(-t.dx, dGdr, col.fx);
+        col.fy = fmaf(-t.dy, dGdr, col.fy);
+        col.fz = fmaf(-t.dz, dGdr, col.fz);
+        col.g = fmaf(te, u, col.g);
+        if (ADJ) col.dq = fmaf(pi, t.rf, col.dq);
+    }
+}
 
 __device__ inline PairTerms pair_terms(double xj, double yj, double zj, double xi, double yi, double zi, float Bi,
                                        float Bj, float kexp_i, float iBj) {
@@ -1694,8 +1731,9 @@ __device__ inline PairTerms pair_terms(double xj, double yj, double zj, double x
     t.dy = (float)(yj - yi);
     t.dz = (float)(zj - zi);
     t.r2 = fmaf(t.dx, t.dx, fmaf(t.dy, t.dy, t.dz * t.dz));
+    t.bb = Bi * Bj;
     t.ex = __builtin_amdgcn_exp2f(-(t.r2 * kexp_i) * iBj);
-    t.rf = __builtin_amdgcn_rsqf(fmaf(Bi * Bj, t.ex, t.r2));
+    t.rf = __builtin_amdgcn_rsqf(fmaf(t.bb, t.ex, t.r2));
     return t;
 }
 
@@ -1754,8 +1792,9 @@ __device__ inline PairTerms pair_terms_cut(double xj, double yj, double zj, doub
         t.dz = min_image(t.dz, bx.L[2], bx.inv[2]);
     }
     t.r2 = fmaf(t.dx, t.dx, fmaf(t.dy, t.dy, t.dz * t.dz));
+    t.bb = Bi * Bj;
     t.ex = __builtin_amdgcn_exp2f(-(t.r2 * kexp_i) * iBj);
-    t.rf = __builtin_amdgcn_rsqf(fmaf(Bi * Bj, t.ex, t.r2));
+    t.rf = __builtin_amdgcn_rsqf(fmaf(t.bb, t.ex, t.r2));
     return t;
 }
 
@@ -1805,11 +1844,13 @@ __device__ inline bool blocks_apart(const KParams& p, const SysDesc& sd, const B
     return gap2 > sd.cut2_hi * 1.001f;
 }
 
-// Column partial of row block I for local atom j (block J = j / 64 > I): triangular, the
-// row blocks of one column block stored one after the other, 64 atoms each.
-__device__ inline long long colpart_index(const SysDesc& sd, int I, int j) {
+// Column partial of row tile t for local atom j (a row tile holds pair_rows blocks of 64; block
+// J = j / 64 meets the tiles that begin before it): triangular, the row tiles of one column block
+// stored one after the other, 64 atoms each.
+__device__ inline long long colpart_index(const SysDesc& sd, int t, int j) {
     const long long J = j / kWave;
-    return sd.colpart_base + (long long)kWave * (J * (J - 1) / 2 + I) + (j - kWave * J);
+    const long long before = sd.pair_rows == 1 ? J * (J - 1) / 2 : J * J / 4;
+    return sd.colpart_base + (long long)kWave * (before + t) + (j - kWave * J);
 }
 
 // Lane l receives lane l + 1's value (mod 64): DPP wave_rol:1.
@@ -1817,19 +1858,46 @@ __device__ inline float rotate_down(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x134, 0xF, 0xF, false));
 }
 
+// The column sums move one lane down, so that after 64 steps lane l holds column l's.
+template <bool ADJ>
+__device__ inline void rotate_sums(PairSums& c) {
+    c.fx = rotate_down(c.fx);
+    c.fy = rotate_down(c.fy);
+    c.fz = rotate_down(c.fz);
+    c.g = rotate_down(c.g);
+    if (ADJ) c.dq = rotate_down(c.dq);
+}
+
+// half = -1/(2 B) of the column atom.
+template <bool ADJ>
+__device__ inline void store_column(const KParams& p, long long o, const PairSums& c, float half) {
+    const long long T = p.colpart_total;
+    p.colpart[o] = c.fx;
+    p.colpart[T + o] = c.fy;
+    p.colpart[2 * T + o] = c.fz;
+    p.colpart[3 * T + o] = half * c.g;
+    if (ADJ) p.colpart[4 * T + o] = c.dq;
+}
+
 // CUT: systems with a cutoff drop the pairs outside it (rf = 0 zeroes every term), reduce
 // periodic differences to the minimum image (positions wrapped into the box on load, so one
 // box vector at most) and skip column blocks whose bounding boxes are beyond the cutoff
 // (their column partials are written as zeros); excluded pairs (a ParticlePair term,
 // CharmmReferenceGBMV.cpp:272-284) are dropped through the block's 64 x 64 bit mask.
-template <bool ADJ, bool CUT>
-__global__ void __launch_bounds__(64) k_pairs(KParams p) {
+// WAVES: 4 for small systems, whose tiles leave the chip idle: each wave takes 16 of a block's 64
+// column steps, and the waves' sums are added in wave order through LDS.
+template <bool ADJ, bool CUT, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) k_pairs(KParams p) {
+    constexpr int kSteps = kWave / WAVES;
     __shared__ double s_px[64], s_py[64], s_pz[64];
-    __shared__ float4 s_col[64];  // (q, B, 1/B, 1/(4B))
+    __shared__ float4 s_col[64];  // (q, B, 1/B, -1/(2B))
     __shared__ int s_atom[64];
+    __shared__ PairSums s_row[WAVES > 1 ? WAVES : 1][WAVES > 1 ? kWave : 1];
+    __shared__ PairSums s_cs[WAVES > 1 ? WAVES : 1][WAVES > 1 ? kWave : 1];
     if (batch_fatal(p)) return;
-    const int lane = threadIdx.x;
-    const int4 tile = p.pair_tiles[blockIdx.x];
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    // the tiles of 4 waves come first, then those of one row block, then those of two
+    const int4 tile = p.pair_tiles[(WAVES == 1 ? p.n_tiles4 : 0) + blockIdx.x];
     const int s = p.atom_sys[tile.x];
     const SysDesc sd = p.sys[s];  // a copy: read once
     const int ab = sd.atom_begin, ae = sd.atom_end;
@@ -1858,23 +1926,14 @@ __global__ void __launch_bounds__(64) k_pairs(KParams p) {
     const float qi = iv ? (float)p.charge[ai] : 0.f;  // zero charge: an absent row adds nothing
     const float Bi = iv ? (float)p.born[ai] : 1.f;
     const float Pq = P * qi;
-    const float q4Bi = 0.25f / Bi;
-    const float kexp = 1.4426950408889634f * q4Bi;
+    const float kexp = 1.4426950408889634f * (0.25f / Bi), half = -0.5f / Bi;
     const int I_row = (tile.x - ab) / kWave;
     double fx = 0.0, fy = 0.0, fz = 0.0, dedb = 0.0, e = 0.0, dq = 0.0;
     for (int jb = tile.y; jb < tile.z; jb += kWave) {
         const int jj = jb + lane;
         const bool jv = jj < ae;
         if (cut && jb != tile.x && blocks_apart(p, sd, bx, sd.blk_base + I_row, sd.blk_base + (jb - ab) / kWave)) {
-            if (jv) {
-                const long long o = colpart_index(sd, I_row, jj - ab);
-                const long long T = p.colpart_total;
-                p.colpart[o] = 0.f;
-                p.colpart[T + o] = 0.f;
-                p.colpart[2 * T + o] = 0.f;
-                p.colpart[3 * T + o] = 0.f;
-                if (ADJ) p.colpart[4 * T + o] = 0.f;
-            }
+            if (jv && wid == 0) store_column<ADJ>(p, colpart_index(sd, I_row, jj - ab), PairSums{}, 0.f);
             continue;
         }
         unsigned long long emask = 0ull;  // bit c: pair (this row, column c of the block) excluded
@@ -1887,9 +1946,9 @@ __global__ void __launch_bounds__(64) k_pairs(KParams p) {
                 }
         }
         __syncthreads();
-        const int aj = jv ? p.pair_atom[jj] : 0;
-        s_atom[lane] = aj;
-        {
+        if (wid == 0) {
+            const int aj = jv ? p.pair_atom[jj] : 0;
+            s_atom[lane] = aj;
             double xj = jv ? p.pos[3 * aj] : 0.0, yj = jv ? p.pos[3 * aj + 1] : 0.0, zj = jv ? p.pos[3 * aj + 2] : 0.0;
             if (per) {
                 xj = wrap_box(xj, Lx);
@@ -1899,18 +1958,16 @@ __global__ void __launch_bounds__(64) k_pairs(KParams p) {
             s_px[lane] = xj;
             s_py[lane] = yj;
             s_pz[lane] = zj;
-        }
-        {
             const float Bj = jv ? (float)p.born[aj] : 1.f;
             const float iB = 1.f / Bj;
-            s_col[lane] = make_float4(jv ? (float)p.charge[aj] : 0.f, Bj, iB, 0.25f * iB);
+            s_col[lane] = make_float4(jv ? (float)p.charge[aj] : 0.f, Bj, iB, -0.5f * iB);
         }
         __syncthreads();
-        float efs = 0.f, dqs = 0.f, fxs = 0.f, fys = 0.f, fzs = 0.f, dbs = 0.f;
+        PairSums row = {}, col = {};
         if (jb == tile.x) {
             // diagonal block: ordered pairs from the row side, half the pair energy each
-            const int cnt = min(kWave, ae - jb);
-            for (int m = 0; m < cnt; ++m) {
+            const int cnt = min((wid + 1) * kSteps, ae - jb);
+            for (int m = wid * kSteps; m < cnt; ++m) {
                 if (jb + m == i) continue;
                 const float4 cj = s_col[m];
                 PairTerms t;
@@ -1921,20 +1978,13 @@ __global__ void __launch_bounds__(64) k_pairs(KParams p) {
                     t = pair_terms(s_px[m], s_py[m], s_pz[m], xi, yi, zi, Bi, cj.y, kexp, cj.z);
                 }
                 if (CUT && ((emask >> m) & 1ull)) t.rf = 0.f;
-                const float eij = Pq * cj.x * t.rf;
-                efs = fmaf(0.5f, eij, efs);
-                if (ADJ) dqs = fmaf(P * cj.x, t.rf, dqs);
-                const float t3 = eij * (t.rf * t.rf);
-                const float dGdr = t3 * fmaf(0.25f, t.ex, -1.f);  // -Pqq (4 - ex) / (4 f^3)
-                fxs = fmaf(t.dx, dGdr, fxs);
-                fys = fmaf(t.dy, dGdr, fys);
-                fzs = fmaf(t.dz, dGdr, fzs);
-                dbs = fmaf(-0.5f * t3 * t.ex, fmaf(t.r2, q4Bi, cj.y), dbs);
+                add_pair<ADJ, false>(t, Pq * cj.x, Pq, P * cj.x, row, col);
             }
+            row.e *= 0.5f;
         } else {
             // off-diagonal block: each unordered pair once, column sums rotate through the lanes
-            float cfx = 0.f, cfy = 0.f, cfz = 0.f, cdb = 0.f, cdq = 0.f;
-            for (int m = 0; m < kWave; ++m) {
+#pragma unroll 2
+            for (int m = wid * kSteps; m < (wid + 1) * kSteps; ++m) {
                 const int c = (lane + m) & (kWave - 1);
                 const float4 cj = s_col[c];
                 PairTerms t;
@@ -1945,47 +1995,32 @@ __global__ void __launch_bounds__(64) k_pairs(KParams p) {
                     t = pair_terms(s_px[c], s_py[c], s_pz[c], xi, yi, zi, Bi, cj.y, kexp, cj.z);
                 }
                 if (CUT && ((emask >> c) & 1ull)) t.rf = 0.f;
-                const float eij = Pq * cj.x * t.rf;  // P q_i q_j / f
-                efs += eij;
-                const float t3 = eij * (t.rf * t.rf);
-                const float dGdr = t3 * fmaf(0.25f, t.ex, -1.f);  // -Pqq (4 - ex) / (4 f^3)
-                const float hb = -0.5f * t3 * t.ex;               // dE/dB_i = hb (r^2/(4B_i) + B_j)
-                fxs = fmaf(t.dx, dGdr, fxs);
-                fys = fmaf(t.dy, dGdr, fys);
-                fzs = fmaf(t.dz, dGdr, fzs);
-                cfx = fmaf(-t.dx, dGdr, cfx);
-                cfy = fmaf(-t.dy, dGdr, cfy);
-                cfz = fmaf(-t.dz, dGdr, cfz);
-                dbs = fmaf(hb, fmaf(t.r2, q4Bi, cj.y), dbs);
-                cdb = fmaf(hb, fmaf(t.r2, cj.w, Bi), cdb);
-                if (ADJ) {
-                    dqs = fmaf(P * cj.x, t.rf, dqs);
-                    cdq = fmaf(Pq, t.rf, cdq);
-                }
-                cfx = rotate_down(cfx);
-                cfy = rotate_down(cfy);
-                cfz = rotate_down(cfz);
-                cdb = rotate_down(cdb);
-                if (ADJ) cdq = rotate_down(cdq);
+                add_pair<ADJ, true>(t, Pq * cj.x, Pq, P * cj.x, row, col);
+                rotate_sums<ADJ>(col);
             }
-            if (jv) {
-                const long long o = colpart_index(sd, I_row, jj - ab);
-                const long long T = p.colpart_total;
-                p.colpart[o] = cfx;
-                p.colpart[T + o] = cfy;
-                p.colpart[2 * T + o] = cfz;
-                p.colpart[3 * T + o] = cdb;
-                if (ADJ) p.colpart[4 * T + o] = cdq;
+            if (WAVES == 1 && jv) store_column<ADJ>(p, colpart_index(sd, I_row, jj - ab), col, s_col[lane].w);
+        }
+        if (WAVES > 1) {
+            s_row[wid][lane] = row;
+            s_cs[wid][(lane + (wid + 1) * kSteps) & (kWave - 1)] = col;  // lane l's sums are this column's now
+            __syncthreads();
+            if (wid == 0) {  // the rows
+                row = {};
+                for (int k = 0; k < WAVES; ++k) row.add(s_row[k][lane]);
+            } else if (wid == 1 && jb != tile.x && jv) {  // the columns
+                col = {};
+                for (int k = 0; k < WAVES; ++k) col.add(s_cs[k][lane]);
+                store_column<ADJ>(p, colpart_index(sd, I_row, jj - ab), col, s_col[lane].w);
             }
         }
-        e += efs;
-        fx += fxs;
-        fy += fys;
-        fz += fzs;
-        dedb += dbs;
-        if (ADJ) dq += dqs;
+        e += row.e;
+        fx += row.fx;
+        fy += row.fy;
+        fz += row.fz;
+        dedb += half * row.g;
+        if (ADJ) dq += row.dq;
     }
-    if (iv) {
+    if (iv && wid == 0) {
         double* out = p.pair_part + (size_t)tile.w * 6 * p.N;
         out[i] = fx;
         out[p.N + i] = fy;
@@ -1996,10 +2031,114 @@ __global__ void __launch_bounds__(64) k_pairs(KParams p) {
     }
 }
 
+// Two row blocks per wave (pair_rows = 2), for large systems without cutoff or exclusions: lane l
+// holds rows l and 64 + l, which meet column (l + m) mod 64 together, so its LDS reads and the
+// rotation of its sums are paid once for two pairs (36 VALU slots per pair against 38, 44 before
+// dE/dB took one term for both atoms), and the column partials halve.  25,000 atoms: 0.368 -> 0.274
+// ms, VALU-bound (312 M pairs at 36 slots of 4.5 cycles: 0.31 ms at 2.4 GHz on 1,024 SIMDs).  A
+// tile's first two column blocks are its rows' own: the diagonal block of each row block, and
+// their mutual block once.
+template <bool ADJ>
+__global__ void __launch_bounds__(64) k_pairs2(KParams p) {
+    __shared__ double s_px[64], s_py[64], s_pz[64];
+    __shared__ float4 s_col[64];  // (q, B, 1/B, -1/(2B))
+    if (batch_fatal(p)) return;
+    const int lane = threadIdx.x;
+    const int4 tile = p.pair_tiles[p.n_tiles4 + p.n_tiles1 + blockIdx.x];
+    const int s = p.atom_sys[tile.x];
+    const SysDesc sd = p.sys[s];  // a copy: read once
+    const int ab = sd.atom_begin, ae = sd.atom_end;
+    const float P = (float)sd.prefactor;
+    double x[2], y[2], z[2];
+    float Pq[2], B[2], kexp[2], half[2];
+    bool iv[2];
+    double out[2][6] = {};
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int i = tile.x + kWave * r + lane;
+        iv[r] = i < ae;
+        const int ai = iv[r] ? p.pair_atom[i] : 0;
+        x[r] = iv[r] ? p.pos[3 * ai] : 0.0;
+        y[r] = iv[r] ? p.pos[3 * ai + 1] : 0.0;
+        z[r] = iv[r] ? p.pos[3 * ai + 2] : 0.0;
+        Pq[r] = iv[r] ? P * (float)p.charge[ai] : 0.f;  // zero charge: an absent row adds nothing
+        B[r] = iv[r] ? (float)p.born[ai] : 1.f;
+        kexp[r] = 1.4426950408889634f * (0.25f / B[r]);
+        half[r] = -0.5f / B[r];
+    }
+    for (int jb = tile.y; jb < tile.z; jb += kWave) {
+        const int jj = jb + lane;
+        const bool jv = jj < ae;
+        __syncthreads();
+        {
+            const int aj = jv ? p.pair_atom[jj] : 0;
+            s_px[lane] = jv ? p.pos[3 * aj] : 0.0;
+            s_py[lane] = jv ? p.pos[3 * aj + 1] : 0.0;
+            s_pz[lane] = jv ? p.pos[3 * aj + 2] : 0.0;
+            const float Bj = jv ? (float)p.born[aj] : 1.f, iB = 1.f / Bj;
+            s_col[lane] = make_float4(jv ? (float)p.charge[aj] : 0.f, Bj, iB, -0.5f * iB);
+        }
+        __syncthreads();
+        PairSums row[2] = {}, col = {};
+        auto pair = [&](int r, int c) {
+            const float4 cj = s_col[c];
+            return pair_terms(s_px[c], s_py[c], s_pz[c], x[r], y[r], z[r], B[r], cj.y, kexp[r], cj.z);
+        };
+        const int own = (jb - tile.x) / kWave;  // 0, 1: the block of these rows
+        if (own > 1) {
+            for (int m = 0; m < kWave; ++m) {
+                const int c = (lane + m) & (kWave - 1);
+                const float4 cj = s_col[c];
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+                    add_pair<ADJ, true>(pair(r, c), Pq[r] * cj.x, Pq[r], P * cj.x, row[r], col);
+                rotate_sums<ADJ>(col);
+            }
+        } else {
+            // the diagonal of row block `own` from the row side, half the pair energy each
+            const int cnt = min(kWave, ae - jb);
+            for (int m = 0; m < cnt; ++m) {
+                if (m == lane) continue;
+                const float qj = s_col[m].x;
+                if (own == 0)
+                    add_pair<ADJ, false>(pair(0, m), Pq[0] * qj, Pq[0], P * qj, row[0], col);
+                else
+                    add_pair<ADJ, false>(pair(1, m), Pq[1] * qj, Pq[1], P * qj, row[1], col);
+            }
+            row[0].e *= 0.5f;
+            row[1].e *= 0.5f;
+            if (own == 1) {
+                for (int m = 0; m < kWave; ++m) {
+                    const int c = (lane + m) & (kWave - 1);
+                    const float qj = s_col[c].x;
+                    add_pair<ADJ, true>(pair(0, c), Pq[0] * qj, Pq[0], P * qj, row[0], col);
+                    rotate_sums<ADJ>(col);
+                }
+            }
+        }
+        if (own > 0 && jv) store_column<ADJ>(p, colpart_index(sd, (tile.x - ab) / (2 * kWave), jj - ab), col, s_col[lane].w);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            out[r][0] += row[r].fx;
+            out[r][1] += row[r].fy;
+            out[r][2] += row[r].fz;
+            out[r][3] += half[r] * row[r].g;
+            out[r][4] += row[r].e;
+            if (ADJ) out[r][5] += row[r].dq;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        if (!iv[r]) continue;
+        double* o = p.pair_part + (size_t)tile.w * 6 * p.N + tile.x + kWave * r + lane;
+        for (int v = 0; v < (ADJ ? 6 : 5); ++v) o[(size_t)v * p.N] = out[r][v];
+    }
+}
+
 // Per atom, one workgroup per 64-atom block: the pair sums in a fixed order, then the self
 // term and dE/dI = dE/dB dB/dI (customGBEnergyPerParticle.cu; CharmmReferenceGBSW.cpp:257-273).
 // Thread (g, lane) sums, for atom lane of the block, the row pieces k = g, g + G, ... and the
-// column partials of row blocks I = g, g + G, ... < bj in FP64 (G = 16 wave groups); the
+// column partials of row tiles t = g, g + G, ... in FP64 (G = 16 wave groups); the
 // groups are added in order.  ADJ: dE/dq and the Born-map parts of dE/dtheta.
 constexpr int kChainGroups = 16;
 
@@ -2014,7 +2153,9 @@ __global__ void __launch_bounds__(kChainGroups * kWave) k_atom_chain(KParams p) 
     const int bj = (j0 - ab) / kWave;
     const int i = j0 + lane;  // pair slot
     const bool iv = i < sd.atom_end;
-    const int pieces = (sd.nblk - bj + sd.pair_k - 1) / sd.pair_k;
+    const int rows = sd.pair_rows, tile = bj / rows;  // the block's row tile
+    const int pieces = (sd.nblk - tile * rows + sd.pair_k - 1) / sd.pair_k;
+    const int col_tiles = (bj + rows - 1) / rows;     // the row tiles that begin before it
     const long long T = p.colpart_total;
     double a[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     if (iv) {
@@ -2027,8 +2168,8 @@ __global__ void __launch_bounds__(kChainGroups * kWave) k_atom_chain(KParams p) 
             a[4] += in[4 * p.N + i];
             if (ADJ) a[5] += in[5 * p.N + i];
         }
-        for (int I = grp; I < bj; I += kChainGroups) {
-            const long long o = colpart_index(sd, I, i - ab);
+        for (int t = grp; t < col_tiles; t += kChainGroups) {
+            const long long o = colpart_index(sd, t, i - ab);
             a[0] += p.colpart[o];
             a[1] += p.colpart[T + o];
             a[2] += p.colpart[2 * T + o];
@@ -2707,6 +2848,15 @@ __global__ void k_stats(KParams p, double* out) {
     }
 }
 
+// The pair tiles: those of 4 waves, of one row block, of two (no cutoffs or exclusions).
+template <bool ADJ, bool CUT>
+void launch_pairs(const KParams& p, hipStream_t stream) {
+    const int n2 = p.n_tiles - p.n_tiles4 - p.n_tiles1;
+    if (p.n_tiles4 > 0) hipLaunchKernelGGL((k_pairs<ADJ, CUT, 4>), dim3(p.n_tiles4), dim3(4 * kWave), 0, stream, p);
+    if (p.n_tiles1 > 0) hipLaunchKernelGGL((k_pairs<ADJ, CUT, 1>), dim3(p.n_tiles1), dim3(kWave), 0, stream, p);
+    if (!CUT && n2 > 0) hipLaunchKernelGGL(k_pairs2<ADJ>, dim3(n2), dim3(kWave), 0, stream, p);
+}
+
 template <bool ADJ>
 void launch_force(const KParams& p, int vk, int blocks, hipStream_t stream) {
     switch (vk) {
@@ -2800,18 +2950,13 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
                       &force_fix, &dedi, &dvdth, &despdth, &pdth, &dvdx, &despdx};
         err = hipModuleLaunchKernel(c.chain, nb, 1, 1, c.chain_threads, 1, 1, 0, stream, ca, nullptr);
         if (err != hipSuccess) return err;
-    } else if (adj) {
-        if (p.any_cut || p.any_excl) {
-            hipLaunchKernelGGL(k_block_box, dim3(p.n_colblocks), dim3(64), 0, stream, p);
-            hipLaunchKernelGGL((k_pairs<true, true>), dim3(p.n_tiles), dim3(64), 0, stream, p);
-        } else {
-            hipLaunchKernelGGL((k_pairs<true, false>), dim3(p.n_tiles), dim3(64), 0, stream, p);
-        }
-    } else if (p.any_cut || p.any_excl) {
-        hipLaunchKernelGGL(k_block_box, dim3(p.n_colblocks), dim3(64), 0, stream, p);
-        hipLaunchKernelGGL((k_pairs<false, true>), dim3(p.n_tiles), dim3(64), 0, stream, p);
     } else {
-        hipLaunchKernelGGL((k_pairs<false, false>), dim3(p.n_tiles), dim3(64), 0, stream, p);
+        const bool cut = p.any_cut || p.any_excl;
+        if (cut) hipLaunchKernelGGL(k_block_box, dim3(p.n_colblocks), dim3(64), 0, stream, p);
+        if (adj)
+            cut ? launch_pairs<true, true>(p, stream) : launch_pairs<true, false>(p, stream);
+        else
+            cut ? launch_pairs<false, true>(p, stream) : launch_pairs<false, false>(p, stream);
     }
     if (!p.custom) {
         mark(5);
