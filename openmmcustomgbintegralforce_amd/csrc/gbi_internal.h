@@ -293,6 +293,12 @@ hipError_t launch_gather_posq(double* pos, const void* posq, int posq_double, co
 hipError_t launch_add_forces_fixed(long long* dst, int padded_n, const long long* force_fix, const int* atom_slot,
                                    int n, hipStream_t stream);
 
+// Copies a block whose addresses are multiples of 8, either side device memory or page-locked host
+// memory, by a kernel.
+hipError_t launch_export(char* dst, const char* src, size_t bytes, hipStream_t stream);
+// dst[3 a + d] = force_fix[d n + a] / 2^32.
+hipError_t launch_export_forces(double* dst, const long long* force_fix, int n, hipStream_t stream);
+
 // gbi_execute_noalloc: bytes of the static device scratch array (per GPU), and its device
 // address on the current device (gbi_noalloc.hip).
 constexpr size_t kNoAllocScratchBytes = size_t(256) << 20;

@@ -3016,7 +3016,33 @@ __global__ void k_add_forces_fixed(long long* dst, int padded_n, const long long
     for (int d = 0; d < 3; ++d) dst[(long long)d * padded_n + slot] += force_fix[(long long)d * n + a];
 }
 
+__global__ void k_export(double* dst, const double* src, size_t n) {
+    for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < n; k += (size_t)gridDim.x * blockDim.x)
+        dst[k] = src[k];
+}
+
+__global__ void k_export_forces(double* dst, const long long* force_fix, int n) {
+    for (long long k = blockIdx.x * blockDim.x + threadIdx.x; k < 3ll * n; k += (long long)gridDim.x * blockDim.x) {
+        const long long a = k / 3, d = k - 3 * a;
+        dst[k] = (double)force_fix[d * n + a] * (1.0 / kFix32);
+    }
+}
+
+unsigned export_blocks(size_t n) { return (unsigned)std::min<size_t>(std::max<size_t>((n + 255) / 256, 1), 1024); }
+
 }  // namespace
+
+hipError_t launch_export_forces(double* dst, const long long* force_fix, int n, hipStream_t stream) {
+    hipLaunchKernelGGL(k_export_forces, dim3(export_blocks(3 * (size_t)n)), dim3(256), 0, stream, dst, force_fix, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_export(char* dst, const char* src, size_t bytes, hipStream_t stream) {
+    const size_t n = bytes / sizeof(double);
+    hipLaunchKernelGGL(k_export, dim3(export_blocks(n)), dim3(256), 0, stream, reinterpret_cast<double*>(dst),
+                       reinterpret_cast<const double*>(src), n);
+    return hipGetLastError();
+}
 
 hipError_t launch_gather_posq(double* pos, const void* posq, int posq_double, const int* atom_slot, int n,
                               hipStream_t stream) {
