@@ -948,6 +948,7 @@ gbi::KParams make_kparams(gbi_ctx& c, bool adjoint) {
             (s.kind == gbi::GRID_TIGHT && !s.periodic() ? k.gbsw_exact : k.gbsw_other) = 1;
             k.gbsw_q = std::max(k.gbsw_q, (s.Q + 1) & ~1);
         }
+    k.gbsw_run = c.kinds[gbi::VOL_GBMV1] || c.kinds[gbi::VOL_GBMV2] ? 64 : std::max(1, (c.N + 7) / 8);
     k.cell_sub = c.cell_sub.p;
     k.cell_mask = c.kinds[gbi::VOL_GBSW] ? c.cell_mask.p : nullptr;
     k.grec = c.grec.p;

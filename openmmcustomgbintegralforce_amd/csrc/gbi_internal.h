@@ -245,6 +245,7 @@ struct KParams {
     float4* prec;            // per system: cell_cap x pt_cap slots; records (FP32 point - corner, packed point),
                              // or, binning by bricks, packed points (atom << kQBits | q) in the range's first quarter
     int gbsw_exact, gbsw_other;    // some GBSW system has the exact non-periodic grid, another one
+    int gbsw_run;                  // consecutive atoms that one XCD takes in k_gbsw_points
     int gbsw_q;                    // the most points per atom of a GBSW system, rounded up to even
     ulonglong2* cell_mask;         // cell_total (null without GBSW systems): sub-cells with V = 0, with V = 1
     unsigned long long* cell_sub;  // cell_total x 64 (GBSW cells with atoms): the atoms that reach each sub-cell;

@@ -64,6 +64,18 @@ __device__ inline int wave_scan_incl(int v, int lane) {
     return v;
 }
 
+// Item of workgroup b when runs of `run` items go to the XCDs in turn (workgroup b runs on XCD b
+// mod 8): neighbouring cells or atoms share lines of what they read and write, and a line stays in
+// one XCD's L2.  n items need run_blocks(n, run) workgroups, some of whose items are beyond n.
+__device__ inline int run_item(int b, int run) {
+    const int k = b / kXcds;
+    return ((k / run) * kXcds + b % kXcds) * run + k % run;
+}
+__host__ __device__ inline int run_blocks(int n, int run) { return (n + kXcds * run - 1) / (kXcds * run) * (kXcds * run); }
+// Cells per run of the volume and chain-rule passes (GBMV-II 5,000 atoms: volume pass 0.151 ->
+// 0.148 ms, chain-rule pass 0.1115 -> 0.1097; a mixed batch of 16: 0.828 -> 0.811, 0.591 -> 0.579).
+constexpr int kCellRun = 64;
+
 // Any system of the batch hit a fatal condition: the host grows its buffers and redoes
 // the whole evaluation, so every later pass stops early.
 __device__ inline bool batch_fatal(const KParams& p) { return (*p.flags_all & kFatalFlags) != 0; }
@@ -1191,10 +1203,11 @@ __global__ void __launch_bounds__(kGbswThreads) k_gbsw_points(KParams p) {
     __shared__ double s_sum[2][kGbswThreads / kWave];
     if (batch_fatal(p)) return;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
-    // workgroup b runs on XCD b mod 8: each XCD takes a run of atoms, neighbours along the chain, so
-    // the lists that their points share stay in its L2 (atoms in the strided binning order: 2.6 GB
-    // of L2 misses at 25,000 atoms against 0.7)
-    const int i = (int)(blockIdx.x % kXcds) * (int)(gridDim.x / kXcds) + (int)(blockIdx.x / kXcds);
+    // runs of atoms, neighbours along the chain, per XCD, so the lists that their points share stay
+    // in its L2 (atoms in the strided binning order: 2.6 GB of L2 misses at 25,000 atoms against
+    // 0.7): an eighth of the atoms each, or short runs where GBMV systems would leave XCDs idle (a
+    // mixed batch of 16: 0.39 -> 0.25 ms; 25,000 GBSW atoms in runs of 64: 0.275 -> 0.281)
+    const int i = run_item(blockIdx.x, p.gbsw_run);
     if (i >= p.N) return;
     const int s = p.atom_sys[i];
     const SysDesc sd = p.sys[s];
@@ -1443,7 +1456,9 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
     const int nwork = p.work[VK];
     const int* worklist = p.worklist + VK * p.cell_total;
     const int* worklist_sys = p.worklist_sys + VK * p.cell_total;
-    for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
+    for (int b = blockIdx.x; b < run_blocks(nwork, kCellRun); b += gridDim.x) {
+        const int w = run_item(b, kCellRun);
+        if (w >= nwork) continue;
         const int c = worklist[w];
         const int sys = worklist_sys[w];
         // references (copies put part of the geometry in scratch memory: the GBMV-II pass
@@ -2280,7 +2295,9 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
     const int nwork = p.work[VK];
     const int* worklist = p.worklist + VK * p.cell_total;
     const int* worklist_sys = p.worklist_sys + VK * p.cell_total;
-    for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
+    for (int b = blockIdx.x; b < run_blocks(nwork, kCellRun); b += gridDim.x) {
+        const int w = run_item(b, kCellRun);
+        if (w >= nwork) continue;
         const int c = worklist[w];
         const int s = worklist_sys[w];
         const SysDesc sd = p.sys[s];  // a copy: read once per cell
@@ -2494,7 +2511,9 @@ __global__ void __launch_bounds__(64) k_force_gbsw(KParams p) {
     const int nwork = p.work[VOL_GBSW];
     const int* worklist = p.worklist + VOL_GBSW * p.cell_total;
     const int* worklist_sys = p.worklist_sys + VOL_GBSW * p.cell_total;
-    for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
+    for (int b = blockIdx.x; b < run_blocks(nwork, kCellRun); b += gridDim.x) {
+        const int w = run_item(b, kCellRun);
+        if (w >= nwork) continue;
         const int c = worklist[w];
         const int s = worklist_sys[w];
         const SysDesc sd = p.sys[s];  // a copy: read once per cell
@@ -2898,7 +2917,7 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
     const bool any_gbmv = kinds[VOL_GBMV1] || kinds[VOL_GBMV2];
     if (!any_gbmv) mark(2);
     if (kinds[VOL_GBSW]) {
-        const dim3 grid((p.N + kXcds - 1) / kXcds * kXcds);
+        const dim3 grid(run_blocks(p.N, p.gbsw_run));
         const size_t lds = (size_t)p.gbsw_q * kGbswLds;
         if (p.gbsw_exact) hipLaunchKernelGGL(k_gbsw_points<true>, grid, dim3(kGbswThreads), lds, stream, p);
         if (p.gbsw_other) hipLaunchKernelGGL(k_gbsw_points<false>, grid, dim3(kGbswThreads), lds, stream, p);
@@ -2918,7 +2937,7 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
     }
     hipLaunchKernelGGL(k_worklist, dim3(std::max(1, std::min((p.cell_total + kWorkThreads - 1) / kWorkThreads, 4096))),
                        dim3(kWorkThreads), 0, stream, p);
-    const int pb = std::max(1, std::min(p.cell_total, p.persist_blocks));
+    const int pb = (std::max(1, std::min(p.cell_total, p.persist_blocks)) + kXcds - 1) / kXcds * kXcds;
     if (any_gbmv) mark(2);
     if (kinds[VOL_GBMV1]) hipLaunchKernelGGL(k_volume<VOL_GBMV1>, dim3(pb), dim3(64), 0, stream, p);
     if (kinds[VOL_GBMV2]) hipLaunchKernelGGL(k_volume<VOL_GBMV2>, dim3(pb), dim3(64), 0, stream, p);
