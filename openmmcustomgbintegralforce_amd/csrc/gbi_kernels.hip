@@ -2269,6 +2269,11 @@ __global__ void __launch_bounds__(1024) k_energy(KParams p) {
 // (GBSWIntegral.cpp:271-314, GBMVIntegralTypeI.cpp:195-224, GBMVIntegralTypeII.cpp:221-282;
 //  CharmmReferenceGBMV.cpp:376-383).  Atom partials are quantised to 2^-24 and summed
 // exactly in FP64, so the per-cell totals do not depend on the point order.
+// Per pair 40 VALU slots: the three terms of dV/dx_j share G = s fac dV/dF_j, the point's c3 v is one
+// vector, and everything is in quanta (46 before; 0.111 -> 0.105 ms at 5,000 GBMV-II atoms).  What
+// bounds the pass: 0.062 ms is left with one of its three atom rows, the chain of loads of each
+// cell, its staging and its sums; 0.013 the owners' scattered stores; the exact sums 0.004.  Six
+// or five atoms per lane at 4 waves per SIMD were slower (0.125), their lists needing two rounds.
 // ADJ: also s fac dV_p/dR_j for every list atom including the owner, and the per-system
 // parameter sums (VolAcc).
 // ---------------------------------------------------------------------------
@@ -2284,7 +2289,9 @@ __device__ inline float sum8(float v) {
 template <int VK, bool ADJ>
 __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
     __shared__ float q_x[kWave], q_y[kWave], q_z[kWave];
-    __shared__ float q_0[kWave], q_1[kWave], q_2[kWave], q_3[kWave], q_4[kWave], q_5[kWave];
+    // GBMV-II: c1, c2 and c3 v of the point times s fac; GBMV-I: dV/dS times s fac; all in units of
+    // 2^-24 (the quantum), so the partials below need no scaling of their own
+    __shared__ float q_0[kWave], q_1[kWave], q_vx[kWave], q_vy[kWave], q_vz[kWave];
     __shared__ int q_own[kWave], q_pid[kWave];
     // one axis of the per-lane atom partials at a time; rows padded by 8 doubles so the 8 rows
     // that one read instruction touches start 64 bytes apart (unpadded, 512-byte rows put 8
@@ -2310,12 +2317,13 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
         const float fclamp = sd.fclamp, sign_chain = sd.sign_chain, P1x10 = 10.f * sd.P1;
         double pacc0 = 0.0, pacc1 = 0.0;  // ADJ: VolAcc partials of this lane
         for (int ab = 0; ab < na; ab += kWave) {
-            float ax[8], ay[8], az[8], a0[8], a1[8], a2[8], aR[8];
+            float ax[8], ay[8], az[8], a0[8], a1[8], aR[8];
             int aj[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
                 const int sl = ab + ag + 8 * k;
-                float4 e = make_float4(0.f, 0.f, 0.f, 0.f), q = make_float4(0.f, 0.f, __int_as_float(-1), 0.f);
+                // past the list: C = 0 (gamma = 0), b = 1, nothing to add
+                float4 e = make_float4(0.f, 0.f, 0.f, 0.f), q = make_float4(1.f, 0.f, __int_as_float(-1), 1.f);
                 if (sl < na) {
                     e = p.ent_pos[as + sl];
                     q = p.ent_par[as + sl];
@@ -2325,10 +2333,10 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
                 az[k] = e.z;
                 a0[k] = e.w;
                 a1[k] = q.x;
-                a2[k] = q.y;
                 aj[k] = __float_as_int(q.z);
                 aR[k] = q.w;
             }
+            const int kmax = (min(kWave, na - ab) + 7) / 8;  // atoms per lane
             double acc[8][3];
             double accr[8];
 #pragma unroll
@@ -2350,7 +2358,7 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
                     const uint32_t pk = __float_as_uint(r0.w);
                     const int i = (int)(pk >> kQBits), q = (int)(pk & ((1u << kQBits) - 1));
                     const double fac = p.dedi[i] * p.quad_pw[qb + q] + p.dedi[p.N + i] * p.quad_pw[p.quad_rows + qb + q];
-                    const float facs = sign_chain * (float)fac;
+                    const float facs = sign_chain * (float)fac * kQuantum;
                     q_x[lane] = r0.x;
                     q_y[lane] = r0.y;
                     q_z[lane] = r0.z;
@@ -2358,12 +2366,12 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
                     q_pid[lane] = pt_base + (i - abeg) * Q + q;
                     if (VK == VOL_GBMV2) {
                         const float4 r2 = p.frec2[o];
+                        const float c3 = facs * r1.z;
                         q_0[lane] = facs * r1.x;
                         q_1[lane] = facs * r1.y;
-                        q_2[lane] = facs * r1.z;
-                        q_3[lane] = r1.w;
-                        q_4[lane] = r2.x;
-                        q_5[lane] = r2.y;
+                        q_vx[lane] = c3 * r1.w;
+                        q_vy[lane] = c3 * r2.x;
+                        q_vz[lane] = c3 * r2.y;
                     } else {
                         q_0[lane] = facs * r1.x;
                     }
@@ -2376,64 +2384,66 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
                     if (m < cntp) {
                         const float px = q_x[m], py = q_y[m], pz = q_z[m];
                         const int own = q_own[m];
-                        const float d0 = q_0[m], d1 = q_1[m];
-                        const float d2c = VK == VOL_GBMV2 ? q_2[m] : 0.f;
-                        const float vx = VK == VOL_GBMV2 ? q_3[m] : 0.f;
-                        const float vy = VK == VOL_GBMV2 ? q_4[m] : 0.f;
-                        const float vz = VK == VOL_GBMV2 ? q_5[m] : 0.f;
+                        const float d0 = q_0[m], d1 = VK == VOL_GBMV2 ? q_1[m] : 0.f;
+                        const float vx = VK == VOL_GBMV2 ? q_vx[m] : 0.f;
+                        const float vy = VK == VOL_GBMV2 ? q_vy[m] : 0.f;
+                        const float vz = VK == VOL_GBMV2 ? q_vz[m] : 0.f;
 #pragma unroll
                         for (int k = 0; k < 8; ++k) {
-                            if (aj[k] < 0) continue;
+                            if (k >= kmax) break;
                             const bool is_own = aj[k] == own;
                             if (!ADJ && is_own) continue;
                             const float dx = ax[k] - px, dy = ay[k] - py, dz = az[k] - pz;
                             const float dd = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                            float sv = 0.f, c3F = 0.f;
+                            float cx, cy, cz;
                             if (VK == VOL_GBMV2) {
-                                const float tt = fmaf(100.f, dd, a1[k]);
-                                const float rt = fast_rcp(tt);
+                                // F = (C/t)^2, dF/d(d) / d = D = -400 C^2 / t^3; G = s fac dV/dF_j
+                                const float rt = fast_rcp(fmaf(100.f, dd, a1[k]));
                                 const float ct = a0[k] * rt;
-                                const float F = fminf(ct * ct, fclamp);
-                                const float D = -a2[k] * rt * rt * rt;
-                                const float vdr = fmaf(vx, dx, fmaf(vy, dy, vz * dz));
-                                sv = fmaf(d0, D, fmaf(d1 * F, fmaf(D, dd, F), d2c * vdr * D));
-                                c3F = d2c * F;
+                                const float F0 = ct * ct, F = fminf(F0, fclamp);
+                                const float D = -400.f * F0 * rt;
+                                const float e = d1 * F;
+                                const float G = fmaf(e, dd, fmaf(vx, dx, fmaf(vy, dy, fmaf(vz, dz, d0))));
+                                const float sv = fmaf(D, G, e * F);
+                                cx = fmaf(sv, dx, F * vx);
+                                cy = fmaf(sv, dy, F * vy);
+                                cz = fmaf(sv, dz, F * vz);
                                 if (ADJ) {
-                                    // s fac dV/dF_j; F = (C/t)^2, t = b + 100 d^2, b = C - 100 R^2
-                                    const float G = fmaf(d1 * dd, F, fmaf(d2c, vdr, d0));
+                                    // t = b + 100 d^2, b = C - 100 R^2
                                     const float dFdC = 2.f * ct * rt, dFdb = -2.f * ct * ct * rt;
                                     const float gab = G * (dFdC + dFdb);
-                                    accr[k] += quant(fmaf(G * dFdb, -200.f * aR[k], gab * P1x10));
-                                    pacc0 += quant(gab);
-                                    pacc1 += quant(gab * 10.f * aR[k]);
+                                    accr[k] += (double)rintf(fmaf(G * dFdb, -200.f * aR[k], gab * P1x10));
+                                    pacc0 += (double)rintf(gab);
+                                    pacc1 += (double)rintf(gab * 10.f * aR[k]);
                                 }
                             } else {
                                 const float gam = a0[k];
                                 const float ex = __expf(gam * (dd * dd));
-                                sv = d0 * gam * ex * 4.f * dd;
+                                const float sv = d0 * gam * ex * 4.f * dd;
+                                cx = sv * dx;
+                                cy = sv * dy;
+                                cz = sv * dz;
                                 if (ADJ) {
                                     // dS/dgamma_j = d^4 e_j; dgamma_j/dR_j = -4 gamma_j/R_j
                                     const float tg = d0 * (dd * dd) * ex;
-                                    accr[k] += quant(tg * (-4.f * gam / aR[k]));
-                                    pacc0 += quant(tg * gam);
+                                    accr[k] += (double)rintf(tg * (-4.f * gam / aR[k]));
+                                    pacc0 += (double)rintf(tg * gam);
                                 }
                             }
                             if (ADJ && is_own) continue;  // the owner moves with its points
-                            const float cx = fmaf(sv, dx, c3F * vx);
-                            const float cy = fmaf(sv, dy, c3F * vy);
-                            const float cz = fmaf(sv, dz, c3F * vz);
-                            acc[k][0] += quant(cx);
-                            acc[k][1] += quant(cy);
-                            acc[k][2] += quant(cz);
+                            acc[k][0] += (double)rintf(cx);
+                            acc[k][1] += (double)rintf(cy);
+                            acc[k][2] += (double)rintf(cz);
                             ox += cx;
                             oy += cy;
                             oz += cz;
                         }
                     }
                     {
-                        ox = sum8(ox);
-                        oy = sum8(oy);
-                        oz = sum8(oz);
+                        constexpr float kUnit = 1.f / kQuantum;
+                        ox = kUnit * sum8(ox);
+                        oy = kUnit * sum8(oy);
+                        oz = kUnit * sum8(oz);
                         if (ag == 0 && m < cntp) {
                             const int pid = q_pid[m];
                             if (ab == 0) {
