@@ -195,7 +195,8 @@ struct gbi_ctx {
         atom_energy, energy, stats, dedq, dedr, theta_atom, theta;
     DevBuf<float4> aparam;
     DevBuf<int> cell_fill, cell_start, cell_count_eff, cell_atoms_tmp, cell_atoms, cell_pt_count,
-        cell_act_count, frec_base, worklist, worklist_sys, work, scan_tmp;
+        cell_act_count, work_act, work, scan_tmp;
+    DevBuf<int4> work_a, work_b;
     DevBuf<float4> ent_pos, ent_par, prec, frec0, frec1, frec2, vrec;
     DevBuf<int> brick_count, cell_ctr;
     DevBuf<uint2> brick_rec;
@@ -284,8 +285,10 @@ struct gbi_ctx {
         bbox_done.release();
         DevBuf<int>* ib[] = {&flags_all,      &atom_sys,     &cell_sys,       &bin_order,       &cell_fill,
                              &cell_start,     &cell_count_eff, &cell_atoms_tmp, &cell_atoms, &cell_pt_count,
-                             &cell_act_count, &frec_base,    &worklist,       &worklist_sys, &work, &scan_tmp};
+                             &cell_act_count, &work_act,     &work,           &scan_tmp};
         for (auto* b : ib) b->release();
+        work_a.release();
+        work_b.release();
         DevBuf<float4>* fb[] = {&ent_pos, &ent_par, &prec, &frec0, &frec1, &frec2, &vrec};
         for (auto* b : fb) b->release();
         brick_count.release();
@@ -494,6 +497,13 @@ gbi::SysDesc make_desc(const gbi_ctx& c, const SysHost& s, long long cell_base, 
     return d;
 }
 
+// Volume kinds of the batch.
+int n_kinds(const gbi_ctx& c) {
+    int n = 0;
+    for (bool k : c.kinds) n += k;
+    return n;
+}
+
 // Cell, slot and worklist buffers for the systems' current capacities; uploads the
 // system descriptors and the cell -> system map.
 gbi_status layout(gbi_ctx& c) {
@@ -541,9 +551,10 @@ gbi_status layout(gbi_ctx& c) {
     c.any_bricks = any_bricks;
     c.any_cells = any_cells;
     HIP_TRY(c.cell_act_count.ensure(cells));
-    HIP_TRY(c.frec_base.ensure(cells + 1));
-    HIP_TRY(c.worklist.ensure(gbi::VOL_KINDS * cells));
-    HIP_TRY(c.worklist_sys.ensure(gbi::VOL_KINDS * cells));
+    const long long entries = cells * n_kinds(c);
+    HIP_TRY(c.work_a.ensure(entries));
+    HIP_TRY(c.work_b.ensure(entries));
+    HIP_TRY(c.work_act.ensure(entries));
     HIP_TRY(c.cell_sys.ensure(cells));
     HIP_TRY(c.scan_tmp.ensure((cells + 4095) / 4096 + 16));
     HIP_TRY(c.prec.ensure(std::max<long long>(1, slots)));
@@ -933,9 +944,13 @@ gbi::KParams make_kparams(gbi_ctx& c, bool adjoint) {
     k.ctr_perm = perm ? 1 : 0;
     k.ctr_len = (int)(perm ? (c.cell_total + 4095) / 4096 * 4096 : c.cell_total);
     k.cell_act_count = c.cell_act_count.p;
-    k.frec_base = c.frec_base.p;
-    k.worklist = c.worklist.p;
-    k.worklist_sys = c.worklist_sys.p;
+    k.work_a = c.work_a.p;
+    k.work_b = c.work_b.p;
+    k.work_act = c.work_act.p;
+    for (int vk = 0, at = 0; vk < gbi::VOL_KINDS; ++vk) {
+        k.work_at[vk] = at;
+        if (c.kinds[vk]) at += (int)c.cell_total;
+    }
     k.prec = c.prec.p;
     k.brick_count = c.brick_count.p;
     k.brick_rec = c.brick_rec.p;
@@ -1496,7 +1511,7 @@ NoAllocCaps noalloc_caps(const SysHost& s, const double* pos, const double* radi
     }
     caps.tmp_cap = max_raw + max_raw / 8 + 16;
     caps.pt_cap = max_pts + max_pts / 8 + 16;
-    caps.entries = members + members / 8 + 1024;
+    caps.entries = members + members / 16 + 1024;
     return caps;
 }
 
@@ -2011,8 +2026,8 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
             clear(c.dbdi), clear(c.dedi), clear(c.atom_energy), clear(c.energy), clear(c.pair_part), clear(c.colpart);
             clear(c.force_fix), clear(c.cell_fill), clear(c.cell_count_eff), clear(c.cell_pt_count);
             clear(c.cell_ctr);
-            clear(c.cell_act_count), clear(c.cell_sys), clear(c.cell_start), clear(c.frec_base), clear(c.worklist);
-            clear(c.worklist_sys), clear(c.scan_tmp), clear(c.cell_atoms_tmp), clear(c.cell_atoms), clear(c.ent_pos);
+            clear(c.cell_act_count), clear(c.cell_sys), clear(c.cell_start), clear(c.work_a), clear(c.work_b);
+            clear(c.work_act), clear(c.scan_tmp), clear(c.cell_atoms_tmp), clear(c.cell_atoms), clear(c.ent_pos);
             clear(c.ent_par), clear(c.prec), clear(c.frec0), clear(c.frec1), clear(c.frec2), clear(c.vval);
             clear(c.vrec), clear(c.brick_count), clear(c.brick_rec), clear(c.cell_mask), clear(c.grec);
             clear(c.gval), clear(c.atom_nact);
@@ -2066,8 +2081,8 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     sc.take(c.colpart, (size_t)5 * c.colpart_total), sc.take(c.force_fix, 3 * N);
     sc.take(c.cell_fill, cells), sc.take(c.cell_count_eff, cells), sc.take(c.cell_pt_count, cells);
     sc.take(c.cell_act_count, cells), sc.take(c.cell_sys, cells), sc.take(c.cell_start, cells + 1);
-    sc.take(c.frec_base, cells + 1), sc.take(c.worklist, gbi::VOL_KINDS * cells);
-    sc.take(c.worklist_sys, gbi::VOL_KINDS * cells), sc.take(c.scan_tmp, (cells + 4095) / 4096 + 16);
+    sc.take(c.work_a, cells), sc.take(c.work_b, cells), sc.take(c.work_act, cells);
+    sc.take(c.scan_tmp, (cells + 4095) / 4096 + 16);
     sc.take(c.cell_atoms_tmp, cells * (size_t)caps.tmp_cap), sc.take(c.cell_atoms, caps.entries);
     sc.take(c.ent_pos, caps.entries), sc.take(c.ent_par, caps.entries);
     sc.take(c.prec, gbsw ? 1 : c.prec_total), sc.take(c.grec, gbsw ? c.prec_total : 1);

@@ -226,7 +226,7 @@ struct KParams {
     float4* ent_pos;         // entry_cap: position relative to the cell corner, aparam.x
     float4* ent_par;         // entry_cap: aparam.y, aparam.z, atom index bits, R
     // points
-    int* cell_pt_count;      // cell_total: points per cell (gathered from cell_ctr by the scan)
+    int* cell_pt_count;      // cell_total: points per cell (gathered from cell_ctr by k_worklist)
     int* cell_ctr;           // ctr_len: the binning passes' point counters, cell c's at ctr_slot(c)
                              // (ctr_perm = 1), or cell_pt_count itself (ctr_perm = 0)
     int ctr_perm;
@@ -238,10 +238,11 @@ struct KParams {
     int brick_max;           // the largest brick range of a system
     int any_bricks;          // some system bins by bricks (SysDesc::sk > 1)
     int any_cellbin;         // some GBMV system bins by cells (SysDesc::sk = 1)
-    int* cell_act_count;     // cell_total
-    int* frec_base;          // cell_total + 1: exclusive scan of the point counts
-    int* worklist;           // VOL_KINDS x cell_total
-    int* worklist_sys;       // VOL_KINDS x cell_total: system of each worklist cell
+    int* cell_act_count;     // cell_total (diagnostics)
+    int4* work_a;            // worklist entries (k_worklist), cell_total for each volume kind present:
+    int4* work_b;            //   those of kind k from work_at[k]
+    int* work_act;           // per entry of a GBMV kind: its active points
+    int work_at[VOL_KINDS];
     float4* prec;            // per system: cell_cap x pt_cap slots; records (FP32 point - corner, packed point),
                              // or, binning by bricks, packed points (atom << kQBits | q) in the range's first quarter
     int gbsw_exact, gbsw_other;    // some GBSW system has the exact non-periodic grid, another one
@@ -277,7 +278,7 @@ struct KParams {
     double* theta;           // S x TH_COUNT (adjoint): dE/dtheta
     long long* force_fix;    // 3 x N, scale 2^32
     double* energy;          // S
-    int* work;               // counters [8]
+    int* work;               // counters [8]: worklist entries per volume kind, chain-rule records handed out
     int* scan_tmp;           // scan block sums
 };
 

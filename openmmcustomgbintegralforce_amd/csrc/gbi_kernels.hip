@@ -757,15 +757,13 @@ __global__ void __launch_bounds__(64) k_grid_sort(KParams p) {
 // Slot of cell c's binning counter: within each tile of 4,096 counters, cell r of the tile at
 // (r mod 128) x 32 + r / 128, so the 32 counters of a 128-byte line belong to cells 128 apart
 // and the cells of one atom's points, mostly neighbours, reserve on different lines.  Dense:
-// the clear and the scan's gather read whole lines.
+// the clear and the worklist's gather read whole lines.
 __host__ __device__ inline long long ctr_slot(long long c) {
     return (c & ~4095ll) | ((c & 127) << 5) | ((c >> 7) & 31);
 }
 __device__ inline long long cell_ctr_slot(const KParams& p, long long c) { return p.ctr_perm ? ctr_slot(c) : c; }
 
-// perm: the inputs are the binning counters in[ctr_slot(idx)], copied to compact[idx] on the way.
-__global__ void __launch_bounds__(kScanThreads) k_scan_tiles(const int* in, int* out, int n, int* block_sums,
-                                                             int perm, int* compact) {
+__global__ void __launch_bounds__(kScanThreads) k_scan_tiles(const int* in, int* out, int n, int* block_sums) {
     __shared__ int s_wave[kScanThreads / kWave];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
     const long long base = (long long)blockIdx.x * kScanTile + (long long)tid * kScanItems;
@@ -773,8 +771,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_tiles(const int* in, int*
     int tsum = 0;
     for (int k = 0; k < kScanItems; ++k) {
         const long long idx = base + k;
-        v[k] = idx < n ? in[perm ? ctr_slot(idx) : idx] : 0;
-        if (perm && idx < n) compact[idx] = v[k];
+        v[k] = idx < n ? in[idx] : 0;
         tsum += v[k];
     }
     const int incl = wave_scan_incl(tsum, lane);
@@ -832,12 +829,11 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_add(int* out, int n, cons
 }
 
 // out[0..n] = exclusive scan of in[0..n-1] (out[n] = total); flags |= flag when total > limit.
-// perm: the inputs are in[ctr_slot(k)], also copied to compact[k].
 hipError_t scan_exclusive(const int* in, int* out, int n, int* tmp, int limit, int* flags, int flag,
-                          hipStream_t stream, int perm = 0, int* compact = nullptr) {
+                          hipStream_t stream) {
     const int nblocks = (n + kScanTile - 1) / kScanTile;
     if (nblocks > kScanTile || nblocks < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_scan_tiles, dim3(nblocks), dim3(kScanThreads), 0, stream, in, out, n, tmp, perm, compact);
+    hipLaunchKernelGGL(k_scan_tiles, dim3(nblocks), dim3(kScanThreads), 0, stream, in, out, n, tmp);
     hipLaunchKernelGGL(k_scan_add, dim3(nblocks), dim3(kScanThreads), 0, stream, out, n, (const int*)tmp, limit, flags,
                        flag);
     return hipGetLastError();
@@ -1355,41 +1351,42 @@ __global__ void __launch_bounds__(kGbswThreads) k_gbsw_points(KParams p) {
 }
 
 // Cells holding points, one list per volume kind (order irrelevant: every later sum is
-// order independent).  One atomic per workgroup and kind: all of them go to one counter
-// per kind, which serialises them (one per wave took 0.009 ms for 770 waves at 5,000 atoms,
-// one per 1,024-thread workgroup 0.002 ms; 0.014 -> 0.005 ms at 25,000).
-// It also finishes the exclusive scan of the point counts (frec_base), whose tile pass ran
-// before it: each chunk of kWorkThreads cells lies in one scan tile and adds the sum of the
-// tile sums before it (the work of k_scan_add, without a launch of its own).
+// order independent).  An entry holds what the per-cell passes need first, so that a cell's
+// atoms and points load one latency after its entry: work_a (cell, system, atoms, first list
+// entry), work_b (points, first chain-rule record, first slot in two halves).  Reading the cell
+// first, then five arrays by it and the system's slot base, made no pass slower by more than 2 %
+// (chain-rule pass of a mixed batch of 16: 0.573 -> 0.561 ms).
+// One atomic per workgroup and kind: all of them go to one counter per kind, which serialises
+// them (one per wave took 0.009 ms for 770 waves at 5,000 atoms, one per 1,024-thread workgroup
+// 0.002 ms; 0.014 -> 0.005 ms at 25,000).  The GBMV cells' chain-rule records (frec) are handed
+// out here too, a run per workgroup: an exclusive scan of the point counts for them took two
+// launches of its own (an evaluation of 1,203 atoms 0.158 -> 0.152 ms, 2,500 0.1285 -> 0.123).
 constexpr int kWorkThreads = 1024;
-static_assert(kWorkThreads == kScanThreads && kScanTile % kWorkThreads == 0, "a chunk lies in one scan tile");
 
 __global__ void __launch_bounds__(kWorkThreads) k_worklist(KParams p) {
     constexpr int kWaves = kWorkThreads / kWave;
-    __shared__ int s_cnt[VOL_KINDS][kWaves];
-    __shared__ int s_base[VOL_KINDS];
-    __shared__ int s_scan[kScanThreads / kWave];
+    __shared__ int s_cnt[VOL_KINDS][kWaves], s_rec[kWaves];
+    __shared__ int s_base[VOL_KINDS + 1];
     const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     const int stride = gridDim.x * blockDim.x;
-    const int ntiles = (p.cell_total + kScanTile - 1) / kScanTile;
-    for (int base = blockIdx.x * blockDim.x; base < p.cell_total; base += stride) {
-        const int t = base / kScanTile;
-        const int add = tiles_before(p.scan_tmp, t, s_scan);
-        const int c = base + (int)threadIdx.x;
-        if (c < p.cell_total) p.frec_base[c] += add;
-        if (c == p.cell_total - 1) {  // the last cell: the total and its limit
-            const int total = add + p.scan_tmp[ntiles - 1];
-            p.frec_base[p.cell_total] = total;
-            if (total > p.NQ) atomicOr(p.flags_all, FLAG_POINT_OVERFLOW);
-        }
-    }
     if (batch_fatal(p)) return;
     for (int base = blockIdx.x * blockDim.x; base < p.cell_total; base += stride) {
         const int c = base + (int)threadIdx.x;
-        int vk = -1, s = 0;
-        if (c < p.cell_total && p.cell_pt_count[c] > 0) {
-            s = p.cell_sys[c];
-            vk = p.sys[s].vol_kind;
+        int vk = -1, s = 0, np = 0, na = 0, start = 0;
+        long long slot0 = 0;
+        if (c < p.cell_total) {
+            const int pts = p.cell_ctr[cell_ctr_slot(p, c)];
+            if (p.ctr_perm) p.cell_pt_count[c] = pts;
+            if (pts > 0) {
+                s = p.cell_sys[c];
+                na = p.cell_count_eff[c];
+                start = p.cell_start[c];
+                const SysDesc& sd = p.sys[s];
+                vk = sd.vol_kind;
+                np = min(pts, sd.pt_cap);
+                const long long in_sys = (long long)(c - sd.cell_base) * sd.pt_cap;
+                slot0 = (sd.sk > 1 ? 4 : 1) * sd.prec_base + in_sys;  // (bricks: 4-byte packed points)
+            }
         }
         unsigned long long m[VOL_KINDS];
 #pragma unroll
@@ -1397,24 +1394,44 @@ __global__ void __launch_bounds__(kWorkThreads) k_worklist(KParams p) {
             m[k] = __ballot(vk == k);
             if (lane == 0) s_cnt[k][wid] = __popcll(m[k]);
         }
+        const int rec = vk == VOL_GBMV1 || vk == VOL_GBMV2 ? np : 0;
+        const int rec_incl = wave_scan_incl(rec, lane);
+        if (lane == kWave - 1) s_rec[wid] = rec_incl;
         __syncthreads();
-        if (threadIdx.x < VOL_KINDS) {
+        if (threadIdx.x <= VOL_KINDS) {
+            const int* cnt = threadIdx.x < VOL_KINDS ? s_cnt[threadIdx.x] : s_rec;
             int total = 0;
-            for (int w = 0; w < kWaves; ++w) total += s_cnt[threadIdx.x][w];
-            s_base[threadIdx.x] = total > 0 ? atomicAdd(&p.work[threadIdx.x], total) : 0;
+            for (int w = 0; w < kWaves; ++w) total += cnt[w];
+            const int at = total > 0 ? atomicAdd(&p.work[threadIdx.x], total) : 0;
+            if (threadIdx.x == VOL_KINDS && at > p.NQ - total) atomicOr(p.flags_all, FLAG_POINT_OVERFLOW);
+            s_base[threadIdx.x] = at;
         }
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < VOL_KINDS; ++k) {
             if (vk != k) continue;
-            int off = s_base[k];
-            for (int w = 0; w < wid; ++w) off += s_cnt[k][w];
-            const int slot = k * p.cell_total + off + __popcll(m[k] & ((1ull << lane) - 1ull));
-            p.worklist[slot] = c;
-            p.worklist_sys[slot] = s;
+            int off = s_base[k], first = s_base[VOL_KINDS] + rec_incl - rec;
+            for (int w = 0; w < wid; ++w) {
+                off += s_cnt[k][w];
+                first += s_rec[w];
+            }
+            const int slot = p.work_at[k] + off + __popcll(m[k] & ((1ull << lane) - 1ull));
+            p.work_a[slot] = make_int4(c, s, na, start);
+            p.work_b[slot] = make_int4(np, first, (int)(uint32_t)slot0, (int)(slot0 >> 32));
         }
-        __syncthreads();  // s_cnt and s_base are reused by the next iteration
+        __syncthreads();  // s_cnt, s_rec and s_base are reused by the next iteration
     }
+}
+
+// A worklist entry.
+struct WorkCell {
+    int c, s, na, start, np, rec;
+    long long slot;
+};
+
+__device__ inline WorkCell work_cell(const KParams& p, int vk, int w) {
+    const int4 a = p.work_a[p.work_at[vk] + w], b = p.work_b[p.work_at[vk] + w];
+    return {a.x, a.y, a.z, a.w, b.x, b.y, (long long)(uint32_t)b.z | ((long long)b.w << 32)};
 }
 
 // ---------------------------------------------------------------------------
@@ -1451,27 +1468,19 @@ template <int VK>
 __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
     __shared__ float s_x[kMaxAtomChunk], s_y[kMaxAtomChunk], s_z[kMaxAtomChunk];
     __shared__ float s_a[kMaxAtomChunk], s_b[kMaxAtomChunk];
+    const int nwork = p.work[VK];
     if (batch_fatal(p)) return;
     const int lane = threadIdx.x;
-    const int nwork = p.work[VK];
-    const int* worklist = p.worklist + VK * p.cell_total;
-    const int* worklist_sys = p.worklist_sys + VK * p.cell_total;
     for (int b = blockIdx.x; b < run_blocks(nwork, kCellRun); b += gridDim.x) {
         const int w = run_item(b, kCellRun);
         if (w >= nwork) continue;
-        const int c = worklist[w];
-        const int sys = worklist_sys[w];
+        const WorkCell wc = work_cell(p, VK, w);
+        const int c = wc.c, sys = wc.s, np = wc.np, na = wc.na, as = wc.start;
         // references (copies put part of the geometry in scratch memory: the GBMV-II pass
         // took 0.22 ms instead of 0.16 at 5,000 atoms)
         const SysDesc& sd = p.sys[sys];
         const SysGeom& G = p.geom[sys];
-        const int pt_cap = sd.pt_cap;
-        const int np = min(p.cell_pt_count[c], pt_cap);
-        const int na = p.cell_count_eff[c];
-        const long long ps = sd.prec_base + (long long)(c - sd.cell_base) * pt_cap;
-        const int as = p.cell_start[c];
         const bool single = na <= kMaxAtomChunk;
-        const int fb = p.frec_base[c];  // exclusive scan of the point counts
         const int pt_base = sd.pt_base, abeg = sd.atom_begin, Q = sd.Q, qb = sd.quad_base;
         const bool ids = sd.sk > 1;  // the slots hold packed points (bricks), else records
         double corner[3];
@@ -1501,10 +1510,10 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
             uint32_t pk = 0u;
             if (valid) {
                 if (ids) {
-                    pk = *pt_slot(p, sd, c - sd.cell_base, k);
+                    pk = reinterpret_cast<const uint32_t*>(p.prec)[wc.slot + k];
                     pr = point_record(p, sd, G, (int)(pk >> kQBits), qb + (int)(pk & ((1u << kQBits) - 1)), pk, corner);
                 } else {
-                    pr = p.prec[ps + k];
+                    pr = p.prec[wc.slot + k];
                     pk = __float_as_uint(pr.w);
                 }
             }
@@ -1626,14 +1635,17 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
             }
             const unsigned long long mask = __ballot(active);
             if (active) {
-                const int o = fb + act + __popcll(mask & ((1ull << lane) - 1ull));
+                const int o = wc.rec + act + __popcll(mask & ((1ull << lane) - 1ull));
                 p.frec0[o] = pr;
                 p.frec1[o] = r1;
                 if (VK == VOL_GBMV2) p.frec2[o] = r2;
             }
             act += __popcll(mask);
         }
-        if (lane == 0) p.cell_act_count[c] = act;
+        if (lane == 0) {
+            p.cell_act_count[c] = act;  // diagnostics
+            p.work_act[p.work_at[VK] + w] = act;
+        }
     }
 }
 
@@ -2297,22 +2309,17 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
     // that one read instruction touches start 64 bytes apart (unpadded, 512-byte rows put 8
     // lanes on each bank)
     __shared__ double s_red[8][kWave + 8];
+    const int nwork = p.work[VK];
     if (batch_fatal(p)) return;
     const int lane = threadIdx.x, ag = lane & 7, pg = lane >> 3;
-    const int nwork = p.work[VK];
-    const int* worklist = p.worklist + VK * p.cell_total;
-    const int* worklist_sys = p.worklist_sys + VK * p.cell_total;
     for (int b = blockIdx.x; b < run_blocks(nwork, kCellRun); b += gridDim.x) {
         const int w = run_item(b, kCellRun);
         if (w >= nwork) continue;
-        const int c = worklist[w];
-        const int s = worklist_sys[w];
-        const SysDesc sd = p.sys[s];  // a copy: read once per cell
-        const int nact = p.cell_act_count[c];
+        const WorkCell wc = work_cell(p, VK, w);
+        const int nact = p.work_act[p.work_at[VK] + w];
         if (nact == 0) continue;
-        const int na = p.cell_count_eff[c];
-        const int ps = p.frec_base[c];
-        const int as = p.cell_start[c];
+        const int s = wc.s, na = wc.na, ps = wc.rec, as = wc.start;
+        const SysDesc sd = p.sys[s];  // a copy: read once per cell
         const int pt_base = sd.pt_base, abeg = sd.atom_begin, Q = sd.Q, qb = sd.quad_base;
         const float fclamp = sd.fclamp, sign_chain = sd.sign_chain, P1x10 = 10.f * sd.P1;
         double pacc0 = 0.0, pacc1 = 0.0;  // ADJ: VolAcc partials of this lane
@@ -2516,21 +2523,16 @@ __global__ void __launch_bounds__(64) k_force_gbsw(KParams p) {
     __shared__ float4 s_a[kWave];                 // (position - corner, R')
     __shared__ int s_j[kWave];
     __shared__ double s_f[ADJ ? 4 : 3][kWave];    // force partials; ADJ: dE/dR' partials
+    const int nwork = p.work[VOL_GBSW];
     if (batch_fatal(p)) return;
     const int lane = threadIdx.x;
-    const int nwork = p.work[VOL_GBSW];
-    const int* worklist = p.worklist + VOL_GBSW * p.cell_total;
-    const int* worklist_sys = p.worklist_sys + VOL_GBSW * p.cell_total;
     for (int b = blockIdx.x; b < run_blocks(nwork, kCellRun); b += gridDim.x) {
         const int w = run_item(b, kCellRun);
         if (w >= nwork) continue;
-        const int c = worklist[w];
-        const int s = worklist_sys[w];
+        const WorkCell wc = work_cell(p, VOL_GBSW, w);
+        const int c = wc.c, s = wc.s, np = wc.np, na = wc.na, as = wc.start;
+        const long long ps = wc.slot;
         const SysDesc sd = p.sys[s];  // a copy: read once per cell
-        const int np = min(p.cell_pt_count[c], sd.pt_cap);
-        const int na = p.cell_count_eff[c];
-        const int as = p.cell_start[c];
-        const long long ps = sd.prec_base + (long long)(c - sd.cell_base) * sd.pt_cap;
         const bool single = na <= kWave;
         const float k1 = sd.k1, k3 = sd.k3, sw = sd.sw;
         float per_nm[3];  // sub-cells per nm
@@ -2937,14 +2939,6 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
     if (p.any_bricks)
         hipLaunchKernelGGL(k_point_split, dim3(std::max(1, std::min(p.brick_max, 4096)), p.S, kSplitParts), dim3(256),
                            0, stream, p);
-    // records of the active points of cell c start at the exclusive prefix sum of the point counts
-    // (the counters gathered into cell_pt_count); k_worklist adds the tile offsets
-    {
-        const int nblocks = (p.cell_total + kScanTile - 1) / kScanTile;
-        if (nblocks > kScanTile || nblocks < 1) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_scan_tiles, dim3(nblocks), dim3(kScanThreads), 0, stream, p.cell_ctr, p.frec_base,
-                           p.cell_total, p.scan_tmp, p.ctr_perm, p.cell_pt_count);
-    }
     hipLaunchKernelGGL(k_worklist, dim3(std::max(1, std::min((p.cell_total + kWorkThreads - 1) / kWorkThreads, 4096))),
                        dim3(kWorkThreads), 0, stream, p);
     const int pb = (std::max(1, std::min(p.cell_total, p.persist_blocks)) + kXcds - 1) / kXcds * kXcds;
