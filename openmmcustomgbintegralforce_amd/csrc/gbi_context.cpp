@@ -1078,16 +1078,13 @@ gbi_status run(gbi_ctx& c, uint32_t flags) {
 }
 
 // Waits for the stream; `forces`, `adjoint`: with the last evaluation's results in the host
-// blocks (always its flags and energies).  Kernels write them to the host, the forces converted
+// blocks (always its flags and energies).  A kernel writes them to the host, the forces converted
 // to atom-major doubles there, before the only wait.  With pageable copies and a wait for each
 // result and for the positions, a call took 0.10 ms more at 300 atoms (211 -> 109 us), 0.09 at
 // 2,000 and 0.13 with the adjoint of 16,000.
 gbi_status read_results(gbi_ctx& c, bool forces, bool adjoint) {
-    HIP_TRY(gbi::launch_export(c.host_result.p, c.result.p, c.force_at, c.stream));
-    if (forces)
-        HIP_TRY(gbi::launch_export_forces(reinterpret_cast<double*>(c.host_result.p + c.force_at), c.force_fix.p, c.N,
-                                          c.stream));
-    if (adjoint) HIP_TRY(gbi::launch_export(c.host_adj.p, c.adj_result.p, c.adj_bytes, c.stream));
+    HIP_TRY(gbi::launch_export_results(c.host_result.p, c.result.p, c.force_at, c.force_fix.p, forces ? c.N : 0,
+                                       c.host_adj.p, c.adj_result.p, adjoint ? c.adj_bytes : 0, c.stream));
     HIP_TRY(hipStreamSynchronize(c.stream));
     c.header_read = true;
     c.pos_in_flight = false;
@@ -1371,7 +1368,8 @@ gbi_status create_batch(int S, const int32_t* n_atoms, const double* charge, con
     c->energy.p = reinterpret_cast<double*>(c->result.p + c->energy_at);
     c->force_fix.p = reinterpret_cast<long long*>(c->result.p + c->force_at);
     HIP_TRY(c->bbox_part.ensure((size_t)S * gbi::kBboxMaxSlices * gbi::kBboxPart));
-    HIP_TRY(c->bbox_done.ensure(S));
+    HIP_TRY(c->bbox_done.ensure(S + 1));
+    HIP_TRY(hipMemsetAsync(c->bbox_done.p, 0, sizeof(int) * (S + 1), c->stream));
     HIP_TRY(c->atom_sys.ensure(N));
     HIP_TRY(c->pos.ensure(3 * N));
     HIP_TRY(c->d_charge.ensure(N));
@@ -1387,7 +1385,7 @@ gbi_status create_batch(int S, const int32_t* n_atoms, const double* charge, con
     HIP_TRY(c->dedi.ensure(2 * N));
     HIP_TRY(c->atom_energy.ensure(N));
     HIP_TRY(c->stats.ensure(6));
-    HIP_TRY(c->work.ensure(8));
+    HIP_TRY(c->work.ensure(gbi::kWorkCounters));
     const bool any_gbmv = c->kinds[gbi::VOL_GBMV1] || c->kinds[gbi::VOL_GBMV2];
     HIP_TRY(c->frec0.ensure(any_gbmv ? NQ : 1));
     HIP_TRY(c->frec1.ensure(any_gbmv ? NQ : 1));
@@ -2030,7 +2028,7 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
             clear(c.work_act), clear(c.scan_tmp), clear(c.cell_atoms_tmp), clear(c.cell_atoms), clear(c.ent_pos);
             clear(c.ent_par), clear(c.prec), clear(c.frec0), clear(c.frec1), clear(c.frec2), clear(c.vval);
             clear(c.vrec), clear(c.brick_count), clear(c.brick_rec), clear(c.cell_mask), clear(c.grec);
-            clear(c.gval), clear(c.atom_nact);
+            clear(c.gval), clear(c.atom_nact), clear(c.bbox_part), clear(c.bbox_done);
         }
     } unborrow{c};
     const int32_t n = n_atoms;
@@ -2071,7 +2069,7 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     // and once from the scratch array
     const size_t N = c.N, NQ = c.NQ, Q = c.quad_rows, cells = caps.cells;
     auto carve = [&](ScratchCarver& sc) {
-    sc.take(c.d_sys, 1), sc.take(c.geom, 1), sc.take(c.d_box, 3), sc.take(c.flags_all, 1), sc.take(c.work, 8);
+    sc.take(c.d_sys, 1), sc.take(c.geom, 1), sc.take(c.d_box, 3), sc.take(c.flags_all, 1), sc.take(c.work, gbi::kWorkCounters);
     sc.take(c.atom_sys, N), sc.take(c.bin_order, N), sc.take(c.pair_atom, N), sc.take(c.colblk, colblk.size());
     sc.take(c.blk_lo, colblk.size()), sc.take(c.blk_hi, colblk.size()), sc.take(c.pair_tiles, tiles.size());
     sc.take(c.pos, 3 * N), sc.take(c.d_charge, N), sc.take(c.d_radius, N), sc.take(c.d_reach, N), sc.take(c.aparam, N);
@@ -2090,7 +2088,7 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     sc.take(c.frec0, gbsw ? 1 : NQ), sc.take(c.frec1, gbsw ? 1 : NQ);
     sc.take(c.frec2, c.kinds[gbi::VOL_GBMV2] ? NQ : 1), sc.take(c.vval, gbsw ? 1 : NQ), sc.take(c.vrec, NQ);
     sc.take(c.brick_count, gbi::kBrickStride), sc.take(c.brick_rec, 1);
-    sc.take(c.bbox_part, (size_t)gbi::kBboxMaxSlices * gbi::kBboxPart), sc.take(c.bbox_done, 1);
+    sc.take(c.bbox_part, (size_t)gbi::kBboxMaxSlices * gbi::kBboxPart), sc.take(c.bbox_done, 2);
     };
     ScratchCarver dry;
     carve(dry);
@@ -2139,6 +2137,8 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     HIP_TRY(h2d(c.quad_pw.p, t.pw.data(), sizeof(double) * t.pw.size()));
     HIP_TRY(h2d(c.quad_r2.p, t.r2.data(), sizeof(float) * t.r2.size()));
     HIP_TRY(h2d(c.cell_sys.p, cell_sys.data(), sizeof(int) * cells));
+    const int none_done[2] = {0, 0};
+    HIP_TRY(h2d(c.bbox_done.p, none_done, sizeof(none_done)));
     const gbi::KParams k = make_kparams(c, false);
     HIP_TRY(gbi::launch_evaluate(k, c.kinds, st, nullptr));
     gbi::SysGeom G;

@@ -35,6 +35,7 @@ constexpr int kFatalFlags =
     FLAG_CELL_OVERFLOW | FLAG_ENTRY_OVERFLOW | FLAG_GRID_TOO_LARGE | FLAG_NONFINITE_POS | FLAG_POINT_OVERFLOW |
     FLAG_LIST_OVERFLOW;
 
+constexpr int kWorkCounters = 8;         // KParams::work
 constexpr int kMaxAtomChunk = 256;       // atoms staged in LDS per chunk (volume pass)
 constexpr int kQBits = 11;               // packed point = (atom << 11) | q, Q <= 2047
 constexpr int kMaxAtoms = 1 << (32 - kQBits);
@@ -198,7 +199,7 @@ struct KParams {
     const unsigned long long* excl_mask;  // per entry, 64 rows: bit c = pair (row, column c) excluded
     int* flags_all;          // OR of every system's flags
     double* bbox_part;       // S x kBboxMaxSlices x 10: per slice of a system's atoms min, max, sum (xyz), bad
-    int* bbox_done;          // S: slices of the system whose bounding box is in bbox_part
+    int* bbox_done;          // S + 1: slices of the system that are in bbox_part; systems done (0 between evaluations)
     int bbox_slices;         // the largest slice count of a system (bbox_slices())
     const int* atom_sys;     // N
     const int* cell_sys;     // cell_total
@@ -278,8 +279,8 @@ struct KParams {
     double* theta;           // S x TH_COUNT (adjoint): dE/dtheta
     long long* force_fix;    // 3 x N, scale 2^32
     double* energy;          // S
-    int* work;               // counters [8]: worklist entries per volume kind, chain-rule records handed out
-    int* scan_tmp;           // scan block sums
+    int* work;               // kWorkCounters: worklist entries per volume kind, chain-rule records handed out
+    int* scan_tmp;           // per tile of cells: list entries of the tiles before it
 };
 
 // Launchers (gbi_kernels.hip).  All enqueue on `stream`.
@@ -298,8 +299,10 @@ hipError_t launch_add_forces_fixed(long long* dst, int padded_n, const long long
 // Copies a block whose addresses are multiples of 8, either side device memory or page-locked host
 // memory, by a kernel.
 hipError_t launch_export(char* dst, const char* src, size_t bytes, hipStream_t stream);
-// dst[3 a + d] = force_fix[d n + a] / 2^32.
-hipError_t launch_export_forces(double* dst, const long long* force_fix, int n, hipStream_t stream);
+// An evaluation's results to page-locked host memory: the header, behind it dst[3 a + d] =
+// force_fix[d n + a] / 2^32 for n atoms (0: none), and adj_bytes of the adjoint (0: none).
+hipError_t launch_export_results(char* dst, const char* header, size_t header_bytes, const long long* force_fix, int n,
+                                 char* adj_dst, const char* adj, size_t adj_bytes, hipStream_t stream);
 
 // gbi_execute_noalloc: bytes of the static device scratch array (per GPU), and its device
 // address on the current device (gbi_noalloc.hip).

@@ -194,38 +194,46 @@ __device__ inline void cell_corner(const SysDesc& sd, const SysGeom& G, int c, d
 // Clear and geometry
 // ---------------------------------------------------------------------------
 
-__global__ void k_clear(KParams p) {
-    const int stride = gridDim.x * blockDim.x;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < p.cell_total; i += stride) {
+__host__ __device__ inline int scan_tiles(int cells) { return (cells + kScanTile - 1) / kScanTile; }
+
+// By `blocks` workgroups, this one being b.
+__device__ void clear_counters(const KParams& p, int b, int blocks) {
+    const int first = b * (int)blockDim.x + (int)threadIdx.x, stride = blocks * (int)blockDim.x;
+    for (int i = first; i < p.cell_total; i += stride) {
         p.cell_fill[i] = 0;
         p.cell_ctr[i] = 0;
     }
-    for (int i = p.cell_total + blockIdx.x * blockDim.x + threadIdx.x; i < p.ctr_len; i += stride) p.cell_ctr[i] = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < p.brick_total; i += stride)
-        p.brick_count[(long long)i * kBrickStride] = 0;
+    for (int i = p.cell_total + first; i < p.ctr_len; i += stride) p.cell_ctr[i] = 0;
+    for (int i = first; i < p.brick_total; i += stride) p.brick_count[(long long)i * kBrickStride] = 0;
     if (p.adjoint)
-        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < p.S * kVaccCopies * kVaccStride; i += stride)
-            p.vacc_fix[i] = 0;
-    if (blockIdx.x == 0) {
-        if (threadIdx.x < 8) p.work[threadIdx.x] = 0;
-        if (threadIdx.x == 0) *p.flags_all = 0;
-        for (int k = threadIdx.x; k < p.S; k += blockDim.x) p.bbox_done[k] = 0;
-    }
+        for (int i = first; i < p.S * kVaccCopies * kVaccStride; i += stride) p.vacc_fix[i] = 0;
+    for (int i = first; i <= scan_tiles(p.cell_total); i += stride) p.scan_tmp[i] = 0;
+    if (b == 0 && threadIdx.x < kWorkCounters) p.work[threadIdx.x] = 0;
 }
 
-__device__ void bbox_to_geom(const KParams& p, int s, const double* mn, const double* mx, const double* sum, int isbad);
+__device__ int bbox_to_geom(const KParams& p, int s, const double* mn, const double* mx, const double* sum, int isbad);
 
-// Bounding box and centre of geometry -> grid geometry.  Grid (slices, S): workgroup b of
-// system s reduces slice b of its atoms (bbox_slices(n) slices of ceil(n / slices) atoms) to a
+// Bounding box and centre of geometry -> grid geometry.  Workgroup s * slices + b of the first
+// slices x S reduces slice b of system s (bbox_slices(n) slices of ceil(n / slices) atoms) to a
 // partial box; the workgroup that finishes a system's last slice combines the partials in
 // slice order (a fixed order: the centre's sum does not depend on which finishes last) and
 // derives the grid.  One workgroup per system took 0.012 ms for 5,000 atoms and 0.025 ms for
-// 25,000 (a serial chain of position loads).
+// 25,000 (a serial chain of position loads).  The one that finishes the last system writes
+// flags_all, so nothing has to clear it; both counts go back to 0 for the next evaluation.
+// The other workgroups clear the counters meanwhile: no launch of their own (an
+// evaluation of 1,203 atoms 0.152 -> 0.145 ms with this, the list starts in one launch and the
+// energies in k_owner_reduce's; 300 atoms 0.075 -> 0.067, 25,000 0.777 -> 0.764).
 __global__ void __launch_bounds__(256) k_bbox(KParams p) {
     __shared__ double smin[3][4], smax[3][4], ssum[3][4];
+    __shared__ double s_part[kBboxMaxSlices * kBboxPart];
     __shared__ int sbad[4];
-    __shared__ int s_last;
-    const int s = blockIdx.y, b = blockIdx.x;
+    __shared__ int s_last, s_flags;
+    const int boxes = p.bbox_slices * p.S;
+    if ((int)blockIdx.x >= boxes) {
+        clear_counters(p, blockIdx.x - boxes, gridDim.x - boxes);
+        return;
+    }
+    const int s = blockIdx.x / p.bbox_slices, b = blockIdx.x - s * p.bbox_slices;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
     const int ab = p.sys[s].atom_begin, ae = p.sys[s].atom_end;
     const int nsl = bbox_slices(ae - ab);
@@ -260,7 +268,7 @@ __global__ void __launch_bounds__(256) k_bbox(KParams p) {
     }
     __syncthreads();
     if (tid == 0) {
-        double* part = p.bbox_part + ((long long)s * kBboxMaxSlices + b) * kBboxPart;
+        double* part = nsl > 1 ? p.bbox_part + ((long long)s * kBboxMaxSlices + b) * kBboxPart : s_part;
         for (int d = 0; d < 3; ++d) {
             double a0 = smin[d][0], a1 = smax[d][0], a2 = ssum[d][0];
             for (int w = 1; w < 4; ++w) {
@@ -273,28 +281,58 @@ __global__ void __launch_bounds__(256) k_bbox(KParams p) {
             part[6 + d] = a2;
         }
         part[9] = (double)(sbad[0] | sbad[1] | sbad[2] | sbad[3]);
-        __threadfence();  // the partial is visible before the count that announces it
-        s_last = atomicAdd(&p.bbox_done[s], 1) == nsl - 1;
+        if (nsl > 1) {
+            __threadfence();  // the partial is visible before the count that announces it
+            s_last = atomicAdd(&p.bbox_done[s], 1) == nsl - 1;
+        } else {
+            s_last = 1;
+        }
     }
     __syncthreads();
-    if (!s_last || tid != 0) return;
-    __threadfence();  // every other slice's partial is visible after its count
-    double gmn[3], gmx[3], gsm[3];
-    int gbad = 0;
-    for (int k = 0; k < nsl; ++k) {
-        const double* part = p.bbox_part + ((long long)s * kBboxMaxSlices + k) * kBboxPart;
-        for (int d = 0; d < 3; ++d) {
-            gmn[d] = k ? fmin(gmn[d], part[d]) : part[d];
-            gmx[d] = k ? fmax(gmx[d], part[3 + d]) : part[3 + d];
-            gsm[d] = k ? gsm[d] + part[6 + d] : part[6 + d];
-        }
-        gbad |= part[9] != 0.0;
+    if (!s_last) return;
+    if (nsl > 1) {
+        __threadfence();  // every other slice's partial is visible after its count
+        const double* parts = p.bbox_part + (long long)s * kBboxMaxSlices * kBboxPart;
+        for (int k = tid; k < nsl * kBboxPart; k += blockDim.x) s_part[k] = parts[k];
+        __syncthreads();
     }
-    bbox_to_geom(p, s, gmn, gmx, gsm, gbad);
+    if (tid == 0) {
+        double gmn[3], gmx[3], gsm[3];
+        int gbad = 0;
+        for (int k = 0; k < nsl; ++k) {
+            const double* part = s_part + k * kBboxPart;
+            for (int d = 0; d < 3; ++d) {
+                gmn[d] = k ? fmin(gmn[d], part[d]) : part[d];
+                gmx[d] = k ? fmax(gmx[d], part[3 + d]) : part[3 + d];
+                gsm[d] = k ? gsm[d] + part[6 + d] : part[6 + d];
+            }
+            gbad |= part[9] != 0.0;
+        }
+        s_flags = bbox_to_geom(p, s, gmn, gmx, gsm, gbad);
+        p.bbox_done[s] = 0;
+        if (p.S == 1) {
+            *p.flags_all = s_flags;
+            s_last = 0;
+        } else {
+            __threadfence();  // the system's flags are visible before the count that announces them
+            s_last = atomicAdd(&p.bbox_done[p.S], 1) == p.S - 1;
+        }
+    }
+    __syncthreads();
+    if (!s_last) return;
+    __threadfence();
+    int flags = 0;
+    for (int k = tid; k < p.S; k += blockDim.x) flags |= p.geom[k].flags;
+    if (flags) atomicOr(&s_flags, flags);
+    __syncthreads();
+    if (tid == 0) {
+        p.bbox_done[p.S] = 0;
+        *p.flags_all = s_flags;
+    }
 }
 
-// Grid geometry from the system's bounding box and coordinate sum.
-__device__ void bbox_to_geom(const KParams& p, int s, const double* mn, const double* mx, const double* sum, int isbad) {
+// Grid geometry from the system's bounding box and coordinate sum; returns its flags.
+__device__ int bbox_to_geom(const KParams& p, int s, const double* mn, const double* mx, const double* sum, int isbad) {
 #pragma clang fp contract(off)
     const SysDesc& sd = p.sys[s];
     double cog[3];
@@ -380,9 +418,7 @@ __device__ void bbox_to_geom(const KParams& p, int s, const double* mn, const do
     if (G.flags & kFatalFlags) ncell = 0;
     G.ncell = (int)ncell;
     p.geom[s] = G;
-    if (G.flags) atomicOr(p.flags_all, G.flags);
-    // the brute cell holds every atom of the system (its count is known here)
-    if (sd.grid_kind == GRID_BRUTE && ncell == 1) p.cell_fill[sd.cell_base] = sd.atom_end - sd.atom_begin;
+    return G.flags;
 }
 
 // ---------------------------------------------------------------------------
@@ -572,8 +608,9 @@ __global__ void __launch_bounds__(256) k_grid_fill(KParams p) {
     const int s = p.atom_sys[j];
     const SysDesc sd = p.sys[s];  // a copy: read once, not again after each append
     if (sd.grid_kind == GRID_BRUTE) {
-        // index order, no atomics (k_bbox set the count)
+        // the one cell holds every atom of the system, in index order: no atomics
         if (threadIdx.x == 0) {
+            if (j == sd.atom_begin) p.cell_fill[sd.cell_base] = sd.atom_end - sd.atom_begin;
             if (j - sd.atom_begin < sd.tmp_cap)
                 p.cell_atoms_tmp[sd.tmp_base + (j - sd.atom_begin)] = j << kImageBits;
             else
@@ -684,6 +721,40 @@ __device__ inline void sub_cell_lists(const KParams& p, const SysDesc& sd, const
     if (lane == 0) p.cell_mask[c] = make_ulonglong2(in, out_of);
 }
 
+// Starts of the cells' lists, an exclusive scan of cell_fill in two parts: within tiles of
+// kScanTile cells here, to cell_start; and each tile's entries added to scan_tmp of every later
+// tile (the last is the total), which k_grid_sort adds to the first.  0.005 ms at 25,000 atoms, 0.008 for
+// a mixed batch of 16; with the tiles' sums scanned by the workgroup that finishes last 0.010 and
+// 0.018, and with each wave of k_grid_sort adding them up that pass took 0.068 and 0.258 (0.062, 0.226).
+__global__ void __launch_bounds__(kScanThreads) k_list_starts(KParams p) {
+    __shared__ int s_wave[kScanThreads / kWave];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+    const int n = p.cell_total;
+    const long long base = (long long)blockIdx.x * kScanTile + (long long)tid * kScanItems;
+    int v[kScanItems];
+    int tsum = 0;
+    for (int k = 0; k < kScanItems; ++k) {
+        const long long idx = base + k;
+        v[k] = idx < n ? p.cell_fill[idx] : 0;
+        tsum += v[k];
+    }
+    const int incl = wave_scan_incl(tsum, lane);
+    if (lane == kWave - 1) s_wave[wid] = incl;
+    __syncthreads();
+    int before = 0, total = 0;
+    for (int w = 0; w < kScanThreads / kWave; ++w) {
+        if (w == wid) before = total;
+        total += s_wave[w];
+    }
+    for (int k = blockIdx.x + 1 + tid; k <= (int)gridDim.x; k += kScanThreads) atomicAdd(&p.scan_tmp[k], total);
+    int run = before + incl - tsum;
+    for (int k = 0; k < kScanItems; ++k) {
+        const long long idx = base + k;
+        if (idx < n) p.cell_start[idx] = run;
+        run += v[k];
+    }
+}
+
 // SUB: some system is GBSW (its cells also get their sub-cells' lists; without them the kernel
 // holds 6 registers and 1 KB of LDS less).
 template <bool SUB>
@@ -691,8 +762,13 @@ __global__ void __launch_bounds__(64) k_grid_sort(KParams p) {
     __shared__ __align__(16) int s_in[kSortLds];
     __shared__ int s_out[kSortLds];
     __shared__ float4 s_e[SUB ? kWave : 1];
-    if (batch_fatal(p)) return;
     const int lane = threadIdx.x;
+    const int entries = p.scan_tmp[scan_tiles(p.cell_total)];
+    if (blockIdx.x == 0 && lane == 0) {
+        p.cell_start[p.cell_total] = entries;
+        if (entries > p.entry_cap) atomicOr(p.flags_all, FLAG_ENTRY_OVERFLOW);
+    }
+    if (entries > p.entry_cap || batch_fatal(p)) return;
     for (int c = blockIdx.x; c < p.cell_total; c += gridDim.x) {
         const int n_raw = p.cell_fill[c];
         if (n_raw == 0) {
@@ -706,7 +782,7 @@ __global__ void __launch_bounds__(64) k_grid_sort(KParams p) {
         const SysDesc sd = p.sys[s];  // a copy: read once, not again after each entry's stores
         const int n = min(n_raw, sd.tmp_cap);  // (more is a fatal flag: this evaluation is redone)
         const SysGeom G = p.geom[s];
-        const int base = p.cell_start[c];
+        const int base = p.cell_start[c] + p.scan_tmp[c / kScanTile];
         const int eff = n < sd.cap ? n : sd.cap;
         const int* raw = p.cell_atoms_tmp + sd.tmp_base + (long long)(c - sd.cell_base) * sd.tmp_cap;
         double corner[3];
@@ -744,14 +820,17 @@ __global__ void __launch_bounds__(64) k_grid_sort(KParams p) {
             __syncthreads();
             for (int k = lane; k < eff; k += kWave) write_entry(p, sd, G, base + k, p.cell_atoms[base + k], corner);
         }
-        if (lane == 0) p.cell_count_eff[c] = eff;
+        if (lane == 0) {
+            p.cell_count_eff[c] = eff;
+            p.cell_start[c] = base;
+        }
         __syncthreads();
         if (SUB && sd.vol_kind == VOL_GBSW) sub_cell_lists(p, sd, G, c, base, eff, lane, s_e);
     }
 }
 
 // ---------------------------------------------------------------------------
-// Exclusive scan of int arrays (two passes, deterministic)
+// Point binning
 // ---------------------------------------------------------------------------
 
 // Slot of cell c's binning counter: within each tile of 4,096 counters, cell r of the tile at
@@ -762,86 +841,6 @@ __host__ __device__ inline long long ctr_slot(long long c) {
     return (c & ~4095ll) | ((c & 127) << 5) | ((c >> 7) & 31);
 }
 __device__ inline long long cell_ctr_slot(const KParams& p, long long c) { return p.ctr_perm ? ctr_slot(c) : c; }
-
-__global__ void __launch_bounds__(kScanThreads) k_scan_tiles(const int* in, int* out, int n, int* block_sums) {
-    __shared__ int s_wave[kScanThreads / kWave];
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
-    const long long base = (long long)blockIdx.x * kScanTile + (long long)tid * kScanItems;
-    int v[kScanItems];
-    int tsum = 0;
-    for (int k = 0; k < kScanItems; ++k) {
-        const long long idx = base + k;
-        v[k] = idx < n ? in[idx] : 0;
-        tsum += v[k];
-    }
-    const int incl = wave_scan_incl(tsum, lane);
-    if (lane == kWave - 1) s_wave[wid] = incl;
-    __syncthreads();
-    if (wid == 0) {
-        const int nw = kScanThreads / kWave;
-        int w = lane < nw ? s_wave[lane] : 0;
-        const int wi = wave_scan_incl(w, lane);
-        if (lane < nw) s_wave[lane] = wi - w;
-        if (lane == nw - 1) block_sums[blockIdx.x] = wi;
-    }
-    __syncthreads();
-    int run = s_wave[wid] + incl - tsum;
-    for (int k = 0; k < kScanItems; ++k) {
-        const long long idx = base + k;
-        if (idx < n) out[idx] = run;
-        run += v[k];
-    }
-}
-
-// Adds to tile t the sum of the tile sums before it (each workgroup sums them itself: at
-// most kScanTile ints, exact in any order); the last tile also writes the total.
-// Sum of the tile sums before tile t, by a whole workgroup of kScanThreads threads (every
-// thread gets it; s_wave is reused on return).
-__device__ inline int tiles_before(const int* block_sums, int t, int* s_wave) {
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
-    int part = 0;
-    for (int k = tid; k < t; k += kScanThreads) part += block_sums[k];
-    const int wsum = wave_scan_incl(part, lane);
-    if (lane == kWave - 1) s_wave[wid] = wsum;
-    __syncthreads();
-    int add = 0;
-    for (int w = 0; w < kScanThreads / kWave; ++w) add += s_wave[w];
-    __syncthreads();
-    return add;
-}
-
-__global__ void __launch_bounds__(kScanThreads) k_scan_add(int* out, int n, const int* block_sums, int limit,
-                                                           int* flags, int flag) {
-    __shared__ int s_wave[kScanThreads / kWave];
-    const int tid = threadIdx.x;
-    const int t = blockIdx.x;
-    const int add = tiles_before(block_sums, t, s_wave);
-    if (t == (int)gridDim.x - 1 && tid == 0) {
-        const int total = add + block_sums[t];
-        out[n] = total;
-        if (flags && total > limit) atomicOr(flags, flag);
-    }
-    const long long base = (long long)t * kScanTile;
-    for (int k = tid; k < kScanTile; k += kScanThreads) {
-        const long long idx = base + k;
-        if (idx < n) out[idx] += add;
-    }
-}
-
-// out[0..n] = exclusive scan of in[0..n-1] (out[n] = total); flags |= flag when total > limit.
-hipError_t scan_exclusive(const int* in, int* out, int n, int* tmp, int limit, int* flags, int flag,
-                          hipStream_t stream) {
-    const int nblocks = (n + kScanTile - 1) / kScanTile;
-    if (nblocks > kScanTile || nblocks < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_scan_tiles, dim3(nblocks), dim3(kScanThreads), 0, stream, in, out, n, tmp);
-    hipLaunchKernelGGL(k_scan_add, dim3(nblocks), dim3(kScanThreads), 0, stream, out, n, (const int*)tmp, limit, flags,
-                       flag);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Point binning
-// ---------------------------------------------------------------------------
 
 // r_q = x_i + off_q in FP64 (the reference's point, GBSWIntegral.cpp:132-133).
 __device__ inline void quad_point(const KParams& p, double xi, double yi, double zi, int row, double* pt) {
@@ -2166,7 +2165,8 @@ __global__ void __launch_bounds__(64) k_pairs2(KParams p) {
 // term and dE/dI = dE/dB dB/dI (customGBEnergyPerParticle.cu; CharmmReferenceGBSW.cpp:257-273).
 // Thread (g, lane) sums, for atom lane of the block, the row pieces k = g, g + G, ... and the
 // column partials of row tiles t = g, g + G, ... in FP64 (G = 16 wave groups); the
-// groups are added in order.  ADJ: dE/dq and the Born-map parts of dE/dtheta.
+// groups are added in order.  The block's energy goes where its first atom's first row piece was
+// (k_owner_reduce adds the blocks').  ADJ: dE/dq and the Born-map parts of dE/dtheta.
 constexpr int kChainGroups = 16;
 
 template <bool ADJ>
@@ -2206,20 +2206,25 @@ __global__ void __launch_bounds__(kChainGroups * kWave) k_atom_chain(KParams p) 
     }
     for (int v = 0; v < 6; ++v) s_acc[grp][v][lane] = a[v];
     __syncthreads();
-    if (grp != 0 || !iv) return;
-    const int ia = p.pair_atom[i];  // the atom of pair slot i
-    double r[6];
-    for (int v = 0; v < 6; ++v) {
-        r[v] = s_acc[0][v][lane];
-        for (int g = 1; g < kChainGroups; ++g) r[v] += s_acc[g][v][lane];
+    if (grp != 0) return;
+    double r[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    double e = 0.0, q = 0.0, B = 1.0;
+    const double P = sd.prefactor;
+    const int ia = iv ? p.pair_atom[i] : 0;  // the atom of pair slot i
+    if (iv) {
+        for (int v = 0; v < 6; ++v) {
+            r[v] = s_acc[0][v][lane];
+            for (int g = 1; g < kChainGroups; ++g) r[v] += s_acc[g][v][lane];
+        }
+        q = p.charge[ia];
+        B = p.born[ia];
+        e = r[4] + 0.5 * P * q * q / B;
     }
-    const double fx = r[0], fy = r[1], fz = r[2];
-    double dedb = r[3], e = r[4];
-    const double dq = r[5];
-    const double q = p.charge[ia], B = p.born[ia], P = sd.prefactor;
-    e += 0.5 * P * q * q / B;
-    dedb += -0.5 * P * q * q / (B * B);
-    p.atom_energy[ia] = e;
+    const double block_e = wave_sum(e);
+    if (lane == 0) p.pair_part[4 * (size_t)p.N + j0] = block_e;  // (that row piece was read above)
+    if (!iv) return;
+    const double fx = r[0], fy = r[1], fz = r[2], dq = r[5];
+    const double dedb = r[3] - 0.5 * P * q * q / (B * B);
     if (!(fabs(fx) < kFixLimit && fabs(fy) < kFixLimit && fabs(fz) < kFixLimit))
         raise_flag(p, p.atom_sys[ia], FLAG_NONFINITE_RESULT);
     p.force_fix[ia] = (long long)llrint(fx * kFix32);
@@ -2245,29 +2250,6 @@ __global__ void __launch_bounds__(kChainGroups * kWave) k_atom_chain(KParams p) 
         th[TH_ETA * p.N + ia] = g * dDdeta;
         th[TH_SLOPE * p.N + ia] = dedb / D;
         th[TH_SHIFT * p.N + ia] = dedb;
-    }
-}
-
-// Energy of each system: one workgroup per system, fixed-order FP64 sum.
-__global__ void __launch_bounds__(1024) k_energy(KParams p) {
-    __shared__ double s_w[16];
-    const int s = blockIdx.x;
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
-    if (batch_fatal(p)) {
-        if (tid == 0) p.energy[s] = 0.0;
-        return;
-    }
-    const int ab = p.sys[s].atom_begin, ae = p.sys[s].atom_end;
-    double acc = 0.0;
-    for (int i = ab + tid; i < ae; i += blockDim.x) acc += p.atom_energy[i];
-    acc = wave_sum(acc);
-    if (lane == 0) s_w[wid] = acc;
-    __syncthreads();
-    if (tid == 0) {
-        double t = 0.0;
-        for (int w = 0; w < (int)(blockDim.x / kWave); ++w) t += s_w[w];
-        p.energy[s] = t;
-        if (!isfinite(t)) raise_flag(p, s, FLAG_NONFINITE_RESULT);
     }
 }
 
@@ -2668,16 +2650,45 @@ __global__ void __launch_bounds__(64) k_force_gbsw(KParams p) {
     }
 }
 
+// Energy of system s by one wave, in a fixed order: its blocks' (k_atom_chain), or its atoms' where
+// the pair and chain passes are generated.  A launch of its own over the atoms took 0.003 ms
+// at 5,000 atoms and 0.007 at 25,000.
+__device__ inline void system_energy(const KParams& p, int s, int lane) {
+    const int ab = p.sys[s].atom_begin, n = p.sys[s].atom_end - ab;
+    const bool atoms = p.custom != nullptr;
+    const double* in = atoms ? p.atom_energy + ab : p.pair_part + 4 * (size_t)p.N + ab;
+    const int step = atoms ? 1 : kWave;
+    double acc = 0.0;
+#pragma unroll 8
+    for (int k = lane * step; k < n; k += kWave * step) acc += in[k];
+    acc = wave_sum(acc);
+    if (lane != 0) return;
+    p.energy[s] = acc;
+    if (!isfinite(acc)) raise_flag(p, s, FLAG_NONFINITE_RESULT);
+}
+
 // Owner forces: one wave per atom, fixed-order FP64 sum of its points' owner forces, read
 // only where the sign bit of V marks a point with a chain-rule factor (V >= 0 always); GBSW
 // systems keep those points' forces together (about 66 of 912: 0.052 -> 0.012 ms at 25,000 atoms).
 // ADJ (GBMV): the sigmoid parts of dE/dbeta, dE/dlambda, dE/dS0 with
 // V = 1/(1 + exp(beta (S - lambda))): dV/dbeta = -V(1-V)(S - lambda), dV/dlambda = V(1-V) beta,
-// dV/dS0 = -V(1-V) beta S/S0; dE/dtheta = -sum s fac dV/dtheta.
+// dV/dS0 = -V(1-V) beta S/S0; dE/dtheta = -sum s fac dV/dtheta.  ADJ also: dE/dR from the
+// fixed-point chain sums; GBSW the per-atom parts of dE/drscale and dE/droffset
+// (R' = rscale (R + roffset)).
+// The first S workgroups add up the systems' energies.
 template <bool ADJ>
 __global__ void __launch_bounds__(64) k_owner_reduce(KParams p) {
-    if (batch_fatal(p)) return;
-    const int i = blockIdx.x, lane = threadIdx.x;
+    const int lane = threadIdx.x;
+    const bool fatal = batch_fatal(p);
+    if ((int)blockIdx.x < p.S) {
+        if (!fatal)
+            system_energy(p, blockIdx.x, lane);
+        else if (lane == 0)
+            p.energy[blockIdx.x] = 0.0;
+        return;
+    }
+    if (fatal) return;
+    const int i = blockIdx.x - p.S;
     const int s = p.atom_sys[i];
     const SysDesc& sd = p.sys[s];
     const int Q = sd.Q, qb = sd.quad_base;
@@ -2742,27 +2753,11 @@ __global__ void __launch_bounds__(64) k_owner_reduce(KParams p) {
             p.theta_atom[TH_BETA * p.N + i] = tb;
             p.theta_atom[TH_LAMBDA * p.N + i] = tl;
             p.theta_atom[TH_S0 * p.N + i] = sd.S0 != 0.f ? ts / (double)sd.S0 : 0.0;
+            const double g = -(double)p.dedr_fix[i] / kFix32;  // dE/dR'_j (GBSW) or dE/dR_j
+            p.dedr[i] = gbsw ? g * (double)sd.rscale : g;
+            p.theta_atom[TH_RSCALE * p.N + i] = gbsw ? g * (p.radius[i] + (double)sd.roffset) : 0.0;
+            p.theta_atom[TH_ROFFSET * p.N + i] = gbsw ? g * (double)sd.rscale : 0.0;
         }
-    }
-}
-
-// Adjoint, per atom: dE/dR from the fixed-point chain sums; GBSW also the per-atom parts of
-// dE/drscale and dE/droffset (R' = rscale (R + roffset)).
-__global__ void k_adjoint_atoms(KParams p) {
-    if (batch_fatal(p)) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= p.N) return;
-    const SysDesc& sd = p.sys[p.atom_sys[i]];
-    const double g = -(double)p.dedr_fix[i] / kFix32;  // dE/dR'_j (GBSW) or dE/dR_j
-    double* th = p.theta_atom;
-    if (sd.vol_kind == VOL_GBSW) {
-        p.dedr[i] = g * (double)sd.rscale;
-        th[TH_RSCALE * p.N + i] = g * (p.radius[i] + (double)sd.roffset);
-        th[TH_ROFFSET * p.N + i] = g * (double)sd.rscale;
-    } else {
-        p.dedr[i] = g;
-        th[TH_RSCALE * p.N + i] = 0.0;
-        th[TH_ROFFSET * p.N + i] = 0.0;
     }
 }
 
@@ -2912,12 +2907,11 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
     const bool adj = p.adjoint != 0;
     mark(0);
     const int clear_blocks = std::max(1, std::min((p.cell_total + 255) / 256, 4096));
-    hipLaunchKernelGGL(k_clear, dim3(clear_blocks), dim3(256), 0, stream, p);
-    hipLaunchKernelGGL(k_bbox, dim3(p.bbox_slices, p.S), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(k_bbox, dim3(p.bbox_slices * p.S + clear_blocks), dim3(256), 0, stream, p);
     hipLaunchKernelGGL(k_grid_fill, dim3(p.N), dim3(256), 0, stream, p);
-    err = scan_exclusive(p.cell_fill, p.cell_start, p.cell_total, p.scan_tmp, p.entry_cap, p.flags_all,
-                         FLAG_ENTRY_OVERFLOW, stream);
-    if (err != hipSuccess) return err;
+    const int tiles = scan_tiles(p.cell_total);
+    if (tiles > kScanTile || tiles < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_list_starts, dim3(tiles), dim3(kScanThreads), 0, stream, p);
     const dim3 sort_grid(std::max(1, std::min(p.cell_total, 65536)));
     if (kinds[VOL_GBSW])
         hipLaunchKernelGGL(k_grid_sort<true>, sort_grid, dim3(64), 0, stream, p);
@@ -2988,7 +2982,6 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
         else
             hipLaunchKernelGGL(k_atom_chain<false>, dim3(p.n_colblocks), dim3(kChainGroups * kWave), 0, stream, p);
     }
-    hipLaunchKernelGGL(k_energy, dim3(p.S), dim3(1024), 0, stream, p);
     mark(6);
     for (int vk = 0; vk < VOL_KINDS; ++vk) {
         if (!kinds[vk]) continue;
@@ -2999,11 +2992,10 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
     }
     mark(7);
     if (adj) {
-        hipLaunchKernelGGL(k_owner_reduce<true>, dim3(p.N), dim3(64), 0, stream, p);
-        hipLaunchKernelGGL(k_adjoint_atoms, dim3((p.N + 255) / 256), dim3(256), 0, stream, p);
+        hipLaunchKernelGGL(k_owner_reduce<true>, dim3(p.S + p.N), dim3(64), 0, stream, p);
         hipLaunchKernelGGL(k_theta_reduce, dim3(p.S), dim3(kThetaThreads), 0, stream, p);
     } else {
-        hipLaunchKernelGGL(k_owner_reduce<false>, dim3(p.N), dim3(64), 0, stream, p);
+        hipLaunchKernelGGL(k_owner_reduce<false>, dim3(p.S + p.N), dim3(64), 0, stream, p);
     }
     mark(8);
     return hipGetLastError();
@@ -3044,10 +3036,20 @@ __global__ void k_export(double* dst, const double* src, size_t n) {
         dst[k] = src[k];
 }
 
-__global__ void k_export_forces(double* dst, const long long* force_fix, int n) {
-    for (long long k = blockIdx.x * blockDim.x + threadIdx.x; k < 3ll * n; k += (long long)gridDim.x * blockDim.x) {
-        const long long a = k / 3, d = k - 3 * a;
-        dst[k] = (double)force_fix[d * n + a] * (1.0 / kFix32);
+// A header of nh doubles, the forces of n atoms (atom-major doubles, behind it) and na doubles of the
+// adjoint, each to the host.
+__global__ void k_export_results(double* dst, const double* header, size_t nh, const long long* force_fix, size_t n,
+                                 double* adj_dst, const double* adj, size_t na) {
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < nh + 3 * n + na; k += stride) {
+        if (k < nh) {
+            dst[k] = header[k];
+        } else if (k < nh + 3 * n) {
+            const size_t a = (k - nh) / 3, d = k - nh - 3 * a;
+            dst[k] = (double)force_fix[d * n + a] * (1.0 / kFix32);
+        } else {
+            adj_dst[k - nh - 3 * n] = adj[k - nh - 3 * n];
+        }
     }
 }
 
@@ -3055,8 +3057,12 @@ unsigned export_blocks(size_t n) { return (unsigned)std::min<size_t>(std::max<si
 
 }  // namespace
 
-hipError_t launch_export_forces(double* dst, const long long* force_fix, int n, hipStream_t stream) {
-    hipLaunchKernelGGL(k_export_forces, dim3(export_blocks(3 * (size_t)n)), dim3(256), 0, stream, dst, force_fix, n);
+hipError_t launch_export_results(char* dst, const char* header, size_t header_bytes, const long long* force_fix, int n,
+                                 char* adj_dst, const char* adj, size_t adj_bytes, hipStream_t stream) {
+    const size_t nh = header_bytes / sizeof(double), na = adj_bytes / sizeof(double);
+    hipLaunchKernelGGL(k_export_results, dim3(export_blocks(nh + 3 * (size_t)n + na)), dim3(256), 0, stream,
+                       reinterpret_cast<double*>(dst), reinterpret_cast<const double*>(header), nh, force_fix, (size_t)n,
+                       reinterpret_cast<double*>(adj_dst), reinterpret_cast<const double*>(adj), na);
     return hipGetLastError();
 }
 
