@@ -168,7 +168,7 @@ struct gbi_ctx {
     // device buffers
     DevBuf<gbi::SysDesc> d_sys;
     DevBuf<gbi::SysGeom> geom;
-    DevBuf<int> flags_all, atom_sys, cell_sys, bin_order, bbox_done;
+    DevBuf<int> flags_all, atom_sys, cell_sys, bin_order, bin_group, bbox_done;
     DevBuf<double> bbox_part;
     DevBuf<int4> pair_tiles;
     DevBuf<int> colblk;
@@ -283,6 +283,7 @@ struct gbi_ctx {
         colpart.release();
         bbox_part.release();
         bbox_done.release();
+        bin_group.release();
         DevBuf<int>* ib[] = {&flags_all,      &atom_sys,     &cell_sys,       &bin_order,       &cell_fill,
                              &cell_start,     &cell_count_eff, &cell_atoms_tmp, &cell_atoms, &cell_pt_count,
                              &cell_act_count, &work_act,     &work,           &scan_tmp};
@@ -898,6 +899,8 @@ gbi::KParams make_kparams(gbi_ctx& c, bool adjoint) {
     k.colpart_total = c.colpart_total;
     k.adjoint = adjoint ? 1 : 0;
     k.bin_order = c.bin_order.p;
+    k.bin_group = c.bin_group.p;
+    k.n_bin_groups = (int)c.bin_group.n;
     k.persist_blocks = c.num_cus * std::max(1, c.tuning.blocks_per_cu);
     k.sys = c.d_sys.p;
     k.geom = c.geom.p;
@@ -1275,7 +1278,7 @@ gbi_status setup_host(gbi_ctx& c, int S, const int32_t* n_atoms, const double* c
 struct HostTables {
     std::vector<double> off, pw;
     std::vector<float> r2;
-    std::vector<int> atom_sys, bin_order, pair_atom;
+    std::vector<int> atom_sys, bin_order, bin_group, pair_atom;
 };
 
 gbi_status host_tables(const gbi_ctx& c, HostTables& t) {
@@ -1331,6 +1334,8 @@ gbi_status host_tables(const gbi_ctx& c, HostTables& t) {
     for (int w = 0; w < c.N;)
         for (int s = 0; s < c.S; ++s)
             if (next[s] < c.sys[s].N) t.bin_order[w++] = seq[s][next[s]++];
+    for (int a : t.bin_order)
+        if ((a - c.sys[t.atom_sys[a]].atom_begin) % gbi::kBinAtoms == 0) t.bin_group.push_back(a);
     t.pair_atom.resize(c.N);
     for (int k = 0; k < c.N; ++k) t.pair_atom[k] = k;
     return GBI_OK;
@@ -1394,6 +1399,7 @@ gbi_status create_batch(int S, const int32_t* n_atoms, const double* charge, con
     HIP_TRY(c->vval.ensure(any_gbmv ? NQ : 1));
     HIP_TRY(c->atom_nact.ensure(N));
     HIP_TRY(c->bin_order.ensure(N));
+    HIP_TRY(c->bin_group.ensure(t.bin_group.size()));
     HIP_TRY(c->pair_atom.ensure(N));
     HIP_TRY(hipMemcpyAsync(c->quad_off.p, t.off.data(), sizeof(double) * t.off.size(), hipMemcpyHostToDevice, c->stream));
     HIP_TRY(hipMemcpyAsync(c->quad_pw.p, t.pw.data(), sizeof(double) * t.pw.size(), hipMemcpyHostToDevice, c->stream));
@@ -1401,6 +1407,8 @@ gbi_status create_batch(int S, const int32_t* n_atoms, const double* charge, con
     HIP_TRY(hipMemcpyAsync(c->atom_sys.p, t.atom_sys.data(), sizeof(int) * N, hipMemcpyHostToDevice, c->stream));
     HIP_TRY(hipMemcpyAsync(c->pair_atom.p, t.pair_atom.data(), sizeof(int) * N, hipMemcpyHostToDevice, c->stream));
     HIP_TRY(hipMemcpyAsync(c->bin_order.p, t.bin_order.data(), sizeof(int) * N, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(hipMemcpyAsync(c->bin_group.p, t.bin_group.data(), sizeof(int) * t.bin_group.size(), hipMemcpyHostToDevice,
+                           c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->pair_order_host = t.pair_atom;
     ST_TRY(upload_atoms(*c));

@@ -38,6 +38,7 @@ constexpr int kFatalFlags =
 constexpr int kWorkCounters = 8;         // KParams::work
 constexpr int kMaxAtomChunk = 256;       // atoms staged in LDS per chunk (volume pass)
 constexpr int kQBits = 11;               // packed point = (atom << 11) | q, Q <= 2047
+constexpr int kBinAtoms = 2;             // atoms per workgroup of the binning by bricks
 constexpr int kMaxAtoms = 1 << (32 - kQBits);
 constexpr float kQuantum = 16777216.0f;  // 2^24: chain-rule partials are summed exactly on this grid
 constexpr int kBrickStride = 32;         // ints between brick counters (one 128-byte line each)
@@ -184,6 +185,8 @@ struct KParams {
     int adjoint;             // also compute dE/dR, dE/dq, dE/dtheta
     const int* bin_order;    // N: atom visiting order of the binning pass (systems in turn, each
                              // with a stride coprime to its size so concurrent workgroups hit distant cells)
+    const int* bin_group;    // n_bin_groups: first atoms of the groups of kBinAtoms atoms, visited alike
+    int n_bin_groups;
     int persist_blocks;      // workgroups of the per-cell passes
     const SysDesc* sys;
     SysGeom* geom;

@@ -850,8 +850,8 @@ __device__ inline void quad_point(const KParams& p, double xi, double yi, double
     pt[2] = zi + p.quad_off[3 * row + 2];
 }
 
-// Binning of the GBMV kinds.  k_point_bin: one workgroup per atom (systems in turn, each visited with a stride
-// coprime to its size so concurrent workgroups hit distant counters) finds the cell of every
+// Binning of the GBMV kinds.  k_point_bin: one workgroup per atom or group of atoms (systems in
+// turn, each visited with a stride coprime to its size so concurrent workgroups hit distant counters) finds the cell of every
 // quadrature point (FP64, the oracle's arithmetic), counts its points per key in an LDS hash
 // table (local ranks) and reserves each key's slots with one global atomic; these returning
 // atomics bound the pass (3.4 M on per-cell counters took 0.135 ms of 0.19 for 5,000 atoms).
@@ -871,9 +871,16 @@ __device__ inline void quad_point(const KParams& p, double xi, double yi, double
 //   cells: the record (the point relative to its cell's corner in FP32, the packed point),
 //     16 bytes.  There the binning pass is bound by its atomics, not by its writes.
 // Points outside the grid or in an empty cell get their volume directly.
-constexpr int kBinHash = 2048;  // > Q: the table never fills
-// Threads per workgroup: bricks 512 (4 points per thread, 56 VGPRs, 8 waves per SIMD: 0.088 ->
-// 0.075 ms at 5,000 GBMV-II atoms against 256 threads); cells 256 (8 points per thread: with 512
+// Atoms per workgroup: neighbours in the numbering are mostly neighbours in space, whose points
+// share bricks: half the atomics, and stores to a brick twice as long.  The passes that bin took
+// 0.108 ms at 5,000 GBMV-II atoms with one atom per workgroup, 0.095 with two; 0.089 with two and
+// the thread's loads and its atomics in flight together (a mixed batch of 16: 0.720, 0.670, 0.644).
+// Four per workgroup of 1,024 threads: 0.090 and 0.664, and 125 workgroups for 500 atoms.
+template <bool BRICKS>
+constexpr int bin_atoms() { return BRICKS ? kBinAtoms : 1; }
+static_assert(kBinAtoms <= 4, "packed table entries of k_point_bin");
+// Threads per workgroup: bricks 512 (8 points per thread, 8 waves per SIMD; 1,024 for two atoms
+// took 0.707 ms of binning for the batch against 0.670); cells 256 (8 points per thread: with 512
 // threads its pass, bound by its returning atomics, took 0.62 ms against 0.42 for 25,000 atoms on
 // a 0.20 nm grid).
 template <bool BRICKS>
@@ -906,14 +913,17 @@ __device__ inline uint32_t* pt_slot(const KParams& p, const SysDesc& sd, int c, 
 // cost one); cells: register bound at 5.
 template <bool BRICKS>
 __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point_bin(KParams p) {
-    constexpr int kBinThreads = bin_threads<BRICKS>();
+    constexpr int kBinThreads = bin_threads<BRICKS>(), kAtoms = bin_atoms<BRICKS>();
+    constexpr int kBinHash = kAtoms << kQBits;  // more than the points: the table never fills
+    constexpr int kHashBits = kQBits + (kAtoms > 2 ? 2 : kAtoms - 1);
     constexpr int kBinPer = kBinHash / kBinThreads;  // points per thread
+    static_assert(kBinHash == 1 << kHashBits, "a power of two");
     // t_cnt: the points per key, then the key's first reserved slot
     __shared__ int t_key[kBinHash], t_cnt[kBinHash];
     if (batch_fatal(p)) return;
     const int tid = threadIdx.x;
-    const int i = p.bin_order[blockIdx.x];
-    const int s = p.atom_sys[i];
+    const int i0 = BRICKS ? p.bin_group[blockIdx.x] : p.bin_order[blockIdx.x];
+    const int s = p.atom_sys[i0];
     // copies: the fields are read once, not again per point (the LDS atomics between points
     // keep the compiler from reusing values loaded through a reference)
     const SysDesc sd = p.sys[s];
@@ -923,82 +933,105 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
     if ((sk > 1) != BRICKS || sd.vol_kind == VOL_GBSW) return;
     const long long key_slots = (long long)sk * sk * sk * pt_cap;
     const long long prec_base = sd.prec_base;
-    const int pbase = sd.pt_base + (i - sd.atom_begin) * Q;
+    const int npts = min(kAtoms, sd.atom_end - i0) * Q;
+    const int pbase = sd.pt_base + (i0 - sd.atom_begin) * Q;
     const float v_empty = sd.v_empty;
     const float sig_empty = sd.vol_kind == VOL_GBMV1 ? 0.0f : __int_as_float(0x7fc00000);
-    const double xi = p.pos[3 * i], yi = p.pos[3 * i + 1], zi = p.pos[3 * i + 2];
     for (int k = tid; k < kBinHash; k += kBinThreads) {
         t_key[k] = -1;
         t_cnt[k] = 0;
     }
     __syncthreads();
-    int h[kBinPer], rank[kBinPer], cell[kBinPer];       // bricks: the point's cell in its brick
+    // Two passes over the thread's points, so that the cells' counts are all on their way before
+    // the first is waited for: the keys, then the table.
+    int key[kBinPer], in_cell[kBinPer];
+    // the point's table entry, its rank there and (bricks) its cell in the brick; all ones: none
+    uint32_t at[kBinPer];
+    constexpr int kCellBits = 6, kRankBits = kHashBits;
     float rx[kBinPer], ry[kBinPer], rz[kBinPer];        // cells: the record's coordinates
 #pragma unroll
     for (int u = 0; u < kBinPer; ++u) {
-        h[u] = -1;
-        rank[u] = 0;
-        cell[u] = 0;
+        key[u] = -1;
+        at[u] = 0u;
+        in_cell[u] = 0;
         rx[u] = ry[u] = rz[u] = 0.f;
-        const int q = tid + kBinThreads * u;
-        if (q >= Q) continue;
-        const int row = qb + q;
-        int c = -1, idx[3] = {0, 0, 0};
-        double pt[3] = {0.0, 0.0, 0.0};
-        quad_point(p, xi, yi, zi, row, pt);
-        c = sd.periodic ? point_cell_periodic(G, pt, idx) : point_cell(sd, G, pt[0], pt[1], pt[2], idx);
-        if (c >= 0 && p.cell_count_eff[cb + c] == 0) c = -1;
-        if (c < 0) {
-            p.vval[pbase + q] = v_empty;
-            if (p.adjoint) p.vsig[pbase + q] = sig_empty;
-            continue;
-        }
-        int key = c;
+        if (u * kBinThreads >= npts) continue;
+        const int k = min(tid + kBinThreads * u, npts - 1);  // point k % Q of atom i0 + k / Q
+        int a = 0;
+        for (int m = 1; m < kAtoms; ++m) a += k >= m * Q;
+        const int row = qb + k - a * Q, i = i0 + a;
+        int idx[3] = {0, 0, 0};
+        double pt[3];
+        quad_point(p, p.pos[3 * i], p.pos[3 * i + 1], p.pos[3 * i + 2], row, pt);
+        const int c = sd.periodic ? point_cell_periodic(G, pt, idx) : point_cell(sd, G, pt[0], pt[1], pt[2], idx);
+        if (c < 0) continue;
+        in_cell[u] = p.cell_count_eff[cb + c];
         if constexpr (bricks) {
             const int bx = idx[0] / sk, by = idx[1] / sk, bz = idx[2] / sk;
-            key = (bx * G.nb[1] + by) * G.nb[2] + bz;
-            cell[u] = ((idx[0] - bx * sk) * sk + (idx[1] - by * sk)) * sk + (idx[2] - bz * sk);
+            key[u] = (bx * G.nb[1] + by) * G.nb[2] + bz;
+            at[u] = ((idx[0] - bx * sk) * sk + (idx[1] - by * sk)) * sk + (idx[2] - bz * sk);
         } else {
+            key[u] = c;
             double corner[3];  // point_record's arithmetic, pt already wrapped
             cell_corner_idx(sd, G, idx[0], idx[1], idx[2], corner);
             rx[u] = (float)(pt[0] - corner[0]);
             ry[u] = (float)(pt[1] - corner[1]);
             rz[u] = (float)(pt[2] - corner[2]);
         }
-        // open addressing; at most Q < kBinHash distinct keys, so a free entry always exists
-        int e = (int)(((unsigned)key * 2654435761u) >> 21);
+    }
+#pragma unroll
+    for (int u = 0; u < kBinPer; ++u) {
+        const uint32_t in_brick = at[u];
+        at[u] = ~0u;
+        const int k = tid + kBinThreads * u;
+        if (k >= npts) continue;
+        if (key[u] < 0 || in_cell[u] == 0) {
+            p.vval[pbase + k] = v_empty;
+            if (p.adjoint) p.vsig[pbase + k] = sig_empty;
+            continue;
+        }
+        // open addressing; fewer than kBinHash distinct keys, so a free entry always exists
+        int e = (int)(((unsigned)key[u] * 2654435761u) >> (32 - kHashBits));
         for (int probe = 0; probe < kBinHash; ++probe) {
-            const int old = atomicCAS(&t_key[e], -1, key);
-            if (old == -1 || old == key) break;
+            const int old = atomicCAS(&t_key[e], -1, key[u]);
+            if (old == -1 || old == key[u]) break;
             e = (e + 1) & (kBinHash - 1);
         }
-        h[u] = e;
-        rank[u] = atomicAdd(&t_cnt[e], 1);
+        at[u] = ((uint32_t)e << (kRankBits + kCellBits)) | ((uint32_t)atomicAdd(&t_cnt[e], 1) << kCellBits) | in_brick;
     }
     __syncthreads();
-    for (int k = tid; k < kBinHash; k += kBinThreads) {
-        const int n = t_cnt[k];
+    // all of the thread's reservations are on their way before the first is waited for
+    int first[kBinPer];
+#pragma unroll
+    for (int u = 0; u < kBinPer; ++u) {
+        const int k = tid + kBinThreads * u, n = t_cnt[k];
+        first[u] = 0;
         if (n > 0) {
             if constexpr (bricks)
-                t_cnt[k] = atomicAdd(&p.brick_count[(long long)(sd.brick_base + t_key[k]) * kBrickStride], n);
+                first[u] = atomicAdd(&p.brick_count[(long long)(sd.brick_base + t_key[k]) * kBrickStride], n);
             else
-                t_cnt[k] = atomicAdd(&p.cell_ctr[cell_ctr_slot(p, cb + t_key[k])], n);
+                first[u] = atomicAdd(&p.cell_ctr[cell_ctr_slot(p, cb + t_key[k])], n);
         }
     }
+#pragma unroll
+    for (int u = 0; u < kBinPer; ++u) t_cnt[tid + kBinThreads * u] = first[u];
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kBinPer; ++u) {
-        if (h[u] < 0) continue;
-        const int q = tid + kBinThreads * u;
-        const long long slot = (long long)t_cnt[h[u]] + rank[u];
-        const int key = t_key[h[u]];
-        const uint32_t packed = ((uint32_t)i << kQBits) | (uint32_t)q;
+        if (at[u] == ~0u) continue;
+        const int k = tid + kBinThreads * u;
+        int a = 0;
+        for (int m = 1; m < kAtoms; ++m) a += k >= m * Q;
+        const int e = at[u] >> (kRankBits + kCellBits);
+        const long long slot = (long long)t_cnt[e] + ((at[u] >> kCellBits) & ((1u << kRankBits) - 1u));
+        const int of = t_key[e];
+        const uint32_t packed = ((uint32_t)(i0 + a) << kQBits) | (uint32_t)(k - a * Q);
         if (slot >= key_slots) {
             raise_flag(p, s, FLAG_POINT_OVERFLOW);  // bricks: then some cell of the brick has more than pt_cap
         } else if constexpr (bricks) {
-            p.brick_rec[prec_base + key * key_slots + slot] = make_uint2(packed, (uint32_t)cell[u]);
+            p.brick_rec[prec_base + of * key_slots + slot] = make_uint2(packed, at[u] & ((1u << kCellBits) - 1u));
         } else {
-            p.prec[prec_base + (long long)key * pt_cap + slot] = make_float4(rx[u], ry[u], rz[u], __uint_as_float(packed));
+            p.prec[prec_base + (long long)of * pt_cap + slot] = make_float4(rx[u], ry[u], rz[u], __uint_as_float(packed));
         }
     }
 }
@@ -2929,7 +2962,7 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
         if (p.gbsw_other) hipLaunchKernelGGL(k_gbsw_points<false>, grid, dim3(kGbswThreads), lds, stream, p);
     }
     if (p.any_cellbin) hipLaunchKernelGGL(k_point_bin<false>, dim3(p.N), dim3(bin_threads<false>()), 0, stream, p);
-    if (p.any_bricks) hipLaunchKernelGGL(k_point_bin<true>, dim3(p.N), dim3(bin_threads<true>()), 0, stream, p);
+    if (p.any_bricks) hipLaunchKernelGGL(k_point_bin<true>, dim3(p.n_bin_groups), dim3(bin_threads<true>()), 0, stream, p);
     if (p.any_bricks)
         hipLaunchKernelGGL(k_point_split, dim3(std::max(1, std::min(p.brick_max, 4096)), p.S, kSplitParts), dim3(256),
                            0, stream, p);
