@@ -919,7 +919,11 @@ gbi::KParams make_kparams(gbi_ctx& c, bool adjoint) {
     k.bbox_part = c.bbox_part.p;
     k.bbox_done = c.bbox_done.p;
     k.bbox_slices = 1;
-    for (const SysHost& s : c.sys) k.bbox_slices = std::max(k.bbox_slices, gbi::bbox_slices(s.N));
+    k.fill_threads = 64;
+    for (const SysHost& s : c.sys) {
+        k.bbox_slices = std::max(k.bbox_slices, gbi::bbox_slices(s.N));
+        if (s.kind == gbi::GRID_FAITHFUL) k.fill_threads = 128;
+    }
     k.atom_sys = c.atom_sys.p;
     k.cell_sys = c.cell_sys.p;
     k.pos = c.pos.p;

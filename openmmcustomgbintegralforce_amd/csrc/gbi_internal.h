@@ -203,6 +203,7 @@ struct KParams {
     int* flags_all;          // OR of every system's flags
     double* bbox_part;       // S x kBboxMaxSlices x 10: per slice of a system's atoms min, max, sum (xyz), bad
     int* bbox_done;          // S + 1: slices of the system that are in bbox_part; systems done (0 between evaluations)
+    int fill_threads;        // workgroup of k_grid_fill (one atom): 64 where every grid is exact, else 128
     int bbox_slices;         // the largest slice count of a system (bbox_slices())
     const int* atom_sys;     // N
     const int* cell_sys;     // cell_total
