@@ -1068,7 +1068,10 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
 // global atomic (at most sk^3 per chunk) and writes the packed points in that order.
 constexpr int kSplitChunk = 2048;
 constexpr int kSplitPer = kSplitChunk / 256;
-constexpr int kSplitParts = 4;  // workgroups per brick (each takes every 4th chunk)
+// Workgroups per brick (each takes every 2nd chunk): a brick holds 1.3 chunks at the mean, 5 at the
+// most; 4 launched mostly empty ones (a mixed batch of 16: binning 0.644 ms, with 2 0.619, with 1
+// 0.612 but 0.093 instead of 0.090 at 5,000 GBMV-II atoms).
+constexpr int kSplitParts = 2;
 
 __global__ void __launch_bounds__(256) k_point_split(KParams p) {
     constexpr int kCells = kMaxBrickEdge * kMaxBrickEdge * kMaxBrickEdge;
