@@ -1154,12 +1154,14 @@ __global__ void __launch_bounds__(256) k_point_split(KParams p) {
 // Sorting all points into cells first (an atomic per atom and cell, 345 of them per atom, and a
 // pass over the cells' points with the atoms in LDS) took 0.42 + 0.36 ms at 25,000 atoms plus
 // 0.04 ms for the integrals, for points of which 93 % have V = 0 or 1 after an atom or two; this
-// kernel takes 0.274 ms (25k evaluation 1.43 -> 0.87 ms, the adjoint of 8 x 2,000 atoms 1.00 -> 0.70).
+// kernel took 0.274 ms (25k evaluation 1.43 -> 0.87 ms, the adjoint of 8 x 2,000 atoms 1.00 -> 0.70).
 // What bounds it: the gathers.  Each lane's 16 bytes lie on a line of their own (84 M L1 lookups,
 // 0.14 ms at one per cycle and CU); with V = 1 taken for every queued point it took 0.227 ms of
 // 0.359, and without the sub-cells' bits 0.073, in a form that gathered the 8-byte lists of all
 // points in step 1 (the 16-byte masks of a whole cell there instead: 0.274).  Whole lists in place
 // of the sub-cells': 0.51 ms.  VALU issue is at 60 %; the atomics of step 3 are 0.02 ms.
+// The exact grid's form asks for 8 waves per SIMD: with 106 scalar registers it had 7 (0.268 ->
+// 0.251 ms at 25,000 atoms, the adjoint of 8 x 2,000 0.155 -> 0.142; the spilled ones cost nothing).
 // ---------------------------------------------------------------------------
 constexpr int kGbswThreads = 256;
 constexpr int kGbswMaxQ = 1 << kQBits;
@@ -1250,7 +1252,7 @@ __device__ inline int gbsw_place(const KParams& p, const SysDesc& sd, const SysG
 constexpr int kGbswLds = 4 + 2;
 
 template <bool EXACT>
-__global__ void __launch_bounds__(kGbswThreads) k_gbsw_points(KParams p) {
+__global__ void __launch_bounds__(kGbswThreads, EXACT ? 8 : 1) k_gbsw_points(KParams p) {
     constexpr int kWords = kGbswMaxQ / 32;
     extern __shared__ __align__(16) char s_dyn[];
     __shared__ uint32_t s_bits[kWords];
