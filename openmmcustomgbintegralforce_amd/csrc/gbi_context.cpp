@@ -205,9 +205,9 @@ struct gbi_ctx {
     DevBuf<uint2> brick_rec;
     int brick_total = 0, brick_max = 0;
     bool any_bricks = false, any_cells = true, any_cellbin = false;
+    DevBuf<float4> grec;  // with the next three behind it in one allocation (layout)
     DevBuf<unsigned long long> cell_sub;
     DevBuf<ulonglong2> cell_mask;
-    DevBuf<float4> grec;
     DevBuf<float2> gval;
     DevBuf<int> atom_nact;
     DevBuf<float> quad_r2, vsig, vval;
@@ -298,10 +298,7 @@ struct gbi_ctx {
         brick_count.release();
         cell_ctr.release();
         brick_rec.release();
-        cell_sub.release();
-        cell_mask.release();
         grec.release();
-        gval.release();
         atom_nact.release();
         quad_r2.release();
         vsig.release();
@@ -542,13 +539,14 @@ gbi_status layout(gbi_ctx& c) {
     HIP_TRY(c.cell_count_eff.ensure(cells));
     // the binning pass's atomic counters get allocations of their own: sub-allocated beside
     // other small buffers, that pass was measured 15-20 % slower in some processes (0.26 vs
-    // 0.215 ms at 5k atoms, 0.49 vs 0.445 ms at 25k), never with its own allocation
-    HIP_TRY(c.cell_pt_count.ensure(cells, kOwnAllocation));
+    // 0.215 ms at 5k atoms, 0.49 vs 0.445 ms at 25k), never with its own allocation.  Only those
+    // that the context counts in: an allocation of 2 MB takes up to 0.2 ms of a first evaluation.
+    HIP_TRY(c.cell_pt_count.ensure(cells, any_cells ? 0 : kOwnAllocation));
     // counters permuted so that neighbouring cells count on different lines (ctr_slot) where points
     // reserve slots of their cells directly; bricks-only contexts count in cell_pt_count, their
     // split gaining nothing from it
     if (any_cells) HIP_TRY(c.cell_ctr.ensure((cells + 4095) / 4096 * 4096, kOwnAllocation));
-    HIP_TRY(c.brick_count.ensure(std::max<long long>(1, bricks) * gbi::kBrickStride, kOwnAllocation));
+    HIP_TRY(c.brick_count.ensure(std::max<long long>(1, bricks) * gbi::kBrickStride, any_bricks ? kOwnAllocation : 0));
     HIP_TRY(c.brick_rec.ensure(brick_slots));
     c.brick_total = (int)bricks;
     c.brick_max = (int)brick_max;
@@ -563,10 +561,11 @@ gbi_status layout(gbi_ctx& c) {
     HIP_TRY(c.scan_tmp.ensure((cells + 4095) / 4096 + 16));
     HIP_TRY(c.prec.ensure(std::max<long long>(1, slots)));
     if (c.kinds[gbi::VOL_GBSW]) {
-        HIP_TRY(c.grec.ensure(gslots));
-        HIP_TRY(c.gval.ensure(gslots));
-        HIP_TRY(c.cell_sub.ensure(64 * cells));
-        HIP_TRY(c.cell_mask.ensure(cells));
+        static_assert(sizeof(ulonglong2) == sizeof(float4) && 2 * sizeof(float2) == sizeof(float4), "pieces of 16 bytes");
+        HIP_TRY(c.grec.ensure(gslots + (1 + gbi::kGbswSubCells / 2) * cells + (gslots + 1) / 2));
+        c.cell_mask.p = reinterpret_cast<ulonglong2*>(c.grec.p + gslots);
+        c.cell_sub.p = reinterpret_cast<unsigned long long*>(c.cell_mask.p + cells);
+        c.gval.p = reinterpret_cast<float2*>(c.cell_sub.p + gbi::kGbswSubCells * cells);
     }
     HIP_TRY(c.cell_atoms_tmp.ensure(std::max<long long>(1, raw)));
     std::vector<int> cs(cells);

@@ -42,6 +42,7 @@ constexpr int kBinAtoms = 2;             // atoms per workgroup of the binning b
 constexpr int kMaxAtoms = 1 << (32 - kQBits);
 constexpr float kQuantum = 16777216.0f;  // 2^24: chain-rule partials are summed exactly on this grid
 constexpr int kBrickStride = 32;         // ints between brick counters (one 128-byte line each)
+constexpr int kGbswSubCells = 64;        // sub-cells of a GBSW cell (KParams::cell_sub)
 constexpr int kMaxBrickEdge = 4;         // cells per brick edge (<= 64 cells per brick)
 // Bounding box: a system's atoms in up to kBboxMaxSlices slices of about kBboxSlice atoms,
 // one workgroup each (the count depends on the system's size only).

@@ -700,6 +700,7 @@ constexpr int kSortLds = 256;  // cells with more raw members sort in global mem
 // the rounding of the FP32 coordinates and distances (1e-7 nm), so a point has the V that its
 // whole list would give.
 constexpr int kSub = 4;
+static_assert(kSub * kSub * kSub == kGbswSubCells && kGbswSubCells == kWave, "a lane per sub-cell");
 constexpr float kSubMargin = 1e-6f;
 constexpr unsigned long long kSubScan = 1ull << 63;
 
