@@ -26,7 +26,7 @@ COPY_BYTES = 256 << 20
 
 # the kernels of each pass (the binning pass: the brick or cell binning kernel and, for brick
 # binning, the split that moves the points into their cells)
-KERNELS = {"volume": ("k_volume",), "force": ("k_force",), "pairs": ("k_pairs",),
+KERNELS = {"volume": ("k_volume", "k_gbsw_points"), "force": ("k_force",), "pairs": ("k_pairs",),
            "bin": ("k_point_bin", "k_point_split")}
 
 
