@@ -375,7 +375,7 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
 
 /*
  * Replay evaluations from a captured hipGraph (one graph launch per evaluation instead of
- * ~25 kernel launches).  The graph is re-captured when buffers grow.  Not used while
+ * 11 to 16 kernel launches).  The graph is re-captured when buffers grow.  Not used while
  * profiling is enabled.
  */
 gbi_status gbi_set_graph(gbi_ctx* ctx, int32_t enable);

@@ -137,11 +137,13 @@ int brick_edge(const SysHost& s) {
 }
 
 // Point slots per cell: 1.6 times the points of a cell at 100 atoms/nm^3; of a GBSW system, whose
-// slots hold its active points only (7 % of the points in a 25,000-atom globule, at most three
-// times that in a cell near the surface), a quarter of it.  An overflow doubles them.
+// slots hold its active points only (7 % of the points in a 25,000-atom globule, three to five
+// times that in the fullest cells), half of it: with a third every first evaluation from 9,000
+// atoms on was done twice (globules of 5,000 to 25,000 atoms, a 6,400-atom liquid; 0.4 was enough
+// for six of each).  An overflow doubles them.
 int pt_cap_estimate(const SysHost& s) {
     if (s.kind == gbi::GRID_BRUTE) return std::max(1, s.N * s.Q);
-    const double share = s.vol == gbi::VOL_GBSW ? 0.25 : 1.0;
+    const double share = s.vol == gbi::VOL_GBSW ? 0.5 : 1.0;
     const double est = share * 1.6 * 100.0 * s.Q * s.g * s.g * s.g + 64.0;
     return std::max(1, (int)std::min<double>(est, (double)s.N * s.Q));
 }
