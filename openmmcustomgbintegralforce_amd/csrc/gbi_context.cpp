@@ -194,6 +194,7 @@ struct gbi_ctx {
     DevBuf<int> c_ex_ptr, c_ex_idx;
     bool any_cut = false, any_trunc = false;
     DevBuf<float> colpart;
+    DevBuf<uint8_t> pair_near;
     int n_tiles = 0, n_tiles4 = 0, n_tiles1 = 0, max_splits = 1, n_colblocks = 0;
     long long colpart_total = 1;
     DevBuf<double> pos, d_charge, d_radius, d_reach, quad_off, quad_pw, integrals, born, dbdi, dedi, pair_part,
@@ -286,6 +287,7 @@ struct gbi_ctx {
         c_ex_idx.release();
         cprog.reset();
         colpart.release();
+        pair_near.release();
         bbox_part.release();
         bbox_done.release();
         bin_group.release();
@@ -663,6 +665,8 @@ gbi_status build_tiles(gbi_ctx& c) {
     HIP_TRY(c.blk_hi.ensure(colblk.size()));
     HIP_TRY(c.pair_part.ensure((size_t)c.max_splits * 6 * c.N));
     HIP_TRY(c.colpart.ensure((size_t)5 * c.colpart_total));
+    if (c.any_cut)
+        HIP_TRY(c.pair_near.ensure((size_t)c.colpart_total / 64 + 1 + (size_t)c.n_colblocks * c.max_splits));
     HIP_TRY(hipMemcpyAsync(c.pair_tiles.p, tiles.data(), sizeof(int4) * tiles.size(), hipMemcpyHostToDevice,
                            c.stream));
     HIP_TRY(hipMemcpyAsync(c.colblk.p, colblk.data(), sizeof(int) * colblk.size(), hipMemcpyHostToDevice,
@@ -901,6 +905,7 @@ gbi::KParams make_kparams(gbi_ctx& c, bool adjoint) {
     k.max_splits = c.max_splits;
     k.n_colblocks = c.n_colblocks;
     k.colpart_total = c.colpart_total;
+    k.pair_near = c.any_cut ? c.pair_near.p : nullptr;
     k.adjoint = adjoint ? 1 : 0;
     k.bin_order = c.bin_order.p;
     k.bin_group = c.bin_group.p;

@@ -273,6 +273,7 @@ struct KParams {
     double* dbdi;            // 2 x N
     double* dedi;            // 2 x N
     double* pair_part;       // max_splits x 6 x N (fx, fy, fz, dE/dB, E, dE/dq): row sums per tile
+    uint8_t* pair_near;      // cutoff contexts: which partials the pair tiles wrote (near_column, near_row); else null
     float* colpart;          // 5 planes x colpart_total (fx, fy, fz, dE/dB, dE/dq) per (row block, atom)
     double* atom_energy;     // N
     double* dedq;            // N (adjoint)
