@@ -80,6 +80,15 @@ constexpr int kCellRun = 64;
 // the whole evaluation, so every later pass stops early.
 __device__ inline bool batch_fatal(const KParams& p) { return (*p.flags_all & kFatalFlags) != 0; }
 
+// The same, one thread's reading for the whole workgroup: where waves share LDS and other
+// workgroups of the same launch may raise such a flag meanwhile, waves that read it each for
+// themselves could part, and those that stay would use LDS that the others were to set.
+__device__ inline bool workgroup_fatal(const KParams& p, int& s_fatal) {
+    if (threadIdx.x == 0) s_fatal = batch_fatal(p);
+    __syncthreads();
+    return s_fatal != 0;
+}
+
 __device__ inline void raise_flag(const KParams& p, int s, int flag) {
     atomicOr(&p.geom[s].flags, flag);
     atomicOr(p.flags_all, flag);
@@ -946,7 +955,7 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
     static_assert(kBinHash == 1 << kHashBits, "a power of two");
     // t_cnt: the points per key, then the key's first reserved slot
     __shared__ int t_key[kBinHash], t_cnt[kBinHash];
-    if (batch_fatal(p)) return;
+    __shared__ int s_fatal;
     const int tid = threadIdx.x;
     const int i0 = BRICKS ? p.bin_group[blockIdx.x] : p.bin_order[blockIdx.x];
     const int s = p.atom_sys[i0];
@@ -967,7 +976,7 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
         t_key[k] = -1;
         t_cnt[k] = 0;
     }
-    __syncthreads();
+    if (workgroup_fatal(p, s_fatal)) return;  // (its barrier: the table is cleared)
     // Two passes over the thread's points, so that the cells' counts are all on their way before
     // the first is waited for: the keys, then the table.
     int key[kBinPer], in_cell[kBinPer];
@@ -1078,7 +1087,8 @@ __global__ void __launch_bounds__(256) k_point_split(KParams p) {
     constexpr int kCells = kMaxBrickEdge * kMaxBrickEdge * kMaxBrickEdge;
     __shared__ uint2 s_rec[kSplitChunk];
     __shared__ int s_cnt[kCells], s_off[kCells], s_base[kCells];
-    if (batch_fatal(p)) return;
+    __shared__ int s_fatal;
+    if (workgroup_fatal(p, s_fatal)) return;
     const int s = blockIdx.y, tid = threadIdx.x;
     const SysDesc sd = p.sys[s];  // copies, read once (as in k_point_bin)
     const SysGeom G = p.geom[s];
@@ -1258,9 +1268,8 @@ __global__ void __launch_bounds__(kGbswThreads, EXACT ? 8 : 1) k_gbsw_points(KPa
     extern __shared__ __align__(16) char s_dyn[];
     __shared__ uint32_t s_bits[kWords];
     __shared__ int s_pre[kWords];
-    __shared__ int s_nq, s_nact;
+    __shared__ int s_nq, s_nact, s_fatal;
     __shared__ double s_sum[2][kGbswThreads / kWave];
-    if (batch_fatal(p)) return;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
     // runs of atoms, neighbours along the chain, per XCD, so the lists that their points share stay
     // in its L2 (atoms in the strided binning order: 2.6 GB of L2 misses at 25,000 atoms against
@@ -1283,7 +1292,7 @@ __global__ void __launch_bounds__(kGbswThreads, EXACT ? 8 : 1) k_gbsw_points(KPa
     for (int d = 0; d < 3; ++d) sub[d] = kSub * fast_rcp((float)(!EXACT && sd.periodic ? G.step[d] : sd.g));
     if (tid == 0) s_nq = 0;
     if (tid < kWords) s_bits[tid] = 0u;
-    __syncthreads();
+    if (workgroup_fatal(p, s_fatal)) return;  // (its barrier: s_nq and s_bits are cleared)
     for (int q0 = 0; q0 < Q; q0 += kGbswThreads * kGbswBatch) {
         // kGbswBatch points per thread: their gathers are all in flight together
         int cell[kGbswBatch], bit[kGbswBatch];
@@ -1429,10 +1438,10 @@ constexpr int kWorkThreads = 1024;
 __global__ void __launch_bounds__(kWorkThreads) k_worklist(KParams p) {
     constexpr int kWaves = kWorkThreads / kWave;
     __shared__ int s_cnt[VOL_KINDS][kWaves], s_rec[kWaves];
-    __shared__ int s_base[VOL_KINDS + 1];
+    __shared__ int s_base[VOL_KINDS + 1], s_fatal;
     const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     const int stride = gridDim.x * blockDim.x;
-    if (batch_fatal(p)) return;
+    if (workgroup_fatal(p, s_fatal)) return;
     for (int base = blockIdx.x * blockDim.x; base < p.cell_total; base += stride) {
         const int c = base + (int)threadIdx.x;
         int vk = -1, s = 0, np = 0, na = 0, start = 0;
