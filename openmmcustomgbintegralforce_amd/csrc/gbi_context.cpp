@@ -1519,15 +1519,14 @@ NoAllocCaps noalloc_caps(const SysHost& s, const double* pos, const double* radi
         }
     int max_raw = 0, max_pts = 0;
     long long members = 0;
-    const int cap = (s.P.cell_cap > 0) ? s.P.cell_cap : INT_MAX;
     for (long long c = 0; c < ncell; ++c) {
         max_raw = std::max(max_raw, raw[c]);
         max_pts = std::max(max_pts, pts[c]);
-        members += std::min(raw[c], cap);
+        members += raw[c];  // the lists are laid out before they are cut at cell_cap
     }
     caps.tmp_cap = max_raw + max_raw / 8 + 16;
     caps.pt_cap = max_pts + max_pts / 8 + 16;
-    caps.entries = members + members / 16 + 1024;
+    caps.entries = members + members / 64 + 1024;
     return caps;
 }
 
