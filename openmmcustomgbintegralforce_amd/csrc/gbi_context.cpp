@@ -2096,12 +2096,17 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     sc.take(c.colpart, (size_t)5 * c.colpart_total), sc.take(c.force_fix, 3 * N);
     sc.take(c.cell_fill, cells), sc.take(c.cell_count_eff, cells), sc.take(c.cell_pt_count, cells);
     sc.take(c.cell_act_count, cells), sc.take(c.cell_sys, cells), sc.take(c.cell_start, cells + 1);
-    sc.take(c.work_a, cells), sc.take(c.work_b, cells), sc.take(c.work_act, cells);
     sc.take(c.scan_tmp, (cells + 4095) / 4096 + 16);
-    sc.take(c.cell_atoms_tmp, cells * (size_t)caps.tmp_cap), sc.take(c.cell_atoms, caps.entries);
-    sc.take(c.ent_pos, caps.entries), sc.take(c.ent_par, caps.entries);
+    // the worklist lies over the raw lists, which nothing reads once they are sorted
+    const size_t raw_at = sc.used;
+    sc.take(c.cell_atoms_tmp, cells * (size_t)caps.tmp_cap);
+    const size_t raw_end = sc.used;
+    sc.used = raw_at;
+    sc.take(c.work_a, cells), sc.take(c.work_b, cells), sc.take(c.work_act, cells);
+    sc.used = std::max(sc.used, raw_end);
+    sc.take(c.cell_atoms, caps.entries), sc.take(c.ent_pos, caps.entries), sc.take(c.ent_par, caps.entries);
     sc.take(c.prec, gbsw ? 1 : c.prec_total), sc.take(c.grec, gbsw ? c.prec_total : 1);
-    sc.take(c.gval, gbsw ? c.prec_total : 1), sc.take(c.cell_mask, gbsw ? cells : 1), sc.take(c.atom_nact, gbsw ? N : 1);
+    sc.take(c.gval, gbsw ? NQ : 1), sc.take(c.cell_mask, gbsw ? cells : 1), sc.take(c.atom_nact, gbsw ? N : 1);
     sc.take(c.frec0, gbsw ? 1 : NQ), sc.take(c.frec1, gbsw ? 1 : NQ);
     sc.take(c.frec2, c.kinds[gbi::VOL_GBMV2] ? NQ : 1), sc.take(c.vval, gbsw ? 1 : NQ), sc.take(c.vrec, NQ);
     sc.take(c.brick_count, gbi::kBrickStride), sc.take(c.brick_rec, 1);

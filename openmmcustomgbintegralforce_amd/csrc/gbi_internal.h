@@ -258,7 +258,7 @@ struct KParams {
     unsigned long long* cell_sub;  // cell_total x 64 (GBSW cells with atoms): the atoms that reach each sub-cell;
                                    // null in gbi_execute_noalloc
     float4* grec;            // GBSW systems: slots of their active points (prec_base, pt_cap as in prec)
-    float2* gval;            // per grec slot: V, rank among its owner's active points
+    float2* gval;            // per grec slot (by pid where cell_sub is null): V, rank among its owner's active points
     int* atom_nact;          // N: active points of each atom (GBSW)
     float4* frec0;           // NQ (GBMV): active points, grouped by cell (corner-relative FP32 point, packed point)
     float4* frec1;           // NQ: GBMV1 (dV/dS, V, 0, 0) / GBMV2 (c1, c2, c3, vx)

@@ -1397,7 +1397,8 @@ __global__ void __launch_bounds__(kGbswThreads, EXACT ? 8 : 1) k_gbsw_points(KPa
         }
         const long long o = sd.prec_base + (long long)c * sd.pt_cap + slot;
         p.grec[o] = make_float4(r[0], r[1], r[2], __uint_as_float(((uint32_t)i << kQBits) | (uint32_t)q));
-        p.gval[o] = make_float2(V, __int_as_float(k));
+        // (gbi_execute_noalloc has no room for another array of the slots' length)
+        p.gval[p.cell_sub ? o : sd.pt_base + (long long)(i - sd.atom_begin) * Q + q] = make_float2(V, __int_as_float(k));
     }
     double a0 = 0.0, a1 = 0.0;
     for (int q = tid; q < Q; q += kGbswThreads) {
@@ -2656,10 +2657,12 @@ __global__ void __launch_bounds__(64) k_force_gbsw(KParams p) {
             float2 g = make_float2(0.f, 0.f);
             if (valid) {
                 r = p.grec[ps + pb + lane];
-                g = p.gval[ps + pb + lane];
+                if (p.cell_sub) g = p.gval[ps + pb + lane];
             }
             const uint32_t pk = __float_as_uint(r.w);
             const int own = (int)(pk >> kQBits), row = sd.quad_base + (int)(pk & ((1u << kQBits) - 1));
+            const long long own_pid = sd.pt_base + (long long)(own - sd.atom_begin) * sd.Q;  // its first point
+            if (valid && !p.cell_sub) g = p.gval[own_pid + (row - sd.quad_base)];
             int b = 0;
             b = min(max((int)(r.x * per_nm[0]), 0), kSub - 1);
             b = b * kSub + min(max((int)(r.y * per_nm[1]), 0), kSub - 1);
@@ -2743,8 +2746,7 @@ __global__ void __launch_bounds__(64) k_force_gbsw(KParams p) {
                 }
             }
             if (valid)
-                p.vrec[sd.pt_base + (long long)(own - sd.atom_begin) * sd.Q + __float_as_int(g.y)] =
-                    make_float4(-ox, -oy, -oz, 0.f);
+                p.vrec[own_pid + __float_as_int(g.y)] = make_float4(-ox, -oy, -oz, 0.f);
         }
         __syncthreads();
         if (single) flush();
