@@ -594,7 +594,7 @@ gbi_status layout(gbi_ctx& c) {
 // J >= I (each unordered pair once).  K column blocks per tile: `pair_columns` / 64 when set, else the
 // smallest K that keeps about 12,800 tiles over the batch (every system's share of the block
 // pairs; with 8,192 the 25,000-atom pass and its reduction took 323 us, with 12,800 310).
-// Column partials: one entry per (row tile, atom) of each system.
+// Column partials: one entry per (row block, atom) of each system.
 void tile_layout(gbi_ctx& c, std::vector<int4>& tiles, std::vector<int>& colblk) {
     long long pairs_total = 0;
     for (const SysHost& s : c.sys) {
@@ -629,8 +629,7 @@ void tile_layout(gbi_ctx& c, std::vector<int4>& tiles, std::vector<int>& colblk)
         s.pair_splits = (nb + K - 1) / K;  // pieces of row block 0, the most of any block
         s.colpart_base = cp;
         s.blk_base = (int)colblk.size();
-        // row tiles that begin before column block J, for every J
-        cp += 64ll * (R == 1 ? (long long)nb * (nb - 1) / 2 : (long long)nb * nb / 4);
+        cp += 64ll * nb * (nb - 1) / 2;  // row blocks I < J for every column block J
         c.max_splits = std::max(c.max_splits, s.pair_splits);
         for (int I = 0; I < nb; ++I) {
             colblk.push_back(s.atom_begin + 64 * I);

@@ -1944,13 +1944,11 @@ __device__ inline bool blocks_apart(const KParams& p, const SysDesc& sd, const B
     return gap2 > sd.cut2_hi * 1.001f;
 }
 
-// Column partial of row tile t for local atom j (a row tile holds pair_rows blocks of 64; block
-// J = j / 64 meets the tiles that begin before it): triangular, the row tiles of one column block
-// stored one after the other, 64 atoms each.
-__device__ inline long long colpart_index(const SysDesc& sd, int t, int j) {
+// Column partial I of local atom j, one for each row block before its own (I < J = j / 64): triangular,
+// the partials of one column block stored one after the other, 64 atoms each.
+__device__ inline long long colpart_index(const SysDesc& sd, int I, int j) {
     const long long J = j / kWave;
-    const long long before = sd.pair_rows == 1 ? J * (J - 1) / 2 : J * J / 4;
-    return sd.colpart_base + (long long)kWave * (before + t) + (j - kWave * J);
+    return sd.colpart_base + (long long)kWave * (J * (J - 1) / 2 + I) + (j - kWave * J);
 }
 
 constexpr int kChainGroups = 16;  // wave groups of k_atom_chain
@@ -2156,11 +2154,12 @@ __global__ void __launch_bounds__(64 * WAVES) k_pairs(KParams p) {
 
 // Two row blocks per wave (pair_rows = 2), for large systems without cutoff or exclusions: lane l
 // holds rows l and 64 + l, which meet column (l + m) mod 64 together, so its LDS reads and the
-// rotation of its sums are paid once for two pairs (36 VALU slots per pair against 38, 44 before
-// dE/dB took one term for both atoms), and the column partials halve.  25,000 atoms: 0.368 -> 0.274
-// ms, VALU-bound (312 M pairs at 36 slots of 4.5 cycles: 0.31 ms at 2.4 GHz on 1,024 SIMDs).  A
-// tile's first two column blocks are its rows' own: the diagonal block of each row block, and
-// their mutual block once.
+// rotation of its sums are paid once for two pairs: 36 VALU instructions per pair against 40.
+// 25,000 atoms: 0.383 -> 0.303 ms, at the issue rate (172,000 VALU instructions per SIMD, 1.7 ns each).
+// The column sums leave twice per block, so that each holds 64 terms as in the other forms (one
+// partial of both rows' 128 terms took 0.288 ms, and k_atom_chain 0.026 instead of 0.033, but the
+// forces' error against FP64 rose from 2.55e-7 to 2.71e-7).  A tile's first two column blocks are its
+// rows' own: the diagonal block of each row block, and their mutual block once.
 template <bool ADJ>
 __global__ void __launch_bounds__(64) k_pairs2(KParams p) {
     __shared__ double s_px[64], s_py[64], s_pz[64];
@@ -2208,14 +2207,21 @@ __global__ void __launch_bounds__(64) k_pairs2(KParams p) {
             return pair_terms(s_px[c], s_py[c], s_pz[c], x[r], y[r], z[r], B[r], cj.y, kexp[r], cj.z);
         };
         const int own = (jb - tile.x) / kWave;  // 0, 1: the block of these rows
+        const int I_row = (tile.x - ab) / kWave;
         if (own > 1) {
-            for (int m = 0; m < kWave; ++m) {
-                const int c = (lane + m) & (kWave - 1);
-                const float4 cj = s_col[c];
+            // the column sums leave after 32 steps of two rows and start again: 64 terms each
+            for (int h = 0; h < 2; ++h) {
+                col = {};
+                for (int m = h * (kWave / 2); m < (h + 1) * (kWave / 2); ++m) {
+                    const int c = (lane + m) & (kWave - 1);
+                    const float4 cj = s_col[c];
 #pragma unroll
-                for (int r = 0; r < 2; ++r)
-                    add_pair<ADJ, true>(pair(r, c), Pq[r] * cj.x, Pq[r], P * cj.x, row[r], col);
-                rotate_sums<ADJ>(col);
+                    for (int r = 0; r < 2; ++r)
+                        add_pair<ADJ, true>(pair(r, c), Pq[r] * cj.x, Pq[r], P * cj.x, row[r], col);
+                    rotate_sums<ADJ>(col);
+                }
+                const int c = (lane + (h + 1) * (kWave / 2)) & (kWave - 1);  // the column whose sums lane holds
+                if (jb + c < ae) store_column<ADJ>(p, colpart_index(sd, I_row + h, jb + c - ab), col, s_col[c].w);
             }
         } else {
             // the diagonal of row block `own` from the row side, half the pair energy each
@@ -2237,9 +2243,9 @@ __global__ void __launch_bounds__(64) k_pairs2(KParams p) {
                     add_pair<ADJ, true>(pair(0, c), Pq[0] * qj, Pq[0], P * qj, row[0], col);
                     rotate_sums<ADJ>(col);
                 }
+                if (jv) store_column<ADJ>(p, colpart_index(sd, I_row, jj - ab), col, s_col[lane].w);
             }
         }
-        if (own > 0 && jv) store_column<ADJ>(p, colpart_index(sd, (tile.x - ab) / (2 * kWave), jj - ab), col, s_col[lane].w);
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             out[r][0] += row[r].fx;
@@ -2261,7 +2267,7 @@ __global__ void __launch_bounds__(64) k_pairs2(KParams p) {
 // Per atom, one workgroup per 64-atom block: the pair sums in a fixed order, then the self
 // term and dE/dI = dE/dB dB/dI (customGBEnergyPerParticle.cu; CharmmReferenceGBSW.cpp:257-273).
 // Thread (g, lane) sums, for atom lane of the block, the row pieces k = g, g + G, ... and the
-// column partials of row tiles t = g, g + G, ... in FP64 (G = 16 wave groups); the
+// column partials of row blocks I = g, g + G, ... in FP64 (G = 16 wave groups); the
 // groups are added in order.  The block's energy goes where its first atom's first row piece was
 // (k_owner_reduce adds the blocks').  ADJ: dE/dq and the Born-map parts of dE/dtheta.
 template <bool ADJ>
@@ -2277,7 +2283,6 @@ __global__ void __launch_bounds__(kChainGroups * kWave) k_atom_chain(KParams p) 
     const bool iv = i < sd.atom_end;
     const int rows = sd.pair_rows, tile = bj / rows;  // the block's row tile
     const int pieces = (sd.nblk - tile * rows + sd.pair_k - 1) / sd.pair_k;
-    const int col_tiles = (bj + rows - 1) / rows;     // the row tiles that begin before it
     const long long T = p.colpart_total;
     double a[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const int ic = min(i, sd.atom_end - 1);  // (lanes without an atom keep the wave whole)
@@ -2290,8 +2295,8 @@ __global__ void __launch_bounds__(kChainGroups * kWave) k_atom_chain(KParams p) 
         a[4] += in[4 * p.N + ic];
         if (ADJ) a[5] += in[5 * p.N + ic];
     };
-    auto add_column = [&](int t) {
-        const long long o = colpart_index(sd, t, ic - ab);
+    auto add_column = [&](int I) {
+        const long long o = colpart_index(sd, I, ic - ab);
         a[0] += p.colpart[o];
         a[1] += p.colpart[T + o];
         a[2] += p.colpart[2 * T + o];
@@ -2304,13 +2309,13 @@ __global__ void __launch_bounds__(kChainGroups * kWave) k_atom_chain(KParams p) 
             for (unsigned long long m = near_mask(rows_near, k0, pieces, grp, lane); m; m &= m - 1ull)
                 add_row(k0 + __ffsll(m) - 1);
         const uint8_t* cols_near = p.pair_near + near_column(sd, 0, bj);
-        for (int t0 = 0; t0 < col_tiles; t0 += kWave)
-            for (unsigned long long m = near_mask(cols_near, t0, col_tiles, grp, lane); m; m &= m - 1ull)
-                add_column(t0 + __ffsll(m) - 1);
+        for (int I0 = 0; I0 < bj; I0 += kWave)
+            for (unsigned long long m = near_mask(cols_near, I0, bj, grp, lane); m; m &= m - 1ull)
+                add_column(I0 + __ffsll(m) - 1);
     } else {
         for (int k = grp; k < pieces; k += kChainGroups) add_row(k);
 #pragma unroll 4
-        for (int t = grp; t < col_tiles; t += kChainGroups) add_column(t);
+        for (int I = grp; I < bj; I += kChainGroups) add_column(I);
     }
     for (int v = 0; v < 6; ++v) s_acc[grp][v][lane] = a[v];
     __syncthreads();
