@@ -58,12 +58,13 @@ constexpr int kDefaultBlocksPerCU = 256;
 // Cell edge of the exact GBSW grid (lists are exact at any edge): 0.20 nm measured fastest at
 // 5k and 25k atoms (0.15 nm: 14 % slower, more distinct cells to bin; 0.30 nm: longer lists).
 constexpr double kDefaultTightGrid = 0.20;
-// Form of a system's pair tiles, by its 64-atom blocks only, so that a system's sums are grouped
-// alike alone and in a batch.  Pair pass measured (us), 4 waves / one row block / two row blocks:
+// Form of a system's pair tiles, by the system alone (its 64-atom blocks, cutoff and exclusions), so
+// that its FP32 sums are grouped alike alone and in a batch; a tile's length, which follows the
+// batch, changes the order of FP64 sums only.  Pair pass measured (us), 4 waves / one row block / two row blocks:
 // 300 atoms 9.4 / 14.2 / -, 2,500 12.9 / 17.6 / 25.6, 5,000 25.6 / 27.3 / 33.3, 8,000 59 / 46 / 48.6,
 // 12,000 - / 102 / 87, 25,000 - / 339 / 274.
 constexpr int kPairWaves4Blocks = 48;   // up to 3,072 atoms: 4 waves (no gain above in a batch)
-constexpr int kPairRows2Blocks = 140;   // from 8,897 atoms, without cutoffs or exclusions: two row blocks
+constexpr int kPairRows2Blocks = 140;   // from 8,897 atoms, without cutoff or exclusions: two row blocks
 constexpr int kCutoffTileBlocks = 3;  // column blocks per pair tile of a cutoff system
 constexpr double kSigmoidFp64Above = 16.0;  // |beta lambda| above which GBMV sums S in FP64
 constexpr size_t kOwnAllocation = 2u << 20;  // bytes: a buffer not sub-allocated beside others
@@ -590,6 +591,11 @@ gbi_status layout(gbi_ctx& c) {
     return GBI_OK;
 }
 
+// Row blocks of a system's pair tiles.
+int tile_rows(const gbi_ctx& c, const SysHost& s) {
+    return !c.cprog && !s.cutoff() && s.excl.empty() && (s.N + 63) / 64 >= kPairRows2Blocks ? 2 : 1;
+}
+
 // Pair tiles: row block I (or blocks I, I + 1) x column blocks [J0, J1) of the same system,
 // J >= I (each unordered pair once).  K column blocks per tile: `pair_columns` / 64 when set, else the
 // smallest K that keeps about 12,800 tiles over the batch (every system's share of the block
@@ -602,14 +608,14 @@ void tile_layout(gbi_ctx& c, std::vector<int4>& tiles, std::vector<int>& colblk)
         pairs_total += nb * (nb + 1) / 2;
     }
     const long long target = 12800;
-    std::vector<int4> tiles1, tiles2;
+    std::vector<int4> tiles1, tiles2;  // (tiles: those of 4 waves)
     tiles.clear();
     colblk.clear();
     c.max_splits = 1;
     long long cp = 0;
     for (SysHost& s : c.sys) {
         const int nb = (s.N + 63) / 64;
-        const int R = !c.any_cut && !c.any_excl && !c.cprog && nb >= kPairRows2Blocks ? 2 : 1;
+        const int R = tile_rows(c, s);
         int K;
         if (c.tuning.pair_columns > 0) {
             K = std::max(1, c.tuning.pair_columns / 64);
@@ -1722,9 +1728,8 @@ gbi_status gbi_set_exclusions(gbi_ctx* ctx, int32_t system, int32_t n_pairs, con
             return fail(GBI_ERR_INVALID_ARGUMENT, "excluded pair out of range or of an atom with itself");
     s.excl.assign(pairs, pairs + 2 * (size_t)n_pairs);
     if (ctx->cprog) return build_custom_exclusions(*ctx);
-    const bool before = ctx->any_excl;
     ST_TRY(build_exclusions(*ctx));
-    if (ctx->any_excl != before) {  // tiles of two row blocks take no exclusions
+    if (tile_rows(*ctx, s) != s.pair_rows) {  // tiles of two row blocks take no exclusions
         ST_TRY(build_tiles(*ctx));
         if (ctx->cell_total > 0) ST_TRY(layout(*ctx));  // the tiles' shape lives in the descriptors
     }

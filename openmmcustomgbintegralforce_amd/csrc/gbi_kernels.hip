@@ -1953,8 +1953,7 @@ __device__ inline long long colpart_index(const SysDesc& sd, int I, int j) {
 
 constexpr int kChainGroups = 16;  // wave groups of k_atom_chain
 
-// pair_near: one byte per column partial of a row block (cutoff systems: tiles of one row block), then
-// one per row block and piece.
+// pair_near: one byte per column partial of a row block, then one per row block and piece.
 __device__ inline long long near_column(const SysDesc& sd, int I, int J) {
     return colpart_index(sd, I, kWave * J) / kWave;
 }
@@ -2152,7 +2151,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_pairs(KParams p) {
     }
 }
 
-// Two row blocks per wave (pair_rows = 2), for large systems without cutoff or exclusions: lane l
+// Two row blocks per wave (pair_rows = 2), for large systems without cutoff or exclusions of their own: lane l
 // holds rows l and 64 + l, which meet column (l + m) mod 64 together, so its LDS reads and the
 // rotation of its sums are paid once for two pairs: 36 VALU instructions per pair against 40.
 // 25,000 atoms: 0.383 -> 0.303 ms, at the issue rate (172,000 VALU instructions per SIMD, 1.7 ns each).
@@ -2221,6 +2220,7 @@ __global__ void __launch_bounds__(64) k_pairs2(KParams p) {
                     rotate_sums<ADJ>(col);
                 }
                 const int c = (lane + (h + 1) * (kWave / 2)) & (kWave - 1);  // the column whose sums lane holds
+                if (p.pair_near && lane == 0) p.pair_near[near_column(sd, I_row + h, (jb - ab) / kWave)] = 1;
                 if (jb + c < ae) store_column<ADJ>(p, colpart_index(sd, I_row + h, jb + c - ab), col, s_col[c].w);
             }
         } else {
@@ -2243,6 +2243,7 @@ __global__ void __launch_bounds__(64) k_pairs2(KParams p) {
                     add_pair<ADJ, true>(pair(0, c), Pq[0] * qj, Pq[0], P * qj, row[0], col);
                     rotate_sums<ADJ>(col);
                 }
+                if (p.pair_near && lane == 0) p.pair_near[near_column(sd, I_row, I_row + 1)] = 1;
                 if (jv) store_column<ADJ>(p, colpart_index(sd, I_row, jj - ab), col, s_col[lane].w);
             }
         }
@@ -2256,6 +2257,8 @@ __global__ void __launch_bounds__(64) k_pairs2(KParams p) {
             if (ADJ) out[r][5] += row[r].dq;
         }
     }
+    if (p.pair_near && lane < 2 && (tile.x - ab) / kWave + lane < sd.nblk)  // beside cutoff systems
+        p.pair_near[near_row(p, sd, (tile.x - ab) / kWave + lane, tile.w)] = 1;
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
         if (!iv[r]) continue;
@@ -2988,13 +2991,13 @@ __global__ void k_stats(KParams p, double* out) {
     }
 }
 
-// The pair tiles: those of 4 waves, of one row block, of two (no cutoffs or exclusions).
+// The pair tiles: those of 4 waves, of one row block, of two (systems without cutoff or exclusions).
 template <bool ADJ, bool CUT>
 void launch_pairs(const KParams& p, hipStream_t stream) {
     const int n2 = p.n_tiles - p.n_tiles4 - p.n_tiles1;
     if (p.n_tiles4 > 0) hipLaunchKernelGGL((k_pairs<ADJ, CUT, 4>), dim3(p.n_tiles4), dim3(4 * kWave), 0, stream, p);
     if (p.n_tiles1 > 0) hipLaunchKernelGGL((k_pairs<ADJ, CUT, 1>), dim3(p.n_tiles1), dim3(kWave), 0, stream, p);
-    if (!CUT && n2 > 0) hipLaunchKernelGGL(k_pairs2<ADJ>, dim3(n2), dim3(kWave), 0, stream, p);
+    if (n2 > 0) hipLaunchKernelGGL(k_pairs2<ADJ>, dim3(n2), dim3(kWave), 0, stream, p);
 }
 
 template <bool ADJ>
