@@ -205,12 +205,15 @@ __device__ inline void cell_corner(const SysDesc& sd, const SysGeom& G, int c, d
 
 __host__ __device__ inline int scan_tiles(int cells) { return (cells + kScanTile - 1) / kScanTile; }
 
-// By `blocks` workgroups, this one being b.
+// By `blocks` workgroups, this one being b.  The masks of empty GBSW cells belong here, whole lines at a
+// time: one store of 16 bytes per cell made k_grid_sort take 1.06 ms instead of 0.66 on a sparse grid of
+// 11 million cells.
 __device__ void clear_counters(const KParams& p, int b, int blocks) {
     const int first = b * (int)blockDim.x + (int)threadIdx.x, stride = blocks * (int)blockDim.x;
     for (int i = first; i < p.cell_total; i += stride) {
         p.cell_fill[i] = 0;
         p.cell_ctr[i] = 0;
+        if (p.cell_mask) p.cell_mask[i] = make_ulonglong2(0ull, ~0ull);  // no atom reaches it
     }
     for (int i = p.cell_total + first; i < p.ctr_len; i += stride) p.cell_ctr[i] = 0;
     for (int i = first; i < p.brick_total; i += stride) p.brick_count[(long long)i * kBrickStride] = 0;
@@ -793,7 +796,7 @@ __global__ void __launch_bounds__(kScanThreads) k_list_starts(KParams p) {
 // SUB: some system is GBSW (its cells also get their sub-cells' lists; without them the kernel
 // holds 6 registers and 1 KB of LDS less).
 template <bool SUB>
-__global__ void __launch_bounds__(64) k_grid_sort(KParams p) {
+__global__ void __launch_bounds__(64, 8) k_grid_sort(KParams p) {
     __shared__ __align__(16) int s_in[kSortLds];
     __shared__ int s_out[kSortLds];
     __shared__ float4 s_e[SUB ? kWave : 1];
@@ -807,10 +810,7 @@ __global__ void __launch_bounds__(64) k_grid_sort(KParams p) {
     for (int c = blockIdx.x; c < p.cell_total; c += gridDim.x) {
         const int n_raw = p.cell_fill[c];
         if (n_raw == 0) {
-            if (lane == 0) {
-                p.cell_count_eff[c] = 0;
-                if (SUB) p.cell_mask[c] = make_ulonglong2(0ull, ~0ull);  // no atom reaches it
-            }
+            if (lane == 0) p.cell_count_eff[c] = 0;  // (its cell_mask: clear_counters)
             continue;
         }
         const int s = p.cell_sys[c];
