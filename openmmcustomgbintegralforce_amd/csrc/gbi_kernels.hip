@@ -2665,7 +2665,7 @@ __global__ void __launch_bounds__(64) k_force_gbsw(KParams p) {
             float2 g = make_float2(0.f, 0.f);
             if (valid) {
                 r = p.grec[ps + pb + lane];
-                if (p.cell_sub) g = p.gval[ps + pb + lane];
+                g = p.gval[p.cell_sub ? ps + pb + lane : 0];
             }
             const uint32_t pk = __float_as_uint(r.w);
             const int own = (int)(pk >> kQBits), row = sd.quad_base + (int)(pk & ((1u << kQBits) - 1));
