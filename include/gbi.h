@@ -125,7 +125,8 @@ typedef struct gbi_stats {
     double n_active;      /* points with a chain-rule term (0 < V < 1 for GBSW) */
     double n_frc_pairs;   /* point/atom pairs the chain-rule pass visits (active points x their lists) */
     double slot_bytes;    /* bytes a binned point occupies in its cell's slots, averaged over the atoms:
-                             4 (packed point; systems binning by bricks) or 16 (FP32 record and packed point) */
+                             4 (packed point; systems binning by bricks), 16 (FP32 record and packed point) or 0
+                             (GBSW systems, whose points are not binned) */
 } gbi_stats;
 
 /* Device view of a context's buffers (for callers that keep data on the GPU). */

@@ -2264,7 +2264,8 @@ gbi_status gbi_get_stats(gbi_ctx* ctx, gbi_stats* stats) {
     stats->n_active = h[4];
     stats->n_frc_pairs = h[5];
     double slot = 0.0;
-    for (const SysHost& s : ctx->sys) slot += (brick_edge(s) > 1 ? 4.0 : 16.0) * s.N;
+    for (const SysHost& s : ctx->sys)
+        if (s.vol != gbi::VOL_GBSW) slot += (brick_edge(s) > 1 ? 4.0 : 16.0) * s.N;
     stats->slot_bytes = slot / ctx->N;
     return GBI_OK;
 }

@@ -3205,7 +3205,7 @@ hipError_t launch_add_forces_fixed(long long* dst, int padded_n, const long long
 
 hipError_t launch_stats(const KParams& p, double* out6, hipStream_t stream) {
     hipLaunchKernelGGL(k_stats, dim3(256), dim3(256), 0, stream, p, out6);
-    hipLaunchKernelGGL(k_stats_gbsw, dim3(p.N), dim3(kGbswThreads), 0, stream, p, out6);
+    if (p.gbsw_exact || p.gbsw_other) hipLaunchKernelGGL(k_stats_gbsw, dim3(p.N), dim3(kGbswThreads), 0, stream, p, out6);
     return hipGetLastError();
 }
 
