@@ -530,7 +530,11 @@ gbi_status layout(gbi_ctx& c) {
     // brick slots share the prec slot layout (a system binning by cells leaves its range unused)
     brick_slots = any_bricks ? slots : 1;
     if (cells > kMaxCells) return fail(GBI_ERR_GRID_TOO_LARGE, "more than 16M lookup cells in the batch");
-    if (slots * (long long)sizeof(float4) + gslots * (long long)(sizeof(float4) + sizeof(float2)) > (200ll << 30))
+    // GBSW: a record and a value per slot, two masks and the sub-cells' lists per cell
+    const long long gbytes = !c.kinds[gbi::VOL_GBSW] ? 0
+                                                     : gslots * (long long)(sizeof(float4) + sizeof(float2)) +
+                                                           cells * (long long)(sizeof(ulonglong2) + 8 * gbi::kGbswSubCells);
+    if (slots * (long long)sizeof(float4) + gbytes > (200ll << 30))
         return fail(GBI_ERR_GRID_TOO_LARGE, "point slots of the lookup grids exceed 200 GB");
     if (raw * (long long)sizeof(int) > (64ll << 30))
         return fail(GBI_ERR_GRID_TOO_LARGE, "raw cell lists of the lookup grids exceed 64 GB");
