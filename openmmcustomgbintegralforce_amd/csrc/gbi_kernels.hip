@@ -917,7 +917,8 @@ static_assert(kBinAtoms <= 4, "packed table entries of k_point_bin");
 // Threads per workgroup: bricks 512 (8 points per thread, 8 waves per SIMD; 1,024 for two atoms
 // took 0.707 ms of binning for the batch against 0.670); cells 256 (8 points per thread: with 512
 // threads its pass, bound by its returning atomics, took 0.62 ms against 0.42 for 25,000 atoms on
-// a 0.20 nm grid).
+// a 0.20 nm grid; with a thread's reservations in flight together, as by bricks, 0.63 against 0.42 for
+// 20,000 GBMV atoms there).
 template <bool BRICKS>
 constexpr int bin_threads() { return BRICKS ? 512 : 256; }
 
@@ -1035,21 +1036,23 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
         at[u] = ((uint32_t)e << (kRankBits + kCellBits)) | ((uint32_t)atomicAdd(&t_cnt[e], 1) << kCellBits) | in_brick;
     }
     __syncthreads();
-    // all of the thread's reservations are on their way before the first is waited for
-    int first[kBinPer];
+    if constexpr (bricks) {
+        // all of the thread's reservations are on their way before the first is waited for
+        int first[kBinPer];
 #pragma unroll
-    for (int u = 0; u < kBinPer; ++u) {
-        const int k = tid + kBinThreads * u, n = t_cnt[k];
-        first[u] = 0;
-        if (n > 0) {
-            if constexpr (bricks)
-                first[u] = atomicAdd(&p.brick_count[(long long)(sd.brick_base + t_key[k]) * kBrickStride], n);
-            else
-                first[u] = atomicAdd(&p.cell_ctr[cell_ctr_slot(p, cb + t_key[k])], n);
+        for (int u = 0; u < kBinPer; ++u) {
+            const int k = tid + kBinThreads * u, n = t_cnt[k];
+            first[u] = n > 0 ? atomicAdd(&p.brick_count[(long long)(sd.brick_base + t_key[k]) * kBrickStride], n) : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < kBinPer; ++u) t_cnt[tid + kBinThreads * u] = first[u];
+    } else {  // one at a time: the pass is bound by their rate
+#pragma unroll 1
+        for (int k = tid; k < kBinHash; k += kBinThreads) {
+            const int n = t_cnt[k];
+            if (n > 0) t_cnt[k] = atomicAdd(&p.cell_ctr[cell_ctr_slot(p, cb + t_key[k])], n);
         }
     }
-#pragma unroll
-    for (int u = 0; u < kBinPer; ++u) t_cnt[tid + kBinThreads * u] = first[u];
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kBinPer; ++u) {
