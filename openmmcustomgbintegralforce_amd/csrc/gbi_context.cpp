@@ -137,6 +137,20 @@ int brick_edge(const SysHost& s) {
     return sk >= 3 ? std::min(gbi::kMaxBrickEdge, sk) : 1;
 }
 
+// Half-width of the switching shells from which GBSW systems are binned: most points of a cell are
+// active then and most list atoms in reach of them, which is what the cells' passes do best, while
+// k_gbsw_points gathers whole lists and the lanes of k_force_gbsw meet on the same atoms.  Evaluation
+// (us on the device), points per atom / binned, at half-widths of 0.08, 0.09, 0.10 and 0.20 nm: GBSW, 3,000
+// atoms 272 / 283, 308 / 302, 339 / 317, 1,019 / 518; 12,000 atoms 835 / 895, 968 / 924, 1,117 / 990, 3,802 /
+// 1,643; on the reference grid 12,000 atoms 650 / 656, 729 / 682, 810 / 715, 1,476 / 811 (the reference's
+// 0.03 nm: a half to a third of the binned time).  The brute cell stays with points per atom (100 atoms,
+// 0.2 nm: 12.4 ms / 18.5).
+constexpr double kWideShell = 0.09;  // nm
+gbi::VolKind volume_kind(const gbi_params& P, gbi::GridKind kind) {
+    const gbi::VolKind vol = (gbi::VolKind)P.integral_type;
+    return vol == gbi::VOL_GBSW && P.sw > kWideShell && kind != gbi::GRID_BRUTE ? gbi::VOL_GBSW_WIDE : vol;
+}
+
 // Point slots per cell: 1.6 times the points of a cell at 100 atoms/nm^3; of a GBSW system, whose
 // slots hold its active points only (7 % of the points in a 25,000-atom globule, three to five
 // times that in the fullest cells), half of it: with a third every first evaluation from 9,000
@@ -161,7 +175,7 @@ struct gbi_ctx {
     long long cell_total = 0;
     long long prec_total = 0;
     int entry_cap = 0;
-    bool kinds[gbi::VOL_KINDS] = {false, false, false};
+    bool kinds[gbi::VOL_KINDS] = {};
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
     int device = 0;
@@ -380,7 +394,7 @@ void atom_params(const gbi_ctx& c, std::vector<float4>& ap, std::vector<double>&
         for (int j = s.atom_begin; j < s.atom_begin + s.N; ++j) {
             const double R = c.radius[j];
             float4 v = make_float4(0.f, 0.f, 0.f, (float)R);
-            if (s.vol == gbi::VOL_GBSW) {
+            if (gbi::is_gbsw(s.vol)) {
                 const double Rp = (R + P.roffset) * P.rscale;
                 const double lo = Rp - P.sw, hi = Rp + P.sw;
                 v.x = (float)Rp;
@@ -480,15 +494,15 @@ gbi::SysDesc make_desc(const gbi_ctx& c, const SysHost& s, long long cell_base, 
     d.vguard = (float)P.vguard;
     d.fclamp = 1.0e6f;
     d.P1 = (float)P.P1;
-    d.v_empty = s.vol == gbi::VOL_GBSW    ? 1.0f
+    d.v_empty = gbi::is_gbsw(s.vol)       ? 1.0f
                 : s.vol == gbi::VOL_GBMV2 ? 0.0f
                                           : (float)(1.0 / (1.0 + std::exp(P.beta * (0.0 - P.lambda))));
-    d.sign_chain = s.vol == gbi::VOL_GBSW ? 1.0f : -1.0f;
+    d.sign_chain = gbi::is_gbsw(s.vol) ? 1.0f : -1.0f;
     // V = 1/(1 + exp(beta (S - lambda))) moves by |beta| S eps_S for a relative error eps_S of
     // S, and its derivative by about as much relative to itself: the FP32 sums' eps_S ~ 3e-7
     // stays well inside the force tolerance up to |beta lambda| ~ 16 (the reference constants
     // have 10); steeper or later sigmoids sum S in FP64
-    d.acc64 = (s.vol != gbi::VOL_GBSW && std::fabs(P.beta * P.lambda) > kSigmoidFp64Above) ? 1 : 0;
+    d.acc64 = (!gbi::is_gbsw(s.vol) && std::fabs(P.beta * P.lambda) > kSigmoidFp64Above) ? 1 : 0;
     d.beta64 = P.beta;
     d.lambda64 = P.lambda;
     d.S064 = P.S0;
@@ -507,6 +521,20 @@ int n_kinds(const gbi_ctx& c) {
     int n = 0;
     for (bool k : c.kinds) n += k;
     return n;
+}
+
+bool any_binned(const gbi_ctx& c) {
+    return c.kinds[gbi::VOL_GBMV1] || c.kinds[gbi::VOL_GBMV2] || c.kinds[gbi::VOL_GBSW_WIDE];
+}
+
+// Buffers per quadrature point of the kinds present.
+gbi_status ensure_point_buffers(gbi_ctx& c) {
+    const size_t NQ = c.NQ, binned = any_binned(c) ? NQ : 1;
+    HIP_TRY(c.frec0.ensure(binned));
+    HIP_TRY(c.frec1.ensure(binned));
+    HIP_TRY(c.frec2.ensure(c.kinds[gbi::VOL_GBMV2] ? NQ : 1));
+    HIP_TRY(c.vval.ensure(binned));
+    return GBI_OK;
 }
 
 // Cell, slot and worklist buffers for the systems' current capacities; uploads the
@@ -987,7 +1015,7 @@ gbi::KParams make_kparams(gbi_ctx& c, bool adjoint) {
             (s.kind == gbi::GRID_TIGHT && !s.periodic() ? k.gbsw_exact : k.gbsw_other) = 1;
             k.gbsw_q = std::max(k.gbsw_q, (s.Q + 1) & ~1);
         }
-    k.gbsw_run = c.kinds[gbi::VOL_GBMV1] || c.kinds[gbi::VOL_GBMV2] ? 64 : std::max(1, (c.N + 7) / 8);
+    k.gbsw_run = any_binned(c) ? 64 : std::max(1, (c.N + 7) / 8);
     k.cell_sub = c.cell_sub.p;
     k.cell_mask = c.kinds[gbi::VOL_GBSW] ? c.cell_mask.p : nullptr;
     k.grec = c.grec.p;
@@ -1267,13 +1295,13 @@ gbi_status setup_host(gbi_ctx& c, int S, const int32_t* n_atoms, const double* c
         h.Q = h.P.n_radial * h.P.n_lebedev;
         h.quad_base = qrow;
         h.pt_base = pt;
-        h.vol = (gbi::VolKind)h.P.integral_type;
         if (h.P.lookup_policy == GBI_LOOKUP_BRUTE)
             h.kind = gbi::GRID_BRUTE;
         else if (h.P.model == GBI_MODEL_GBSW)
             h.kind = gbi::GRID_TIGHT;  // the standalone lists are complete, so exact lists give the same V
         else
             h.kind = gbi::GRID_FAITHFUL;
+        h.vol = volume_kind(h.P, h.kind);
         h.g = h.kind == gbi::GRID_FAITHFUL ? h.P.grid_length : h.P.tight_grid_length;
         h.halfdiag = std::sqrt(3.0) / 2.0 * h.P.grid_length;
         h.gpad = 0.03 + h.halfdiag + h.P.buffer;  // CustomGBIntegral.cpp:174-175
@@ -1410,12 +1438,8 @@ gbi_status create_batch(int S, const int32_t* n_atoms, const double* charge, con
     HIP_TRY(c->atom_energy.ensure(N));
     HIP_TRY(c->stats.ensure(6));
     HIP_TRY(c->work.ensure(gbi::kWorkCounters));
-    const bool any_gbmv = c->kinds[gbi::VOL_GBMV1] || c->kinds[gbi::VOL_GBMV2];
-    HIP_TRY(c->frec0.ensure(any_gbmv ? NQ : 1));
-    HIP_TRY(c->frec1.ensure(any_gbmv ? NQ : 1));
-    HIP_TRY(c->frec2.ensure(c->kinds[gbi::VOL_GBMV2] ? NQ : 1));
+    ST_TRY(ensure_point_buffers(*c));
     HIP_TRY(c->vrec.ensure(NQ));
-    HIP_TRY(c->vval.ensure(any_gbmv ? NQ : 1));
     HIP_TRY(c->atom_nact.ensure(N));
     HIP_TRY(c->bin_order.ensure(N));
     HIP_TRY(c->bin_group.ensure(t.bin_group.size()));
@@ -1968,6 +1992,18 @@ gbi_status gbi_update_constants(gbi_ctx* ctx, int32_t system, const gbi_params* 
     ST_TRY(validate_params(P, s.N, s.custom));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     s.P = P;
+    const gbi::VolKind vol = volume_kind(P, s.kind);
+    if (vol != s.vol) {  // a switching width across the line: the other form, sized on the next evaluation
+        s.vol = vol;
+        std::fill(std::begin(ctx->kinds), std::end(ctx->kinds), false);
+        for (const SysHost& h : ctx->sys) ctx->kinds[h.vol] = true;
+        ctx->drop_graphs();
+        ST_TRY(ensure_point_buffers(*ctx));
+        s.pt_cap = pt_cap_estimate(s);
+        s.cell_cap = 0;
+        s.tmp_cap = 0;
+        ctx->cell_total = 0;
+    }
     ST_TRY(upload_atoms(*ctx));  // the volume constants enter each atom's parameters and reach
     if (ctx->cell_total > 0) ST_TRY(layout(*ctx));  // the descriptors; drops captured graphs
     if (ctx->have_positions && ctx->cell_total > 0) return size_from_device(*ctx, 0);

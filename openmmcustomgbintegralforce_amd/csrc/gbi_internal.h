@@ -18,8 +18,10 @@ enum GridKind : int {
     GRID_BRUTE = 2      // one cell holding every atom of the system
 };
 
-// Volume function of the integral.
-enum VolKind : int { VOL_GBSW = 0, VOL_GBMV1 = 1, VOL_GBMV2 = 2, VOL_KINDS = 3 };
+// Volume function of the integral.  GBSW has two forms with the same function: points per atom
+// (VOL_GBSW), and binned into cells like GBMV's where the switching shells are wide (VOL_GBSW_WIDE).
+enum VolKind : int { VOL_GBSW = 0, VOL_GBMV1 = 1, VOL_GBMV2 = 2, VOL_GBSW_WIDE = 3, VOL_KINDS = 4 };
+constexpr bool is_gbsw(int kind) { return kind == VOL_GBSW || kind == VOL_GBSW_WIDE; }
 
 // Device-side flags (SysGeom::flags of the system, OR-ed into *flags_all).
 enum : int {
@@ -243,15 +245,15 @@ struct KParams {
     int brick_total;         // sum of the systems' brick ranges
     int brick_max;           // the largest brick range of a system
     int any_bricks;          // some system bins by bricks (SysDesc::sk > 1)
-    int any_cellbin;         // some GBMV system bins by cells (SysDesc::sk = 1)
+    int any_cellbin;         // some system of a binned kind bins by cells (SysDesc::sk = 1)
     int* cell_act_count;     // cell_total (diagnostics)
     int4* work_a;            // worklist entries (k_worklist), cell_total for each volume kind present:
     int4* work_b;            //   those of kind k from work_at[k]
-    int* work_act;           // per entry of a GBMV kind: its active points
+    int* work_act;           // per entry of a binned kind: its active points
     int work_at[VOL_KINDS];
     float4* prec;            // per system: cell_cap x pt_cap slots; records (FP32 point - corner, packed point),
                              // or, binning by bricks, packed points (atom << kQBits | q) in the range's first quarter
-    int gbsw_exact, gbsw_other;    // some GBSW system has the exact non-periodic grid, another one
+    int gbsw_exact, gbsw_other;    // some VOL_GBSW system has the exact non-periodic grid, another one
     int gbsw_run;                  // consecutive atoms that one XCD takes in k_gbsw_points
     int gbsw_q;                    // the most points per atom of a GBSW system, rounded up to even
     ulonglong2* cell_mask;         // cell_total (null without GBSW systems): sub-cells with V = 0, with V = 1
@@ -260,11 +262,11 @@ struct KParams {
     float4* grec;            // GBSW systems: slots of their active points (prec_base, pt_cap as in prec)
     float2* gval;            // per grec slot (by pid where cell_sub is null): V, rank among its owner's active points
     int* atom_nact;          // N: active points of each atom (GBSW)
-    float4* frec0;           // NQ (GBMV): active points, grouped by cell (corner-relative FP32 point, packed point)
-    float4* frec1;           // NQ: GBMV1 (dV/dS, V, 0, 0) / GBMV2 (c1, c2, c3, vx)
+    float4* frec0;           // NQ (binned kinds): active points, grouped by cell (corner-relative FP32 point, packed point)
+    float4* frec1;           // NQ: GBSW (V, 0, 0, 0) / GBMV1 (dV/dS, V, 0, 0) / GBMV2 (c1, c2, c3, vx)
     float4* frec2;           // NQ: GBMV2 (vy, vz, V, 0)
-    float* vval;             // NQ by pid (GBMV): V, sign bit set on the points with a chain-rule factor
-    float4* vrec;            // NQ: owner force of those points only (others stale), .w unused; by pid, GBSW:
+    float* vval;             // NQ by pid (binned kinds): V, sign bit set on the points with a chain-rule factor
+    float4* vrec;            // NQ: owner force of those points only (others stale), .w unused; by pid, VOL_GBSW:
                              // by rank among the owner's active points
     float* vsig;             // NQ (adjoint, GBMV) by pid: S of the sigmoid, NaN where V has no derivative
     // per atom

@@ -885,7 +885,7 @@ __device__ inline void quad_point(const KParams& p, double xi, double yi, double
     pt[2] = zi + p.quad_off[3 * row + 2];
 }
 
-// Binning of the GBMV kinds.  k_point_bin: one workgroup per atom or group of atoms (systems in
+// Binning of the binned kinds (GBMV, and GBSW with wide shells).  k_point_bin: one workgroup per atom or group of atoms (systems in
 // turn, each visited with a stride coprime to its size so concurrent workgroups hit distant counters) finds the cell of every
 // quadrature point (FP64, the oracle's arithmetic), counts its points per key in an LDS hash
 // table (local ranks) and reserves each key's slots with one global atomic; these returning
@@ -973,6 +973,8 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
     const int pbase = sd.pt_base + (i0 - sd.atom_begin) * Q;
     const float v_empty = sd.v_empty;
     const float sig_empty = sd.vol_kind == VOL_GBMV1 ? 0.0f : __int_as_float(0x7fc00000);
+    // GBSW points inside their owner have V = 0, where the lists surely hold the owner (k_gbsw_points)
+    const bool in_owner = sd.vol_kind == VOL_GBSW_WIDE && sd.grid_kind != GRID_FAITHFUL;
     for (int k = tid; k < kBinHash; k += kBinThreads) {
         t_key[k] = -1;
         t_cnt[k] = 0;
@@ -996,6 +998,10 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
         int a = 0;
         for (int m = 1; m < kAtoms; ++m) a += k >= m * Q;
         const int row = qb + k - a * Q, i = i0 + a;
+        if (in_owner && p.quad_r2[row] <= p.aparam[i].y) {
+            in_cell[u] = -1;
+            continue;
+        }
         int idx[3] = {0, 0, 0};
         double pt[3];
         quad_point(p, p.pos[3 * i], p.pos[3 * i + 1], p.pos[3 * i + 2], row, pt);
@@ -1022,7 +1028,7 @@ __global__ void __launch_bounds__(bin_threads<BRICKS>(), BRICKS ? 8 : 1) k_point
         const int k = tid + kBinThreads * u;
         if (k >= npts) continue;
         if (key[u] < 0 || in_cell[u] == 0) {
-            p.vval[pbase + k] = v_empty;
+            p.vval[pbase + k] = in_cell[u] < 0 ? 0.f : v_empty;
             if (p.adjoint) p.vsig[pbase + k] = sig_empty;
             continue;
         }
@@ -1470,7 +1476,7 @@ __global__ void __launch_bounds__(kWorkThreads) k_worklist(KParams p) {
             m[k] = __ballot(vk == k);
             if (lane == 0) s_cnt[k][wid] = __popcll(m[k]);
         }
-        const int rec = vk == VOL_GBMV1 || vk == VOL_GBMV2 ? np : 0;
+        const int rec = vk > VOL_GBSW ? np : 0;  // the binned kinds
         const int rec_incl = wave_scan_incl(rec, lane);
         if (lane == kWave - 1) s_rec[wid] = rec_incl;
         __syncthreads();
@@ -1511,9 +1517,10 @@ __device__ inline WorkCell work_cell(const KParams& p, int vk, int w) {
 }
 
 // ---------------------------------------------------------------------------
-// Volume pass of the GBMV kinds: one wave per cell, lanes = quadrature points, the cell's
+// Volume pass of the binned kinds: one wave per cell, lanes = quadrature points, the cell's
 // atoms staged in LDS (corner-relative FP32).  Writes V per point (vval, by point; stored negated, -0 for
 // V = 0, on the points that carry a chain-rule factor) and their compacted records.
+// GBSW (wide shells): V = prod_j H_j (GBSWIntegral.cpp:187-224), chain-rule factor where 0 < V < 1;
 // GBMV-I: S = sum exp(gamma_j d^4) (GBMVIntegralTypeI.cpp:155-173);
 // GBMV-II: sum1, sum2, v, S = S0 sum1 sum2/|v|^2 (GBMVIntegralTypeII.cpp:163-191).
 // ---------------------------------------------------------------------------
@@ -1544,6 +1551,7 @@ template <int VK>
 __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
     __shared__ float s_x[kMaxAtomChunk], s_y[kMaxAtomChunk], s_z[kMaxAtomChunk];
     __shared__ float s_a[kMaxAtomChunk], s_b[kMaxAtomChunk];
+    __shared__ float s_c[VK == VOL_GBSW_WIDE ? kMaxAtomChunk : 1];
     const int nwork = p.work[VK];
     if (batch_fatal(p)) return;
     const int lane = threadIdx.x;
@@ -1563,7 +1571,8 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
         cell_corner(sd, G, c - sd.cell_base, corner);
         const float fclamp = sd.fclamp, S0 = sd.S0, vguard = sd.vguard;
         const float beta = sd.beta, lambda = sd.lambda;
-        const bool acc64 = sd.acc64;
+        const float k1 = sd.k1, k3 = sd.k3;
+        const bool acc64 = VK != VOL_GBSW_WIDE && sd.acc64;
         auto stage = [&](int ab, int cnt) {
             for (int k = lane; k < cnt; k += kWave) {
                 const float4 e = p.ent_pos[as + ab + k];
@@ -1573,6 +1582,13 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
                 s_z[k] = e.z;
                 s_a[k] = e.w;
                 s_b[k] = q.x;
+                if (VK == VOL_GBSW_WIDE) s_c[k] = q.y;
+            }
+            if (VK == VOL_GBSW_WIDE && lane < ((cnt + 3) & ~3) - cnt) {
+                // pad to a multiple of 4 with atoms that neither bury nor touch any point
+                const int k = cnt + lane;
+                s_x[k] = s_y[k] = s_z[k] = s_a[k] = 0.f;
+                s_b[k] = s_c[k] = -1.f;
             }
         };
         __syncthreads();
@@ -1595,6 +1611,7 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
             }
             const int i = (int)(pk >> kQBits), q = (int)(pk & ((1u << kQBits) - 1));
             const float prx = pr.x, pry = pr.y, prz = pr.z;
+            float V = valid ? 1.f : 0.f;  // GBSW
             float s1 = 0.f, s2 = 0.f, vx = 0.f, vy = 0.f, vz = 0.f;
             double S1 = 0.0, S2 = 0.0, VX = 0.0, VY = 0.0, VZ = 0.0;  // acc64 systems
             for (int ab = 0; ab < na; ab += kMaxAtomChunk) {
@@ -1604,7 +1621,24 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
                     stage(ab, cnt);
                     __syncthreads();
                 }
-                if (VK == VOL_GBMV2) {
+                if (VK == VOL_GBSW_WIDE) {
+                    // branch-free: H = 0 inside R' - w, the cubic in the shell, 1 beyond R' + w; the
+                    // wave leaves once every point is buried (V = 0), checked every 4 atoms
+                    const int cnt4 = (cnt + 3) & ~3;
+                    for (int m = 0; m < cnt4; m += 4) {
+                        if (__all(V == 0.f)) break;
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const float dx = s_x[m + u] - prx, dy = s_y[m + u] - pry, dz = s_z[m + u] - prz;
+                            const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                            const float x = fast_sqrt(d2) - s_a[m + u];
+                            float h = fmaxf(fmaf(x, fmaf(-k3 * x, x, k1), 0.5f), 0.f);
+                            h = d2 < s_c[m + u] ? h : 1.f;
+                            h = d2 <= s_b[m + u] ? 0.f : h;
+                            V *= h;
+                        }
+                    }
+                } else if (VK == VOL_GBMV2) {
                     if (valid && !acc64) {
                         #pragma unroll 4
                         for (int m = 0; m < cnt; ++m) {
@@ -1657,7 +1691,11 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
             float4 r1 = make_float4(0.f, 0.f, 0.f, 0.f), r2 = make_float4(0.f, 0.f, 0.f, 0.f);
             if (valid) {
                 const int pid = pt_base + (i - abeg) * Q + q;
-                if (VK == VOL_GBMV2) {
+                if (VK == VOL_GBSW_WIDE) {
+                    active = V > 0.f && V < 1.f;
+                    p.vval[pid] = mark_active(V, active);
+                    r1.x = V;
+                } else if (VK == VOL_GBMV2) {
                     float vsq, S, t;
                     bool guard;
                     if (acc64) {
@@ -1727,7 +1765,7 @@ __global__ void __launch_bounds__(64, 7) k_volume(KParams p) {
 
 // ---------------------------------------------------------------------------
 // Integrals and Born radii: one wave per atom, fixed-order FP64 sums over q.
-// I_k(i) = sum_q w_q / r_q^(n_k - 2) * (1 - V) [GBSW, in k_gbsw_points] or * V [GBMV]
+// I_k(i) = sum_q w_q / r_q^(n_k - 2) * (1 - V) [GBSW; VOL_GBSW in k_gbsw_points] or * V [GBMV]
 // (GBSWIntegral.cpp:142-146; GBMVIntegralTypeII.cpp:145-149).
 // B = slope / (a0 (1/eta - I4) + a1 (1/(4 eta^4) - I7)^(1/4)) + shift
 // (CharmmReferenceGBSW.cpp:591-593; dB/dI as :607-609).
@@ -1741,6 +1779,7 @@ __global__ void __launch_bounds__(64) k_integrals(KParams p) {
     if (sd.vol_kind == VOL_GBSW) return;  // k_gbsw_points
     const int Q = sd.Q, qb = sd.quad_base;
     const int pbase = sd.pt_base + (i - sd.atom_begin) * Q;
+    const bool gbsw = sd.vol_kind == VOL_GBSW_WIDE;
     double a0 = 0.0, a1 = 0.0;
     // Q a multiple of 4 (every system's points start on a multiple of 4): 4 points per lane
     // and load (0.045 -> 0.037 ms at 25k GBSW atoms), in a fixed order either way
@@ -1752,7 +1791,7 @@ __global__ void __launch_bounds__(64) k_integrals(KParams p) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int q = 4 * q4 + j;
-                const double f = (double)volume_of(vv[j]);
+                const double v = (double)volume_of(vv[j]), f = gbsw ? 1.0 - v : v;
                 a0 += p.quad_pw[qb + q] * f;
                 a1 += p.quad_pw[p.quad_rows + qb + q] * f;
             }
@@ -1760,7 +1799,7 @@ __global__ void __launch_bounds__(64) k_integrals(KParams p) {
     } else {
 #pragma unroll 4
         for (int q = lane; q < Q; q += kWave) {
-            const double f = (double)volume_of(p.vval[pbase + q]);
+            const double v = (double)volume_of(p.vval[pbase + q]), f = gbsw ? 1.0 - v : v;
             a0 += p.quad_pw[qb + q] * f;
             a1 += p.quad_pw[p.quad_rows + qb + q] * f;
         }
@@ -2373,7 +2412,7 @@ __global__ void __launch_bounds__(kChainGroups * kWave) k_atom_chain(KParams p) 
 }
 
 // ---------------------------------------------------------------------------
-// Chain-rule force pass of the GBMV kinds: one wave per cell.  Lanes form an 8 x 8 tile: lane = atom group
+// Chain-rule force pass of the binned kinds: one wave per cell.  Lanes form an 8 x 8 tile: lane = atom group
 // (lane & 7) x point group (lane >> 3); a lane owns 8 atoms of the chunk (registers) and
 // 8 points of each 64-point chunk (LDS).  For a point p of owner i with
 // fac = sum_k dE/dI_k(i) w_q / r_q^(n_k - 2) and s = +1 (GBSW) / -1 (GBMV):
@@ -2387,8 +2426,8 @@ __global__ void __launch_bounds__(kChainGroups * kWave) k_atom_chain(KParams p) 
 // bounds the pass: 0.062 ms is left with one of its three atom rows, the chain of loads of each
 // cell, its staging and its sums; 0.013 the owners' scattered stores; the exact sums 0.004.  Six
 // or five atoms per lane at 4 waves per SIMD were slower (0.125), their lists needing two rounds.
-// ADJ: also s fac dV_p/dR_j for every list atom including the owner, and the per-system
-// parameter sums (VolAcc).
+// ADJ: also s fac dV_p/dR_j (GBSW: dR'_j) for every list atom including the owner, and the per-system
+// parameter sums (VolAcc).  GBSW and TRUNC: wide shells, as k_force_gbsw.
 // ---------------------------------------------------------------------------
 
 // Sum over the 8 lanes 8g..8g+7 (DPP: quad xor 1, quad xor 2, half-row mirror).
@@ -2399,11 +2438,14 @@ __device__ inline float sum8(float v) {
     return v;
 }
 
-template <int VK, bool ADJ>
-__global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
+template <int VK, bool ADJ, bool TRUNC>
+__global__ void __launch_bounds__(64, ADJ || TRUNC ? 2 : 3) k_force(KParams p) {
+    constexpr bool kGbsw = VK == VOL_GBSW_WIDE;
     __shared__ float q_x[kWave], q_y[kWave], q_z[kWave];
-    // GBMV-II: c1, c2 and c3 v of the point times s fac; GBMV-I: dV/dS times s fac; all in units of
-    // 2^-24 (the quantum), so the partials below need no scaling of their own
+    __shared__ float q_w[TRUNC ? 3 : 1][kWave];  // TRUNC: owner position relative to the cell corner
+    __shared__ int q_tf[TRUNC ? kWave : 1];      // TRUNC: 0 every shell atom within c of the owner, 1 test, 2 none
+    // GBMV-II: c1, c2 and c3 v of the point times s fac; GBMV-I: dV/dS times s fac; GBSW: s fac (q_0) and
+    // V (q_1); all but V in units of 2^-24 (the quantum), so the partials below need no scaling of their own
     __shared__ float q_0[kWave], q_1[kWave], q_vx[kWave], q_vy[kWave], q_vz[kWave];
     __shared__ int q_own[kWave], q_pid[kWave];
     // one axis of the per-lane atom partials at a time; rows padded by 8 doubles so the 8 rows
@@ -2423,14 +2465,18 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
         const SysDesc sd = p.sys[s];  // a copy: read once per cell
         const int pt_base = sd.pt_base, abeg = sd.atom_begin, Q = sd.Q, qb = sd.quad_base;
         const float fclamp = sd.fclamp, sign_chain = sd.sign_chain, P1x10 = 10.f * sd.P1;
+        const float k1 = sd.k1, k3 = sd.k3, inv_sw = sd.inv_sw;
+        const bool trunc = TRUNC && sd.chain_trunc;
+        BoxF bx;
+        if (TRUNC) bx = box_f(p, s, sd);
         double pacc0 = 0.0, pacc1 = 0.0;  // ADJ: VolAcc partials of this lane
         for (int ab = 0; ab < na; ab += kWave) {
-            float ax[8], ay[8], az[8], a0[8], a1[8], aR[8];
+            float ax[8], ay[8], az[8], a0[8], a1[8], aR[8];  // GBSW: R', (R' - w)^2, (R' + w)^2 (in aR)
             int aj[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
                 const int sl = ab + ag + 8 * k;
-                // past the list: C = 0 (gamma = 0), b = 1, nothing to add
+                // past the list: C = 0 (gamma = 0), b = 1, no shell; nothing to add
                 float4 e = make_float4(0.f, 0.f, 0.f, 0.f), q = make_float4(1.f, 0.f, __int_as_float(-1), 1.f);
                 if (sl < na) {
                     e = p.ent_pos[as + sl];
@@ -2442,7 +2488,7 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
                 a0[k] = e.w;
                 a1[k] = q.x;
                 aj[k] = __float_as_int(q.z);
-                aR[k] = q.w;
+                aR[k] = kGbsw ? q.y : q.w;
             }
             const int kmax = (min(kWave, na - ab) + 7) / 8;  // atoms per lane
             double acc[8][3];
@@ -2472,7 +2518,18 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
                     q_z[lane] = r0.z;
                     q_own[lane] = i;
                     q_pid[lane] = pt_base + (i - abeg) * Q + q;
-                    if (VK == VOL_GBMV2) {
+                    if (TRUNC) {
+                        const int row = qb + q;
+                        q_w[0][lane] = r0.x - (float)p.quad_off[3 * row];
+                        q_w[1][lane] = r0.y - (float)p.quad_off[3 * row + 1];
+                        q_w[2][lane] = r0.z - (float)p.quad_off[3 * row + 2];
+                        const float rq = fast_sqrt(p.quad_r2[row]);
+                        q_tf[lane] = !trunc || rq < sd.trunc_in ? 0 : (rq > sd.trunc_out ? 2 : 1);
+                    }
+                    if (kGbsw) {
+                        q_0[lane] = facs;
+                        q_1[lane] = r1.x;
+                    } else if (VK == VOL_GBMV2) {
                         const float4 r2 = p.frec2[o];
                         const float c3 = facs * r1.z;
                         q_0[lane] = facs * r1.x;
@@ -2492,10 +2549,13 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
                     if (m < cntp) {
                         const float px = q_x[m], py = q_y[m], pz = q_z[m];
                         const int own = q_own[m];
-                        const float d0 = q_0[m], d1 = VK == VOL_GBMV2 ? q_1[m] : 0.f;
+                        const float d0 = q_0[m], d1 = VK == VOL_GBMV2 || kGbsw ? q_1[m] : 0.f;
                         const float vx = VK == VOL_GBMV2 ? q_vx[m] : 0.f;
                         const float vy = VK == VOL_GBMV2 ? q_vy[m] : 0.f;
                         const float vz = VK == VOL_GBMV2 ? q_vz[m] : 0.f;
+                        const int tf = TRUNC ? q_tf[m] : 0;
+                        const float wx = TRUNC ? q_w[0][m] : 0.f, wy = TRUNC ? q_w[1][m] : 0.f,
+                                    wz = TRUNC ? q_w[2][m] : 0.f;
 #pragma unroll
                         for (int k = 0; k < 8; ++k) {
                             if (k >= kmax) break;
@@ -2504,7 +2564,24 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
                             const float dx = ax[k] - px, dy = ay[k] - py, dz = az[k] - pz;
                             const float dd = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
                             float cx, cy, cz;
-                            if (VK == VOL_GBMV2) {
+                            if (kGbsw) {
+                                if (!(dd < aR[k] && dd > a1[k])) continue;  // shell atoms only
+                                const float d = fast_sqrt(dd), x = d - a0[k];
+                                const float h = fmaf(x, fmaf(-k3 * x, x, k1), 0.5f);
+                                if (!(h > 0.f)) continue;
+                                const float dh = fmaf(-3.f * k3 * x, x, k1);
+                                const float gV = d0 * (d1 * fast_rcp(h));  // s fac V / H_j
+                                if (ADJ) {
+                                    // dV/dR'_j = -V H'_j/H_j; dV/dw = V (dH_j/dw)/H_j
+                                    accr[k] += (double)rintf(-gV * dh);
+                                    const float xw = x * inv_sw;
+                                    pacc0 += (double)rintf(gV * 0.75f * xw * inv_sw * fmaf(xw, xw, -1.f));
+                                }
+                                const float sv = gV * dh * fast_rcp(d);
+                                cx = sv * dx;
+                                cy = sv * dy;
+                                cz = sv * dz;
+                            } else if (VK == VOL_GBMV2) {
                                 // F = (C/t)^2, dF/d(d) / d = D = -400 C^2 / t^3; G = s fac dV/dF_j
                                 const float rt = fast_rcp(fmaf(100.f, dd, a1[k]));
                                 const float ct = a0[k] * rt;
@@ -2539,9 +2616,21 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
                                 }
                             }
                             if (ADJ && is_own) continue;  // the owner moves with its points
-                            acc[k][0] += (double)rintf(cx);
-                            acc[k][1] += (double)rintf(cy);
-                            acc[k][2] += (double)rintf(cz);
+                            bool keep = !TRUNC || tf != 2;
+                            if (TRUNC && tf == 1) {
+                                float ex = ax[k] - wx, ey = ay[k] - wy, ez = az[k] - wz;
+                                if (sd.periodic) {
+                                    ex = min_image(ex, bx.L[0], bx.inv[0]);
+                                    ey = min_image(ey, bx.L[1], bx.inv[1]);
+                                    ez = min_image(ez, bx.L[2], bx.inv[2]);
+                                }
+                                keep = within_cutoff(p, s, sd, fmaf(ex, ex, fmaf(ey, ey, ez * ez)), own, aj[k]);
+                            }
+                            if (keep) {
+                                acc[k][0] += (double)rintf(cx);
+                                acc[k][1] += (double)rintf(cy);
+                                acc[k][2] += (double)rintf(cz);
+                            }
                             ox += cx;
                             oy += cy;
                             oz += cz;
@@ -2593,7 +2682,7 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
             pacc1 = wave_sum(pacc1);
             if (lane == 0) {
                 long long* va = p.vacc_fix + ((long long)s * kVaccCopies + (w & (kVaccCopies - 1))) * kVaccStride;
-                const int i0 = VK == VOL_GBMV2 ? VA_A : VA_GAMMA;
+                const int i0 = kGbsw ? VA_W : VK == VOL_GBMV2 ? VA_A : VA_GAMMA;
                 if (pacc0 != 0.0) add_fix(&va[i0], pacc0);
                 if (VK == VOL_GBMV2 && pacc1 != 0.0) add_fix(&va[VA_AR], pacc1);
             }
@@ -2602,7 +2691,7 @@ __global__ void __launch_bounds__(64, ADJ ? 2 : 3) k_force(KParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Chain-rule force pass of GBSW: one wave per cell, lanes = active points, the cell's atoms in
+// Chain-rule force pass of VOL_GBSW: one wave per cell, lanes = active points, the cell's atoms in
 // LDS.  A lane runs down the atoms of its point's sub-cell (cell_sub, 6 on average) and takes
 // those whose shell |d - R'| < w holds the point (2 or 3): dV/dx_j = V H'_j/H_j (x_j - p)/d.  The
 // owner's force stays in the lane's registers; the atoms' partials, integers on the 2^-24 grid,
@@ -2813,7 +2902,7 @@ __global__ void __launch_bounds__(64) k_owner_reduce(KParams p) {
     const SysDesc& sd = p.sys[s];
     const int Q = sd.Q, qb = sd.quad_base;
     const int pbase = sd.pt_base + (i - sd.atom_begin) * Q;
-    const bool gbsw = sd.vol_kind == VOL_GBSW;
+    const bool gbsw = is_gbsw(sd.vol_kind);
     const double e4 = p.dedi[i], e7 = p.dedi[p.N + i];
     const double sc = sd.sign_chain;
     const double beta = sd.beta, lambda = sd.lambda;
@@ -2826,7 +2915,7 @@ __global__ void __launch_bounds__(64) k_owner_reduce(KParams p) {
         a[0] += marked ? (double)v.x : 0.0;
         a[1] += marked ? (double)v.y : 0.0;
         a[2] += marked ? (double)v.z : 0.0;
-        if (ADJ) {
+        if (ADJ && !gbsw) {
             const float S = p.vsig[pid];
             if (!isnan(S)) {
                 const double facs = sc * (e4 * p.quad_pw[qb + q] + e7 * p.quad_pw[p.quad_rows + qb + q]);
@@ -2838,7 +2927,7 @@ __global__ void __launch_bounds__(64) k_owner_reduce(KParams p) {
             }
         }
     };
-    if (gbsw) {  // dense: the active points in q order (k_gbsw_points)
+    if (sd.vol_kind == VOL_GBSW) {  // dense: the active points in q order (k_gbsw_points)
         const int n = p.atom_nact[i];
         for (int k = lane; k < n; k += kWave) {
             const float4 v = p.vrec[pbase + k];
@@ -2921,7 +3010,7 @@ __global__ void __launch_bounds__(kThetaThreads) k_theta_reduce(KParams p) {
         double* th = p.theta + s * TH_COUNT;
         for (int r = 0; r < kThetaRows; ++r) th[atom_rows[r]] = s_row[r];
         th[TH_SW] = th[TH_GAMMA0] = th[TH_P1] = th[TH_P2] = 0.0;
-        if (sd.vol_kind == VOL_GBSW) {
+        if (is_gbsw(sd.vol_kind)) {
             th[TH_SW] = -(double)s_va[VA_W] / kFix32;
         } else if (sd.vol_kind == VOL_GBMV2) {
             th[TH_P1] = -(double)s_va[VA_AR] / kFix32;
@@ -3012,8 +3101,14 @@ void launch_force(const KParams& p, int vk, int blocks, hipStream_t stream) {
         else
             hipLaunchKernelGGL((k_force_gbsw<ADJ, false>), dim3(blocks), dim3(64), 0, stream, p);
         break;
-    case VOL_GBMV1: hipLaunchKernelGGL((k_force<VOL_GBMV1, ADJ>), dim3(blocks), dim3(64), 0, stream, p); break;
-    default: hipLaunchKernelGGL((k_force<VOL_GBMV2, ADJ>), dim3(blocks), dim3(64), 0, stream, p); break;
+    case VOL_GBMV1: hipLaunchKernelGGL((k_force<VOL_GBMV1, ADJ, false>), dim3(blocks), dim3(64), 0, stream, p); break;
+    case VOL_GBMV2: hipLaunchKernelGGL((k_force<VOL_GBMV2, ADJ, false>), dim3(blocks), dim3(64), 0, stream, p); break;
+    default:
+        if (p.any_trunc)
+            hipLaunchKernelGGL((k_force<VOL_GBSW_WIDE, ADJ, true>), dim3(blocks), dim3(64), 0, stream, p);
+        else
+            hipLaunchKernelGGL((k_force<VOL_GBSW_WIDE, ADJ, false>), dim3(blocks), dim3(64), 0, stream, p);
+        break;
     }
 }
 
@@ -3040,8 +3135,8 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
     mark(1);
     // GBSW's volumes are k_gbsw_points' work, before the scan and the worklist: timed as the volume
     // pass in contexts without GBMV systems, with the binning otherwise
-    const bool any_gbmv = kinds[VOL_GBMV1] || kinds[VOL_GBMV2];
-    if (!any_gbmv) mark(2);
+    const bool any_binned = kinds[VOL_GBMV1] || kinds[VOL_GBMV2] || kinds[VOL_GBSW_WIDE];
+    if (!any_binned) mark(2);
     if (kinds[VOL_GBSW]) {
         const dim3 grid(run_blocks(p.N, p.gbsw_run));
         const size_t lds = (size_t)p.gbsw_q * kGbswLds;
@@ -3056,11 +3151,12 @@ hipError_t launch_evaluate(const KParams& p, const bool* kinds, hipStream_t stre
     hipLaunchKernelGGL(k_worklist, dim3(std::max(1, std::min((p.cell_total + kWorkThreads - 1) / kWorkThreads, 4096))),
                        dim3(kWorkThreads), 0, stream, p);
     const int pb = (std::max(1, std::min(p.cell_total, p.persist_blocks)) + kXcds - 1) / kXcds * kXcds;
-    if (any_gbmv) mark(2);
+    if (any_binned) mark(2);
     if (kinds[VOL_GBMV1]) hipLaunchKernelGGL(k_volume<VOL_GBMV1>, dim3(pb), dim3(64), 0, stream, p);
     if (kinds[VOL_GBMV2]) hipLaunchKernelGGL(k_volume<VOL_GBMV2>, dim3(pb), dim3(64), 0, stream, p);
+    if (kinds[VOL_GBSW_WIDE]) hipLaunchKernelGGL(k_volume<VOL_GBSW_WIDE>, dim3(pb), dim3(64), 0, stream, p);
     mark(3);
-    if (any_gbmv) hipLaunchKernelGGL(k_integrals, dim3(p.N), dim3(64), 0, stream, p);
+    if (any_binned) hipLaunchKernelGGL(k_integrals, dim3(p.N), dim3(64), 0, stream, p);
     mark(4);
     if (p.custom) {
         // general expressions (one system): values, pair tiles, chain
