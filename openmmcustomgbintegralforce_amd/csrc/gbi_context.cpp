@@ -2129,17 +2129,24 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     // the buffers, carved once without a base (the size check, before the device is touched)
     // and once from the scratch array
     const size_t N = c.N, NQ = c.NQ, Q = c.quad_rows, cells = caps.cells;
+    size_t in_bytes = 0, out_at = 0, out_bytes = 0;  // what the host fills, and what it reads back: a copy each
     auto carve = [&](ScratchCarver& sc) {
-    sc.take(c.d_sys, 1), sc.take(c.geom, 1), sc.take(c.d_box, 3), sc.take(c.flags_all, 1), sc.take(c.work, gbi::kWorkCounters);
+    sc.take(c.d_sys, 1), sc.take(c.d_box, 3), sc.take(c.bbox_done, 2);
     sc.take(c.atom_sys, N), sc.take(c.bin_order, N), sc.take(c.pair_atom, N), sc.take(c.colblk, colblk.size());
-    sc.take(c.blk_lo, colblk.size()), sc.take(c.blk_hi, colblk.size()), sc.take(c.pair_tiles, tiles.size());
+    sc.take(c.pair_tiles, tiles.size());
     sc.take(c.pos, 3 * N), sc.take(c.d_charge, N), sc.take(c.d_radius, N), sc.take(c.d_reach, N), sc.take(c.aparam, N);
-    sc.take(c.quad_off, 3 * Q), sc.take(c.quad_pw, 2 * Q), sc.take(c.quad_r2, Q);
+    sc.take(c.quad_off, 3 * Q), sc.take(c.quad_pw, 2 * Q), sc.take(c.quad_r2, Q), sc.take(c.cell_sys, cells);
+    in_bytes = sc.used;
+    sc.take(c.geom, 1);
+    out_at = (in_bytes + 255) & ~size_t(255);
+    sc.take(c.flags_all, 1), sc.take(c.energy, 1), sc.take(c.force_fix, 3 * N);
+    out_bytes = sc.used - out_at;
+    sc.take(c.work, gbi::kWorkCounters), sc.take(c.blk_lo, colblk.size()), sc.take(c.blk_hi, colblk.size());
     sc.take(c.integrals, 2 * N), sc.take(c.born, N), sc.take(c.dbdi, 2 * N), sc.take(c.dedi, 2 * N);
-    sc.take(c.atom_energy, N), sc.take(c.energy, 1), sc.take(c.pair_part, (size_t)c.max_splits * 6 * N);
-    sc.take(c.colpart, (size_t)5 * c.colpart_total), sc.take(c.force_fix, 3 * N);
+    sc.take(c.atom_energy, N), sc.take(c.pair_part, (size_t)c.max_splits * 6 * N);
+    sc.take(c.colpart, (size_t)5 * c.colpart_total);
     sc.take(c.cell_fill, cells), sc.take(c.cell_count_eff, cells), sc.take(c.cell_pt_count, cells);
-    sc.take(c.cell_act_count, cells), sc.take(c.cell_sys, cells), sc.take(c.cell_start, cells + 1);
+    sc.take(c.cell_act_count, cells), sc.take(c.cell_start, cells + 1);
     sc.take(c.scan_tmp, (cells + 4095) / 4096 + 16);
     // the worklist lies over the raw lists, which nothing reads once they are sorted
     const size_t raw_at = sc.used;
@@ -2154,7 +2161,7 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     sc.take(c.frec0, gbsw ? 1 : NQ), sc.take(c.frec1, gbsw ? 1 : NQ);
     sc.take(c.frec2, c.kinds[gbi::VOL_GBMV2] ? NQ : 1), sc.take(c.vval, gbsw ? 1 : NQ), sc.take(c.vrec, NQ);
     sc.take(c.brick_count, gbi::kBrickStride), sc.take(c.brick_rec, 1);
-    sc.take(c.bbox_part, (size_t)gbi::kBboxMaxSlices * gbi::kBboxPart), sc.take(c.bbox_done, 2);
+    sc.take(c.bbox_part, (size_t)gbi::kBboxMaxSlices * gbi::kBboxPart);
     };
     ScratchCarver dry;
     carve(dry);
@@ -2182,40 +2189,39 @@ gbi_status gbi_execute_noalloc(int32_t n_atoms, const double* charge, const doub
     c.stream = st;
     gbi::SysDesc desc = make_desc(c, sh, 0, 0, 0);
     desc.sk = 1;
-    const double box[3] = {0.0, 0.0, 0.0};
-    std::vector<int> cell_sys(cells, 0);
-    auto h2d = [st](void* dst, const void* src, size_t bytes) {
-        return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
+    std::vector<char> in(in_bytes, 0);  // (zero: d_box, bbox_done, cell_sys)
+    auto put = [&](const void* dst, const void* src, size_t bytes) {
+        std::memcpy(in.data() + (static_cast<const char*>(dst) - sc.base), src, bytes);
     };
-    HIP_TRY(h2d(c.d_sys.p, &desc, sizeof(desc)));
-    HIP_TRY(h2d(c.d_box.p, box, sizeof(box)));
-    HIP_TRY(h2d(c.atom_sys.p, t.atom_sys.data(), sizeof(int) * N));
-    HIP_TRY(h2d(c.bin_order.p, t.bin_order.data(), sizeof(int) * N));
-    HIP_TRY(h2d(c.pair_atom.p, t.pair_atom.data(), sizeof(int) * N));
-    HIP_TRY(h2d(c.colblk.p, colblk.data(), sizeof(int) * colblk.size()));
-    HIP_TRY(h2d(c.pair_tiles.p, tiles.data(), sizeof(int4) * tiles.size()));
-    HIP_TRY(h2d(c.pos.p, pos, sizeof(double) * 3 * N));
-    HIP_TRY(h2d(c.d_charge.p, c.charge.data(), sizeof(double) * N));
-    HIP_TRY(h2d(c.d_radius.p, c.radius.data(), sizeof(double) * N));
-    HIP_TRY(h2d(c.d_reach.p, reach.data(), sizeof(double) * N));
-    HIP_TRY(h2d(c.aparam.p, ap.data(), sizeof(float4) * N));
-    HIP_TRY(h2d(c.quad_off.p, t.off.data(), sizeof(double) * t.off.size()));
-    HIP_TRY(h2d(c.quad_pw.p, t.pw.data(), sizeof(double) * t.pw.size()));
-    HIP_TRY(h2d(c.quad_r2.p, t.r2.data(), sizeof(float) * t.r2.size()));
-    HIP_TRY(h2d(c.cell_sys.p, cell_sys.data(), sizeof(int) * cells));
-    const int none_done[2] = {0, 0};
-    HIP_TRY(h2d(c.bbox_done.p, none_done, sizeof(none_done)));
+    put(c.d_sys.p, &desc, sizeof(desc));
+    put(c.atom_sys.p, t.atom_sys.data(), sizeof(int) * N);
+    put(c.bin_order.p, t.bin_order.data(), sizeof(int) * N);
+    put(c.pair_atom.p, t.pair_atom.data(), sizeof(int) * N);
+    put(c.colblk.p, colblk.data(), sizeof(int) * colblk.size());
+    put(c.pair_tiles.p, tiles.data(), sizeof(int4) * tiles.size());
+    put(c.pos.p, pos, sizeof(double) * 3 * N);
+    put(c.d_charge.p, c.charge.data(), sizeof(double) * N);
+    put(c.d_radius.p, c.radius.data(), sizeof(double) * N);
+    put(c.d_reach.p, reach.data(), sizeof(double) * N);
+    put(c.aparam.p, ap.data(), sizeof(float4) * N);
+    put(c.quad_off.p, t.off.data(), sizeof(double) * t.off.size());
+    put(c.quad_pw.p, t.pw.data(), sizeof(double) * t.pw.size());
+    put(c.quad_r2.p, t.r2.data(), sizeof(float) * t.r2.size());
+    HIP_TRY(hipMemcpyAsync(sc.base, in.data(), in_bytes, hipMemcpyHostToDevice, st));
     const gbi::KParams k = make_kparams(c, false);
     HIP_TRY(gbi::launch_evaluate(k, c.kinds, st, nullptr));
+    std::vector<char> out(out_bytes);
+    HIP_TRY(hipMemcpyAsync(out.data(), sc.base + out_at, out_bytes, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    auto got = [&](const void* src) { return out.data() + (static_cast<const char*>(src) - sc.base - out_at); };
     gbi::SysGeom G;
     int all = 0;
     std::vector<long long> fx(3 * N);
     double e = 0.0;
-    HIP_TRY(hipMemcpyAsync(&G, c.geom.p, sizeof(G), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(&all, c.flags_all.p, sizeof(int), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(&e, c.energy.p, sizeof(double), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(fx.data(), c.force_fix.p, sizeof(long long) * 3 * N, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    std::memcpy(&G, got(c.geom.p), sizeof(G));
+    std::memcpy(&all, got(c.flags_all.p), sizeof(int));
+    std::memcpy(&e, got(c.energy.p), sizeof(double));
+    std::memcpy(fx.data(), got(c.force_fix.p), sizeof(long long) * 3 * N);
     all |= G.flags;
     if (all & gbi::FLAG_NONFINITE_POS) return fail(GBI_ERR_NONFINITE, "non-finite atom position");
     if (all & gbi::FLAG_GRID_TOO_LARGE)
