@@ -3028,26 +3028,33 @@ __global__ void __launch_bounds__(kThetaThreads) k_theta_reduce(KParams p) {
 // no count of their points: k_stats_gbsw locates them again.
 __global__ void __launch_bounds__(kGbswThreads) k_stats_gbsw(KParams p, double* out) {
     if (batch_fatal(p)) return;
-    const int i = blockIdx.x, s = p.atom_sys[i];
-    const SysDesc sd = p.sys[s];
-    if (sd.vol_kind != VOL_GBSW) return;
-    const SysGeom G = p.geom[s];
-    const float own_lo2 = sd.grid_kind != GRID_FAITHFUL ? p.aparam[i].y : -1.f;
     double np = 0.0, pairs = 0.0;
-    for (int q = threadIdx.x; q < sd.Q; q += kGbswThreads) {
-        float r[3];
-        if (p.quad_r2[sd.quad_base + q] <= own_lo2) continue;
-        const int c = gbsw_locate(p, sd, G, p.pos[3 * i], p.pos[3 * i + 1], p.pos[3 * i + 2], sd.quad_base + q, r);
-        const int n = c >= 0 ? p.cell_count_eff[sd.cell_base + c] : 0;
-        np += n > 0 ? 1.0 : 0.0;
-        pairs += n;
+    for (int i = blockIdx.x; i < p.N; i += gridDim.x) {
+        const int s = p.atom_sys[i];
+        const SysDesc& sd = p.sys[s];
+        if (sd.vol_kind != VOL_GBSW) continue;
+        const SysGeom& G = p.geom[s];
+        const float own_lo2 = sd.grid_kind != GRID_FAITHFUL ? p.aparam[i].y : -1.f;
+        for (int q = threadIdx.x; q < sd.Q; q += kGbswThreads) {
+            float r[3];
+            if (p.quad_r2[sd.quad_base + q] <= own_lo2) continue;
+            const int c = gbsw_locate(p, sd, G, p.pos[3 * i], p.pos[3 * i + 1], p.pos[3 * i + 2], sd.quad_base + q, r);
+            const int n = c >= 0 ? p.cell_count_eff[sd.cell_base + c] : 0;
+            np += n > 0 ? 1.0 : 0.0;
+            pairs += n;
+        }
     }
+    __shared__ double s_sum[2][kGbswThreads / kWave];
     np = wave_sum(np);
     pairs = wave_sum(pairs);
     if ((threadIdx.x & (kWave - 1)) == 0) {
-        atomicAdd(&out[0], np);
-        atomicAdd(&out[1], pairs);
+        s_sum[0][threadIdx.x / kWave] = np;
+        s_sum[1][threadIdx.x / kWave] = pairs;
     }
+    __syncthreads();
+    if (threadIdx.x >= 2) return;  // one atomic per workgroup and sum: they serialise
+    for (int w = 1; w < kGbswThreads / kWave; ++w) s_sum[threadIdx.x][0] += s_sum[threadIdx.x][w];
+    atomicAdd(&out[threadIdx.x], s_sum[threadIdx.x][0]);
 }
 
 __global__ void k_stats(KParams p, double* out) {
@@ -3304,7 +3311,7 @@ hipError_t launch_add_forces_fixed(long long* dst, int padded_n, const long long
 
 hipError_t launch_stats(const KParams& p, double* out6, hipStream_t stream) {
     hipLaunchKernelGGL(k_stats, dim3(256), dim3(256), 0, stream, p, out6);
-    if (p.gbsw_exact || p.gbsw_other) hipLaunchKernelGGL(k_stats_gbsw, dim3(p.N), dim3(kGbswThreads), 0, stream, p, out6);
+    if (p.gbsw_exact || p.gbsw_other) hipLaunchKernelGGL(k_stats_gbsw, dim3(std::min(p.N, 1024)), dim3(kGbswThreads), 0, stream, p, out6);
     return hipGetLastError();
 }
 
