@@ -239,6 +239,8 @@ struct gbi_ctx {
     size_t energy_at = 0, force_at = 0, result_bytes = 0, adj_bytes = 0;
     HostBuf host_result, host_adj;  // (host_result: then the positions on their way in, at host_pos)
     double* host_pos = nullptr;
+    bool header_read = false;  // host_result holds the last evaluation's flags and energies
+    bool captured = false;     // an evaluation went into a caller's graph, whose replays the host does not see
     bool pos_in_flight = false;  // a copy from host_pos may still be running
 
     // graph replay (index: adjoint evaluation)
@@ -1093,6 +1095,10 @@ gbi_status run(gbi_ctx& c, uint32_t flags) {
             ST_TRY(check_box(c, s, s.box));
         }
     if (adjoint && c.cprog) return fail(GBI_ERR_UNSUPPORTED, "the adjoint covers the canonical GB forms only");
+    if (!c.captured) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        c.captured = hipStreamIsCapturing(c.stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+    }
     if (c.cell_total == 0) ST_TRY(size_from_device(c, 0));
     if (adjoint) ST_TRY(ensure_adjoint_buffers(c));
     gbi::KParams k = make_kparams(c, adjoint);
@@ -1125,6 +1131,7 @@ gbi_status run(gbi_ctx& c, uint32_t flags) {
     }
     c.computed = true;
     c.computed_adjoint = adjoint;
+    c.header_read = false;
     return GBI_OK;
 }
 
@@ -1137,6 +1144,7 @@ gbi_status read_results(gbi_ctx& c, bool forces, bool adjoint) {
     HIP_TRY(gbi::launch_export_results(c.host_result.p, c.result.p, c.force_at, c.force_fix.p, forces ? c.N : 0,
                                        c.host_adj.p, c.adj_result.p, adjoint ? c.adj_bytes : 0, c.stream));
     HIP_TRY(hipStreamSynchronize(c.stream));
+    c.header_read = true;
     c.pos_in_flight = false;
     return GBI_OK;
 }
@@ -2252,8 +2260,9 @@ gbi_status gbi_execute_adjoint(gbi_ctx* ctx, const double* pos, double* energy, 
 gbi_status gbi_get_energy(gbi_ctx* ctx, double* energy) {
     if (!ctx || !energy) return fail(GBI_ERR_INVALID_ARGUMENT, "null argument");
     if (!ctx->computed) return fail(GBI_ERR_INVALID_ARGUMENT, "nothing computed yet");
-    // always from the device: a caller's own graph of gbi_compute replays without a call here
-    ST_TRY(read_results(*ctx, false, false));
+    // gbi_synchronize has read the evaluation's energies with its flags; not to be trusted once a
+    // caller's graph holds an evaluation: it replays without a call here
+    if (ctx->captured || !ctx->header_read) ST_TRY(read_results(*ctx, false, false));
     host_energy(*ctx, energy);
     return GBI_OK;
 }
