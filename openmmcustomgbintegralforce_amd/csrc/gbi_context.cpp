@@ -50,7 +50,8 @@ gbi_status fail(gbi_status st, const std::string& msg) {
 
 constexpr double kOne4PiEps0 = 138.935456;  // OpenMM 7.x SimTKOpenMMRealType.h
 constexpr double kTightMargin = 1e-6;       // nm, guards the exact GBSW lists against rounding
-constexpr long long kMaxCells = 16ll * 1024 * 1024;  // limit of the three-pass scan
+// Limit of k_list_starts (tiles x tiles / 2 additions: 0.10 ms at 11 million cells) and of the memory.
+constexpr long long kMaxCells = 16ll * 1024 * 1024;
 // Workgroups per CU of the per-cell passes: about one per occupied cell, the dispatcher balances
 // them.  A mixed batch of 16 has more cells than 128 give: volume pass 0.800 -> 0.761 ms with 256
 // (systems of up to 25,000 atoms: as many cells as workgroups either way, no change).
@@ -127,9 +128,9 @@ struct SysHost {
 // Binning bricks: sk x sk x sk cells of about 0.45 nm reserve their point slots together (an
 // atom's 1,200 GBMV-II points fall into about 200 such bricks against 670 cells of 0.15 nm;
 // 0.17 ms for binning 5,000 atoms against 0.21 by cells).  Grids of cells above 0.18 nm bin by
-// cells (sk = 1): on the 0.20 nm exact GBSW grid, bricks of 2 or 3 cells per edge were slower
-// (0.49-0.52 ms against 0.44 for 25,000 atoms), their second pass costing more than the
-// atomics they save.
+// cells (sk = 1): on a 0.20 nm grid, bricks of 2 or 3 cells per edge were slower (0.49-0.52 ms against
+// 0.44 for 25,000 GBSW atoms, all of whose points were binned), their second pass costing more than
+// the atomics they save.
 constexpr double kBrickEdgeNm = 0.45;
 int brick_edge(const SysHost& s) {
     if (s.kind == gbi::GRID_BRUTE || s.vol == gbi::VOL_GBSW) return 1;  // GBSW: k_gbsw_points

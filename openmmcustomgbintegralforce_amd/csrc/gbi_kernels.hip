@@ -2,13 +2,14 @@
 //
 // One evaluation (launch_evaluate) of a batch of systems runs, on one stream, one launch
 // per pass for all systems together:
-//   clear -> bounding boxes / grid geometry (workgroup per system) -> cell lists (count,
-//   scan, fill, sort+cap) -> GBSW: volumes, integrals and Born map (per atom); GBMV: point
-//   binning -> volume pass (per cell, lanes = points, one launch per kind present) ->
+//   bounding boxes / grid geometry (workgroups per slice of atoms; the others clear the
+//   counters) -> cell lists (fill, starts, sort+cap) -> GBSW: volumes, integrals and Born map
+//   (per atom); the binned kinds (GBMV, GBSW with wide shells): point binning; worklist of cells ->
+//   volume pass (per cell, lanes = points, one launch per binned kind present) ->
 //   integrals + Born map (per atom) -> STILL pair pass
-//   (tiles of 64 rows x a column range inside one system) -> per-atom chain (dE/dB ->
-//   dE/dI, self energy) -> energy per system -> chain-rule force pass (per cell, lanes =
-//   list atoms x points) -> owner-force reduction [-> adjoint reductions].
+//   (tiles of 64 or 128 rows x a column range inside one system) -> per-atom chain (dE/dB ->
+//   dE/dI, self energy) -> chain-rule force pass (per cell, lanes = list atoms x points, GBSW:
+//   points) -> owner-force reduction and energies [-> adjoint reductions].
 //
 // Determinism: every sum is taken in a fixed order, except the per-(cell, atom) force
 // partials, which are quantised to 2^-24 and summed exactly in FP64 before one int64
@@ -1782,7 +1783,7 @@ __global__ void __launch_bounds__(64) k_integrals(KParams p) {
     const bool gbsw = sd.vol_kind == VOL_GBSW_WIDE;
     double a0 = 0.0, a1 = 0.0;
     // Q a multiple of 4 (every system's points start on a multiple of 4): 4 points per lane
-    // and load (0.045 -> 0.037 ms at 25k GBSW atoms), in a fixed order either way
+    // and load, in a fixed order either way
     if ((Q & 3) == 0) {
         const float4* v4 = reinterpret_cast<const float4*>(p.vval + pbase);
         for (int q4 = lane; q4 < (Q >> 2); q4 += kWave) {
