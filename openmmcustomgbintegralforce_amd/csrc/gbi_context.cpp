@@ -61,9 +61,9 @@ constexpr int kDefaultBlocksPerCU = 256;
 constexpr double kDefaultTightGrid = 0.20;
 // Form of a system's pair tiles, by the system alone (its 64-atom blocks, cutoff and exclusions), so
 // that its FP32 sums are grouped alike alone and in a batch; a tile's length, which follows the
-// batch, changes the order of FP64 sums only.  Pair pass measured (us), 4 waves / one row block / two row blocks:
-// 300 atoms 9.4 / 14.2 / -, 2,500 12.9 / 17.6 / 25.6, 5,000 25.6 / 27.3 / 33.3, 8,000 59 / 46 / 48.6,
-// 12,000 - / 102 / 87, 25,000 - / 339 / 274.
+// batch, changes the order of FP64 sums only.  Pair pass measured (us), 4 waves / one row block: 300 atoms
+// 9.4 / 14.2, 2,500 12.9 / 17.6, 5,000 25.6 / 27.3, 8,000 59 / 46.  With its per-atom reduction, one row
+// block / two: 5,000 atoms 36.7 / 43.3, 8,000 57.2 / 60.1, 8,897 66.2 / 62.9, 12,000 101 / 94, 25,000 352 / 309.
 constexpr int kPairWaves4Blocks = 48;   // up to 3,072 atoms: 4 waves (no gain above in a batch)
 constexpr int kPairRows2Blocks = 140;   // from 8,897 atoms, without cutoff or exclusions: two row blocks
 constexpr int kCutoffTileBlocks = 3;  // column blocks per pair tile of a cutoff system

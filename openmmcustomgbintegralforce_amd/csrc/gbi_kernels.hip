@@ -2197,9 +2197,9 @@ __global__ void __launch_bounds__(64 * WAVES) k_pairs(KParams p) {
 // Two row blocks per wave (pair_rows = 2), for large systems without cutoff or exclusions of their own: lane l
 // holds rows l and 64 + l, which meet column (l + m) mod 64 together, so its LDS reads and the
 // rotation of its sums are paid once for two pairs: 36 VALU instructions per pair against 40.
-// 25,000 atoms: 0.383 -> 0.303 ms, at the issue rate (172,000 VALU instructions per SIMD, 1.7 ns each).
+// 25,000 atoms: 0.326 -> 0.277 ms, at the issue rate (172,000 VALU instructions per SIMD, 1.6 ns each).
 // The column sums leave twice per block, so that each holds 64 terms as in the other forms (one
-// partial of both rows' 128 terms took 0.288 ms, and k_atom_chain 0.026 instead of 0.033, but the
+// partial of both rows' 128 terms took 0.269 ms, and k_atom_chain 0.025 instead of 0.032, but the
 // forces' error against FP64 rose from 2.55e-7 to 2.71e-7).  A tile's first two column blocks are its
 // rows' own: the diagonal block of each row block, and their mutual block once.
 template <bool ADJ>
