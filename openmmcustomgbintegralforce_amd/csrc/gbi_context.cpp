@@ -1098,7 +1098,9 @@ gbi_status run(gbi_ctx& c, uint32_t flags) {
     if (adjoint && c.cprog) return fail(GBI_ERR_UNSUPPORTED, "the adjoint covers the canonical GB forms only");
     if (!c.captured) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        c.captured = hipStreamIsCapturing(c.stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+        const bool known = hipStreamIsCapturing(c.stream, &capture) == hipSuccess;
+        if (!known) (void)hipGetLastError();
+        c.captured = !known || capture != hipStreamCaptureStatusNone;
     }
     if (c.cell_total == 0) ST_TRY(size_from_device(c, 0));
     if (adjoint) ST_TRY(ensure_adjoint_buffers(c));
